@@ -81,6 +81,10 @@ constexpr int SIRIUS_DRIFT_BINS = 320;
 // sigma^2 of the point-spread function, 10^(-0.4 m), colour (3), padding (3).
 constexpr int SIRIUS_STAR_REC = 12;
 
+// Cells of a celestial sphere's star index: SIRIUS_STAR_NT bands of theta, each of SIRIUS_STAR_NP cells
+// of phi (about 0.025 rad a side at the equator).
+constexpr int SIRIUS_STAR_NT = 128, SIRIUS_STAR_NP = 256;
+
 // Finite test usable on host and device: x - x is NaN exactly when x is NaN or infinite.
 template <class T>
 SIRIUS_HD __forceinline__ bool sfinite(T x) {

@@ -16,8 +16,8 @@
 namespace sirius {
 int bundle_for_launch(Handle& H, Batch& B, int emission, int n_cam, BundleOut& bo);
 hipError_t launch_star_shade(const DevOut& o, int64_t n, const float* rec0, int n0, float b0, const float* rec1, int n1,
-                             float b1, const float* bjac, const uint8_t* bcls, const uint8_t* bflags, float bsize,
-                             float* fb, hipStream_t st);
+                             float b1, const int32_t* cells0, const int32_t* cells1, const float* bjac,
+                             const uint8_t* bcls, const uint8_t* bflags, float bsize, float* fb, hipStream_t st);
 hipError_t launch_shade(const CamConst* cam, const DevOut& o, int64_t n, int emission, const ShadeParams& sp,
                         const uint8_t* bg, int bgw, int bgh, float* fb, hipStream_t st);
 hipError_t launch_pixel_average(const float* sub, int w, int h, int gs, float* fb, hipStream_t st);
@@ -208,8 +208,8 @@ int sirius_hip_launch(SiriusHipHandle hh, const SiriusHipCamera* cam, const Siri
         if ((rc = bundle_for_launch(*H, B, emission, 1, bo))) return rc;
     }
     e = launch_star_shade(dout, B.n, H->star_dev[0], H->star_n[0], H->star_brightness[0], H->star_dev[1],
-                          H->star_n[1], H->star_brightness[1], bo.jac, bo.cls, bo.flags, H->bundle.initial_size,
-                          sub, H->stream);
+                          H->star_n[1], H->star_brightness[1], H->star_cells[0], H->star_cells[1], bo.jac, bo.cls,
+                          bo.flags, H->bundle.initial_size, sub, H->stream);
     if (e != hipSuccess) return H->hip_fail(e, "star shade");
     if (gs > 1 && (e = launch_pixel_average(sub, cam->width, cam->height, gs, H->fb_dev, H->stream)) != hipSuccess)
         return H->hip_fail(e, "pixel average");

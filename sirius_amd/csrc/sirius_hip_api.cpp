@@ -254,6 +254,8 @@ void Handle::release() {
         if (star_dev[i]) (void)hipFree(star_dev[i]);
         star_dev[i] = nullptr;
         star_n[i] = 0;
+        if (star_cells[i]) (void)hipFree(star_cells[i]);
+        star_cells[i] = nullptr;
     }
     if (fb_dev) (void)hipFree(fb_dev);
     fb_dev = nullptr;

@@ -96,6 +96,7 @@ struct Handle {
     float* star_dev[2] = {nullptr, nullptr};
     int star_n[2] = {0, 0};
     float star_brightness[2] = {1.f, 1.f};
+    int32_t* star_cells[2] = {nullptr, nullptr};  // the sphere's cell index (starfield.cpp), or null
     // ray bundle of launch (sirius_hip_set_ray_bundle)
     SiriusHipRayBundle bundle = {0, 0, 0.28867513f, 1e-6f, 100.0f, 0};
     // framebuffer shading of launch (sirius_hip_set_shading)

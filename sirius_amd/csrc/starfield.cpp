@@ -113,6 +113,64 @@ void star_record(const SiriusHipStar& s, const SiriusHipStarfield& c, float* rec
     star_colour(s.temperature_K, rec[6], rec[7], rec[8]);
 }
 
+// Cell index of a catalogue of star records: for each cell of the sphere's (theta, phi) grid, the
+// stars whose cut reaches any direction of the cell, in catalogue order, so that a view direction
+// needs to look at its own cell's stars only and adds them in the order a walk of the whole
+// catalogue would. Layout: cells + 1 offsets, then the star numbers. Empty when the index would
+// exceed STAR_CELL_ENTRIES (spreads of a good part of the sky) or a record is not finite: the
+// shading kernel then walks the catalogue.
+// The device compares float cosines: a star can pass its cut at an angle whose true cosine is up to
+// 1e-6 below it (direction and product roundings, 3e-7), and a direction's cell is found from
+// its float angles (4e-7 rad); the reach is widened by both.
+constexpr size_t STAR_CELL_ENTRIES = (size_t)1 << 24;
+
+std::vector<int32_t> star_cell_index(const std::vector<float>& rec, int n) {
+    constexpr int NT = SIRIUS_STAR_NT, NP = SIRIUS_STAR_NP;
+    constexpr double margin = 2e-6;
+    struct Span {
+        int t0, t1, p0, np;  // theta bands t0..t1, np cells of phi from p0 (mod NP)
+    };
+    std::vector<Span> span(n);
+    std::vector<int32_t> idx((size_t)NT * NP + 1, 0);
+    size_t total = 0;
+    for (int i = 0; i < n; ++i) {
+        const float* s = rec.data() + (size_t)i * SIRIUS_STAR_REC;
+        for (int k = 0; k < 5; ++k)
+            if (!std::isfinite(s[k])) return {};
+        if (s[3] > 1.5f) {  // no direction: never within the cut
+            span[i] = {0, -1, 0, 0};
+            continue;
+        }
+        const double th = std::atan2(std::hypot((double)s[0], (double)s[1]), (double)s[2]);
+        const double ph = std::atan2((double)s[1], (double)s[0]);
+        const double reach = std::acos(std::max(-1.0, (double)s[3] - 1e-6)) + margin;
+        const auto band = [](double t) { return std::clamp((int)std::floor(t * (NT / M_PI)), 0, NT - 1); };
+        Span sp{band(th - reach), band(th + reach), 0, NP};
+        if (th - reach > 0 && th + reach < M_PI) {
+            const double half = std::asin(std::min(1.0, std::sin(reach) / std::sin(th))) + margin;
+            const int lo = (int)std::floor((ph - half + M_PI) * (NP / (2 * M_PI)));
+            const int hi = (int)std::floor((ph + half + M_PI) * (NP / (2 * M_PI)));
+            if (hi - lo + 1 < NP) {
+                sp.p0 = ((lo % NP) + NP) % NP;
+                sp.np = hi - lo + 1;
+            }
+        }
+        span[i] = sp;
+        total += (size_t)(sp.t1 - sp.t0 + 1) * sp.np;
+        if (total > STAR_CELL_ENTRIES) return {};
+        for (int t = sp.t0; t <= sp.t1; ++t)
+            for (int k = 0; k < sp.np; ++k) ++idx[1 + t * NP + (sp.p0 + k) % NP];
+    }
+    for (int c = 0; c < NT * NP; ++c) idx[c + 1] += idx[c];
+    std::vector<int32_t> at(idx.begin(), idx.end() - 1);
+    const size_t base = idx.size();
+    idx.resize(base + total);
+    for (int i = 0; i < n; ++i)
+        for (int t = span[i].t0; t <= span[i].t1; ++t)
+            for (int k = 0; k < span[i].np; ++k) idx[base + at[t * NP + (span[i].p0 + k) % NP]++] = i;
+    return idx;
+}
+
 }  // namespace
 
 }  // namespace sirius
@@ -171,6 +229,8 @@ int sirius_hip_set_starfield(SiriusHipHandle hh, int side, const SiriusHipStarfi
         if (H->star_dev[side]) (void)hipFree(H->star_dev[side]);
         H->star_dev[side] = nullptr;
         H->star_n[side] = 0;
+        if (H->star_cells[side]) (void)hipFree(H->star_cells[side]);
+        H->star_cells[side] = nullptr;
         if (n == 0) return SIRIUS_HIP_OK;
         SiriusHipStarfield c = *cfg;
         validate(c);
@@ -184,6 +244,19 @@ int sirius_hip_set_starfield(SiriusHipHandle hh, int side, const SiriusHipStarfi
         e = hipMemcpyAsync(H->star_dev[side], rec.data(), rec.size() * sizeof(float), hipMemcpyHostToDevice, H->stream);
         if (e == hipSuccess) e = hipStreamSynchronize(H->stream);
         if (e != hipSuccess) return H->hip_fail(e, "starfield upload");
+        const std::vector<int32_t> cells = star_cell_index(rec, n);
+        if (!cells.empty()) {
+            // without room for the index the shading kernel walks the catalogue
+            if (hipMalloc((void**)&H->star_cells[side], cells.size() * sizeof(int32_t)) != hipSuccess) {
+                (void)hipGetLastError();
+                H->star_cells[side] = nullptr;
+            } else {
+                e = hipMemcpyAsync(H->star_cells[side], cells.data(), cells.size() * sizeof(int32_t),
+                                   hipMemcpyHostToDevice, H->stream);
+                if (e == hipSuccess) e = hipStreamSynchronize(H->stream);
+                if (e != hipSuccess) return H->hip_fail(e, "starfield upload");
+            }
+        }
         H->star_n[side] = n;
         H->star_brightness[side] = c.brightness_scale;
         return SIRIUS_HIP_OK;
