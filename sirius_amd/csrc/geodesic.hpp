@@ -119,19 +119,48 @@ struct DevOut {
     int64_t n_rays;
 };
 
-// Reciprocal square root and reciprocal: in FP32 device code the hardware instructions
-// (about 1 ulp), elsewhere the correctly rounded forms.
+// Reciprocal square root, reciprocal and square root of a positive value well inside the range
+// (no zero, infinity or denormal: callers clamp). In FP32 device code the hardware instructions
+// (about 1 ulp); in FP64 device code the hardware estimate (about 24 bits) refined by two Newton
+// steps to the last bit or two; on the host the correctly rounded forms. The IEEE FP64 division
+// and square root carry range scaling and special cases: about 12 and 16 instructions, against 5 for
+// the reciprocal and 8 for the reciprocal square root, which yields the root with 3 more.
 template <class T> SIRIUS_HD __forceinline__ T rsqrt_t(T x) {
 #ifdef __HIP_DEVICE_COMPILE__
-    if constexpr (sizeof(T) == 4) return __builtin_amdgcn_rsqf(x);
+    if constexpr (std::is_same_v<T, float>) return __builtin_amdgcn_rsqf(x);
+    if constexpr (std::is_same_v<T, double>) {
+        double y = __builtin_amdgcn_rsq(x);
+        const double hx = 0.5 * x;
+        y = ::fma(y, ::fma(-hx * y, y, 0.5), y);
+        return ::fma(y, ::fma(-hx * y, y, 0.5), y);
+    }
 #endif
     return T(1) / sqrt(x);
 }
 template <class T> SIRIUS_HD __forceinline__ T rcp_t(T x) {
 #ifdef __HIP_DEVICE_COMPILE__
-    if constexpr (sizeof(T) == 4) return __builtin_amdgcn_rcpf(x);
+    if constexpr (std::is_same_v<T, float>) return __builtin_amdgcn_rcpf(x);
+    if constexpr (std::is_same_v<T, double>) {
+        double y = __builtin_amdgcn_rcp(x);
+        y = ::fma(::fma(-x, y, 1.0), y, y);
+        return ::fma(::fma(-x, y, 1.0), y, y);
+    }
 #endif
     return T(1) / x;
+}
+// sqrt(x) from is = rsqrt_t(x): x is in FP32, with one correction of the residual x - g^2 in FP64
+// (within about half an ulp), sqrt itself on the host.
+template <class T> SIRIUS_HD __forceinline__ T sqrt_from(T x, T is) {
+#ifdef __HIP_DEVICE_COMPILE__
+    if constexpr (std::is_same_v<T, double>) {
+        const double g = x * is;
+        return ::fma(::fma(-g, g, x), 0.5 * is, g);
+    }
+    return x * is;
+#else
+    if constexpr (std::is_same_v<T, float>) return x * is;
+    return sqrt(x);
+#endif
 }
 
 // a * b + c with one rounding in the working precision (fmaf for FP32, also in host builds of
@@ -221,6 +250,17 @@ template <class T, int N> SIRIUS_HD __forceinline__ Dual<T, N> sqrt(const Dual<T
     const T s = sqrt(a.v);
     return chain(a, s, T(0.5) / s);
 }
+template <class T, int N> SIRIUS_HD __forceinline__ Dual<T, N> rsqrt_t(const Dual<T, N>& a) {
+    const T s = rsqrt_t(a.v);
+    return chain(a, s, T(-0.5) * s * s * s);
+}
+template <class T, int N> SIRIUS_HD __forceinline__ Dual<T, N> rcp_t(const Dual<T, N>& a) {
+    const T s = rcp_t(a.v);
+    return chain(a, s, -s * s);
+}
+template <class T, int N> SIRIUS_HD __forceinline__ Dual<T, N> sqrt_from(const Dual<T, N>& a, const Dual<T, N>& is) {
+    return chain(a, sqrt_from(a.v, is.v), T(0.5) * is.v);
+}
 template <class T, int N> SIRIUS_HD __forceinline__ Dual<T, N> fabs(const Dual<T, N>& a) { return a.v < T(0) ? -a : a; }
 template <class T, int N> SIRIUS_HD __forceinline__ Dual<T, N> fmax(const Dual<T, N>& a, const Dual<T, N>& b) { return a.v < b.v ? b : a; }
 template <class T, int N> SIRIUS_HD __forceinline__ Dual<T, N> fmin(const Dual<T, N>& a, const Dual<T, N>& b) { return b.v < a.v ? b : a; }
@@ -286,6 +326,11 @@ SIRIUS_HD __forceinline__ T kerr_r(const Spacetime<T>& s, T x, T y, T z) {
     T w = R2 - s.a2;
     T disc = w * w + T(4) * s.a2 * z * z;
     disc = disc < T(1e-20) ? T(1e-20) : disc;
+    if constexpr (std::is_same_v<T, double>) {
+        T r2 = T(0.5) * (w + sqrt_from(disc, rsqrt_t(disc)));
+        r2 = r2 < T(1e-10) ? T(1e-10) : r2;
+        return sqrt_from(r2, rsqrt_t(r2));
+    }
     T r2 = T(0.5) * (w + sqrt(disc));
     r2 = r2 < T(1e-10) ? T(1e-10) : r2;
     return sqrt(r2);
@@ -358,33 +403,26 @@ SIRIUS_HD __forceinline__ T rhs_ks(const Spacetime<T>& s, const T x[4], const T 
     //   dr/dx = x r / s, dr/dy = y r / s, dr/dz = z (r^2 + a^2) / (r s),
     //   s = sqrt((R^2 - a^2)^2 + 4 a^2 z^2) = 2 r^2 - R^2 + a^2;
     // then dH_i = H_r dr_i + H_z [i = z] and sum_j k_j d_i l_j = A_i + B dr_i.
-    constexpr bool f32 = sizeof(T) == 4;
     const T X = x[1], Y = x[2], Z = x[3];
     const T R2v = X * X + Y * Y + Z * Z;
     const T w = R2v - s.a2;                           // R^2 - a^2
     T disc = tfma(T(4) * s.a2, Z * Z, w * w);         // (R^2 - a^2)^2 + 4 a^2 z^2
     disc = fmax(disc, T(1e-20));  // guards only the ring singularity, deep inside the horizon
-    // FP32: square roots and their reciprocals from one hardware reciprocal square root each,
-    // and 1 / rho, 1 / Dn from one reciprocal of their product (three transcendental
-    // instructions instead of six; rho Dn ~ r^6 stays far inside the FP32 range for r < 1e6)
-    T isq = T(0);
-    const T sq = f32 ? disc * (isq = rsqrt_t(disc)) : sqrt(disc);
+    // square roots and their reciprocals from one reciprocal square root each, and 1 / rho, 1 / Dn
+    // from one reciprocal of their product (three transcendental instructions instead of six or,
+    // in FP64, two IEEE roots and five IEEE divisions: a third of the FP64 right-hand side's
+    // instructions; rho Dn ~ r^6 stays far inside the FP32 range for r < 1e6)
+    const T isq = rsqrt_t(disc);
+    const T sq = sqrt_from(disc, isq);
     T r2 = (w + sq) * T(0.5);
     r2 = fmax(r2, T(1e-10));
-    T ir;
-    const T r = f32 ? r2 * (ir = rsqrt_t(r2)) : sqrt(r2);
-    if constexpr (!f32) ir = T(1) / r;
+    const T ir = rsqrt_t(r2);
+    const T r = sqrt_from(r2, ir);
     const T rho = r2 + s.a2;
     const T Dn = tfma(s.a2 * Z, Z, r2 * r2);          // r^4 + a^2 z^2
-    T irho, iDn;
-    if constexpr (f32) {
-        const T inv = rcp_t(rho * Dn);
-        irho = Dn * inv;
-        iDn = rho * inv;
-    } else {
-        irho = T(1) / rho;
-        iDn = T(1) / Dn;
-    }
+    const T inv = rcp_t(rho * Dn);
+    const T irho = Dn * inv;
+    const T iDn = rho * inv;
     const T l1 = tfma(r, X, s.a * Y) * irho;          // (r x + a y) / (r^2 + a^2)
     const T l2 = tfma(r, Y, -s.a * X) * irho;         // (r y - a x) / (r^2 + a^2)
     const T l3 = Z * ir;                              // z / r
@@ -412,8 +450,8 @@ SIRIUS_HD __forceinline__ T rhs_ks(const Spacetime<T>& s, const T x[4], const T 
     T lk = k[0] + l1 * k[1] + l2 * k[2] + l3 * k[3];
     T hl = T(0.5) * lk * lk, Hlk = H * lk, k00 = k[0] * k[0];
     // gradient of r
-    const T rs = f32 ? r * isq : r / sq;
-    const T drx = X * rs, dry = Y * rs, drz = f32 ? Z * rho * ir * isq : Z * rho * ir / sq;
+    const T rs = r * isq;
+    const T drx = X * rs, dry = Y * rs, drz = Z * rho * ir * isq;
     // H_r = (N_r - H Dn_r) / Dn with N = q r^2, N_r = r (6 M r - 2 Q^2), Dn_r = 4 r^3;
     // H_z = -2 a^2 z H / Dn
     const T Hr = (r * (T(6) * s.M * r - T(2) * s.Q2) - H * T(4) * r2 * r) * iDn;
@@ -655,7 +693,28 @@ SIRIUS_HD __forceinline__ T pow_pos(T x, T e) {
 #ifdef __HIP_DEVICE_COMPILE__
     if constexpr (sizeof(T) == 4) return __builtin_amdgcn_exp2f(e * __builtin_amdgcn_logf(x));
 #endif
+    if (e == T(2)) return x * x;  // the FP32 path's default step exponent
     return pow(x, e);
+}
+
+// err^(-1/5). FP64 on the device: the FP32 hardware value refined by two Newton steps on y^-5 = err
+// (relative error 1e-7, then 3e-14, then rounding), a tenth of pow's instructions. err is clamped
+// to 1e6, where the caller's factor is at its lower limit already.
+template <class T>
+SIRIUS_HD __forceinline__ T root5_inv(T err) {
+#ifdef __HIP_DEVICE_COMPILE__
+    if constexpr (std::is_same_v<T, double>) {
+        const double e = ::fmin(err, 1e6);
+        double y = (double)__builtin_amdgcn_exp2f(-0.2f * __builtin_amdgcn_logf((float)e));
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const double y2 = y * y;
+            y = ::fma(y, 0.2 * ::fma(-e * y, y2 * y2, 1.0), y);
+        }
+        return y;
+    }
+#endif
+    return pow_pos(err, T(-0.2));
 }
 
 // computeOptimalStep (PHGD001A.cpp:471-483): h * clamp(0.9 err^-1/5, 0.1, 2), clamped.
@@ -664,7 +723,7 @@ SIRIUS_HD __forceinline__ T next_step(T h, T err, T hmin, T hmax) {
     T hn;
     if (err < T(1e-15)) hn = h * T(2);
     else {
-        T fac = T(0.9) * pow_pos(err, T(-0.2));
+        T fac = T(0.9) * root5_inv(err);
         fac = fac < T(0.1) ? T(0.1) : (fac > T(2) ? T(2) : fac);
         hn = h * fac;
     }
@@ -689,21 +748,6 @@ template <class T>
 SIRIUS_HD __forceinline__ T event_value(const Spacetime<T>& s, int kind, const T x[4], T target) {
     if (kind == EV_Z) return x[3];
     return event_radius(s, x) - target;
-}
-
-template <class T>
-SIRIUS_HD __forceinline__ T locate_event(const Spacetime<T>& s, int kind, T target, const T x0[4], const T k0[4],
-                                 const T x1[4], const T k1[4], T h) {
-    constexpr int iters = sizeof(T) == 8 ? 52 : 24;
-    T lo = T(0), hi = T(1), xm[4];
-    bool neg_lo = event_value(s, kind, x0, target) < T(0);
-    for (int it = 0; it < iters; ++it) {
-        T mid = T(0.5) * (lo + hi);
-        hermite(x0, k0, x1, k1, h, mid, xm);
-        bool neg = event_value(s, kind, xm, target) < T(0);
-        if (neg == neg_lo) lo = mid; else hi = mid;
-    }
-    return T(0.5) * (lo + hi);
 }
 
 // Position on the dense output of a step (x^0 is carried unchanged: the FP32 path does not
@@ -746,12 +790,13 @@ SIRIUS_HD __forceinline__ T locate_event_newton(const Spacetime<T>& s, int kind,
                                                 const T k0[4], const T x1[4], const T k1[4], const T dn[6], T h,
                                                 T f0, T f1) {
     constexpr int max_iters = 24;
-    const T tol = T(sizeof(T) == 4 ? 2e-7 : 1e-15);
+    const T tol = T(sizeof(T) == 4 ? 2e-7 : 1e-12);  // the last step's own error is its square
     T lo = T(0), hi = T(1);
     const bool neg_lo = f0 < T(0);
     T den = f0 - f1;
     T th = den != T(0) ? f0 / den : T(0.5);
     th = th > T(0) && th < T(1) ? th : T(0.5);
+#pragma unroll 1
     for (int it = 0; it < max_iters; ++it) {
         T f, df;
         if (kind == EV_Z) {
@@ -800,6 +845,16 @@ SIRIUS_HD __forceinline__ T locate_event_dense(const Spacetime<T>& s, int kind, 
         if (neg == neg_lo) lo = mid; else hi = mid;
     }
     return T(0.5) * (lo + hi);
+}
+
+// Event location on the step's cubic Hermite interpolant (the dense output without its r5 term):
+// the FP64 path's locator.
+template <class T>
+SIRIUS_HD __forceinline__ T locate_event(const Spacetime<T>& s, int kind, T target, const T x0[4], const T k0[4],
+                                 const T x1[4], const T k1[4], T h) {
+    const T dn[6] = {T(0), T(0), T(0), T(0), T(0), T(0)};
+    return locate_event_newton(s, kind, target, x0, k0, x1, k1, dn, h, event_value(s, kind, x0, target),
+                               event_value(s, kind, x1, target));
 }
 
 // ------------------------------------------------------------------------------------------

@@ -20,7 +20,7 @@
 
 namespace sirius {
 
-enum { ST_RUN = 0, ST_DONE = 1, ST_ESCALATE = 2 };
+enum { ST_RUN = 0, ST_DONE = 1, ST_ESCALATE = 2, ST_LAND = 3 };
 
 SIRIUS_HD __forceinline__ int find_camera(const CamConst* cams, int n_cam, int64_t id) {
     int lo = 0, hi = n_cam - 1;
@@ -90,6 +90,7 @@ struct Ray {
     T vr_prev;      // radial velocity sign tracking (FP32 escalation)
     T r_cur;        // event radius of the current state (kept from the step that reached it)
     T rdisk;        // disk-hit radius of a finished ray
+    T th;           // FP64: fraction of the step at which the ray ends (ST_LAND)
     int64_t id;
     int cam;
     int cls;        // termination class of a finished ray
@@ -321,28 +322,31 @@ SIRIUS_HD __forceinline__ T vol_step_cap(const Spacetime<T>& s, const TraceParam
     return cap > inner * sig ? cap : inner * sig;
 }
 
-// Land exactly on an event at fraction th of the step: one DP45 step of th*h from the step's
-// start, and for the disk plane one Newton correction of th. Landings always end the ray, so
-// the state is overwritten with the landed one. Returns the final th.
-template <class T, int FAM>
-SIRIUS_HD __forceinline__ T land(Ray<T, FAM>& R, const Spacetime<T>& s, bool plane, T th) {
+// FP64: lands a ray that ended (ST_LAND) exactly on its event at fraction R.th of the step: one DP45
+// step of th*h from the step's start, and for the disk plane one Newton correction of th and a
+// second step. The wave lands its ended rays together, before it takes new ones, not each ray as
+// it ends: a landing is up to two steps of work whatever the number of lanes that need it.
+template <class T, int FAM, int EMIT>
+SIRIUS_HD __forceinline__ void land(Ray<T, FAM>& R, const Spacetime<T>& s) {
     constexpr bool TIME = sizeof(T) == 8;
+    const bool plane = EMIT == SIRIUS_EMISSION_THIN_DISK && R.cls == SIRIUS_RAY_DISK;
     T xl[4], pl[4], err[4];
     Der<T> dl;
-    dp45_step<T, FAM, TIME>(s, R.x, R.p, R.d, th * R.h, xl, pl, dl, err, false);
-    R.landings++;
-    if (plane && fabs(dl.k[3]) > T(1e-30)) {
-        T th2 = th - xl[3] / (dl.k[3] * R.h);
-        if (th2 > T(0) && th2 < T(1.5)) {
-            th = th2;
-            dp45_step<T, FAM, TIME>(s, R.x, R.p, R.d, th * R.h, xl, pl, dl, err, false);
-            R.landings++;
-        }
+    T th = R.th;
+    // one copy of the step's code for both passes
+#pragma unroll 1
+    for (int pass = 0; pass < 2; ++pass) {
+        dp45_step<T, FAM, TIME>(s, R.x, R.p, R.d, th * R.h, xl, pl, dl, err, false);
+        R.landings++;
+        if (pass == 1 || !plane || !(fabs(dl.k[3]) > T(1e-30))) break;
+        const T th2 = th - xl[3] / (dl.k[3] * R.h);
+        if (!(th2 > T(0) && th2 < T(1.5))) break;
+        th = th2;
     }
     R.lam += th * R.h;
     for (int i = 0; i < 4; ++i) { R.x[i] = xl[i]; R.p[i] = pl[i]; }
     R.d = dl;
-    return th;
+    R.rdisk = plane ? kerr_r(s, R.x[1], R.x[2], R.x[3]) : T(0);
 }
 
 // The step's low parts become the state's (t and p_t are not stepped: their low parts stay).
@@ -374,7 +378,8 @@ SIRIUS_HD __forceinline__ void land_dense(Ray<T, FAM>& R, const T x1[4], const T
 
 // One DP45 attempt with error control, events and acceptance. Returns ST_RUN, ST_DONE (the
 // ray ended: R.cls, R.rdisk and the final state are set; the caller writes it out with
-// ray_finish) or ST_ESCALATE (an FP32 lane hands the ray to the FP64 queue). Every event is
+// ray_store), ST_LAND (an FP64 ray ended inside the step, at R.th: the caller lands it, then writes
+// it out) or ST_ESCALATE (an FP32 lane hands the ray to the FP64 queue). Every event is
 // located and landed through one code path, so the landing code exists once per kernel.
 template <class T, int FAM, int EMIT, bool MULTI>
 SIRIUS_HD __forceinline__ int ray_attempt(Ray<T, FAM>& R, const CamConst* cams, const Spacetime<T>& s,
@@ -403,7 +408,9 @@ SIRIUS_HD __forceinline__ int ray_attempt(Ray<T, FAM>& R, const CamConst* cams, 
     T e = T(0);
 #pragma unroll
     for (int i = TIME ? 0 : 1; i < 4; ++i) {
-        T q = err[i] / (T(tp.atol) + T(tp.rtol) * fabs(x1[i]));
+        T q;
+        if constexpr (fp32) q = err[i] / (T(tp.atol) + T(tp.rtol) * fabs(x1[i]));
+        else q = err[i] * rcp_t(T(tp.atol) + T(tp.rtol) * fabs(x1[i]));
         e += q * q;
     }
     e = sqrt(e * (TIME ? T(0.25) : T(1.0 / 3.0)));
@@ -476,8 +483,9 @@ SIRIUS_HD __forceinline__ int ray_attempt(Ray<T, FAM>& R, const CamConst* cams, 
                                                    r1 - target);
                 land_dense<T, FAM>(R, x1, p1, d1, dn, lo1, th);
             } else {
-                T th = plane ? th_disk : locate_event(s, kind, target, R.x, R.d.k, x1, d1.k, R.h);
-                land<T, FAM>(R, s, plane, th);
+                R.th = plane ? th_disk : locate_event(s, kind, target, R.x, R.d.k, x1, d1.k, R.h);
+                R.cls = ev;
+                return ST_LAND;
             }
         } else {
             R.lam += R.h;
@@ -588,6 +596,7 @@ __device__ __forceinline__ void persistent_body(const CamConst* __restrict__ cam
     Spacetime<T> s;
     if (!MULTI) s = make_spacetime<T>(cams[0]);
     bool active = false;
+    bool pending = false;      // FP64: the lane's ray has ended and waits to be landed
     bool exhausted = false;    // no slot left for this wave: neither reserved nor in the queue
     bool queue_done = false;   // the queue head has passed the list's end
     // slots are 32-bit (work lists hold int32 ray ids); the wave's reserved slots [res_lo, res_hi)
@@ -599,6 +608,13 @@ __device__ __forceinline__ void persistent_body(const CamConst* __restrict__ cam
     while (true) {
         unsigned long long idle = __ballot(!active);
         int n_idle = __popcll(idle);
+        if constexpr (sizeof(T) == 8) {
+            if ((n_idle == 64 || (!exhausted && n_idle >= refill_min)) && pending) {
+                land<T, FAM, EMIT>(R, s);
+                ray_store<T, FAM, EMIT>(R, o, tp);
+                pending = false;
+            }
+        }
         if (n_idle == 64 && exhausted) break;
         if (!exhausted && (n_idle >= refill_min || n_idle == 64)) {
             // idle lane of rank r takes reserved slot res_lo + r while reserved ones last, then
@@ -646,6 +662,8 @@ __device__ __forceinline__ void persistent_body(const CamConst* __restrict__ cam
                 esc_list[k] = (int32_t)R.id;
             } else if (st == ST_DONE) {
                 ray_store<T, FAM, EMIT>(R, o, tp);
+            } else if (st == ST_LAND) {
+                pending = true;
             }
             if (st != ST_RUN) {
                 my_attempts += R.attempts;
@@ -666,12 +684,14 @@ __device__ __forceinline__ void persistent_body(const CamConst* __restrict__ cam
 #define SIRIUS_PERSISTENT_ARGS \
     cams, tp, o, ray_list, list_count, n, head, esc_count, esc_list, attempts_out, refill_min, flag_or
 
-// FP64 variants: register allocation left to the compiler (256 VGPRs plus 6-156 AGPRs, one wave
-// per SIMD). Held to the 256 registers of two waves, the thin-disk tracer spills 34 to scratch
-// and the 1920x1080 Kerr frame slows from 11.3 to 14.9 ms. The single-camera warp tracer, which
-// re-traces wall crossers (a tenth of a warp frame, too few rays to hide one wave's latency), is
-// held to two waves: 268 -> 256 registers with 6 spilled, and the 1024x1024 warp frame goes from
-// 2.79 to 2.54 ms.
+// FP64 variants: register allocation left to the compiler (the thin-disk tracer takes 256 VGPRs plus
+// 20 AGPRs, one wave per SIMD). The single-camera warp tracer, which re-traces wall crossers (a
+// tenth of a warp frame, too few rays to hide one wave's latency), is held to two waves (202
+// registers, no spills). Bound by FP64 issue: with roots and reciprocals by Newton steps, events
+// located by Newton iteration and landings deferred to the refill (land, above), the thin-disk
+// tracer runs the 1283x721 Kerr frame in 5.62 ms (8.99 with IEEE roots and divisions, 52 halvings
+// per event and each ray landed as it ended), the warp tracer its 1024x1024 frame's wall crossers
+// in 0.87 ms (1.65), the wormhole tracer its frame's near-throat rays in 0.41 ms (0.72).
 constexpr int fp64_min_waves(int fam, bool multi) { return fam == 2 && !multi ? 2 : 1; }
 // The persistent tracers start on a 4 KiB boundary of the code object. Their loops are about
 // 19 KiB of instructions, and where the linker happened to place them changed their speed: the
