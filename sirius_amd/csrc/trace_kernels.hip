@@ -885,12 +885,16 @@ __global__ void k_fill_u32(uint32_t* p, int n, uint32_t v) {
 // ------------------------------------------------------------------------------------------
 // Symplectic integrator: Tao (2016) extended phase space (q, p, x, y), Strang split
 // A(h/2) B(h/2) C(h) B(h/2) A(h/2), composed to 4th order with the Yoshida triple jump
-// (weights PHSI001A.h:43-47). Fixed step; disk crossing by linear interpolation.
+// (weights PHSI001A.h:43-47). Fixed step; disk crossing on the cubic Hermite interpolant.
+// Bound by the serial chain of right-hand sides of the longest ray (a 320x181 Kerr frame at
+// h = 0.02 has 905 waves for 1024 SIMDs): 36 ms with 9 evaluations per step and their roots by
+// Newton steps, 63-65 ms with 12 and IEEE roots and divisions.
 // ------------------------------------------------------------------------------------------
-template <class T, int FAM>
-SIRIUS_HD __forceinline__ void tao_a(const Spacetime<T>& s, T d, T q[4], T p[4], T x[4], const T y[4]) {
-    Der<T> D;
-    eval<T, FAM>(s, q, y, D);
+// Flow A with H's derivatives D at (q, y). A changes neither q nor y, so the A that ends a substep
+// and the A that begins the next have the same D: it is evaluated once for both (9 evaluations per
+// Yoshida step instead of 12, the same bits).
+template <class T>
+SIRIUS_HD __forceinline__ void tao_a(const Der<T>& D, T d, T p[4], T x[4]) {
     for (int i = 0; i < 3; ++i) p[i + 1] += d * D.f[i];
     for (int i = 0; i < 4; ++i) x[i] += d * D.k[i];
 }
@@ -931,6 +935,8 @@ __global__ __launch_bounds__(256) void k_symplectic_grid(const CamConst* __restr
     int cls = SIRIUS_RAY_MAX_STEPS;
     T rd = T(0), rprev = event_radius(s, q);
     uint32_t n = 0;
+    Der<T> DA;  // H's derivatives at (q, y)
+    eval<T, FAM>(s, q, y, DA);
     while (n < (uint32_t)tp.max_steps) {
         T q0[4], p0[4];
         for (int i = 0; i < 4; ++i) { q0[i] = q[i]; p0[i] = p[i]; }
@@ -938,11 +944,12 @@ __global__ __launch_bounds__(256) void k_symplectic_grid(const CamConst* __restr
         for (int j = 0; j < subs; ++j) {
             T hj = subs == 3 ? wts[j] * h : h;
             T cj = subs == 3 ? cw[j] : cw2, sj = subs == 3 ? sw[j] : sw2;
-            tao_a<T, FAM>(s, T(0.5) * hj, q, p, x, y);
+            tao_a<T>(DA, T(0.5) * hj, p, x);
             tao_b<T, FAM>(s, T(0.5) * hj, q, p, x, y);
             tao_c<T>(cj, sj, q, p, x, y);
             tao_b<T, FAM>(s, T(0.5) * hj, q, p, x, y);
-            tao_a<T, FAM>(s, T(0.5) * hj, q, p, x, y);
+            eval<T, FAM>(s, q, y, DA);
+            tao_a<T>(DA, T(0.5) * hj, p, x);
         }
         n++;
         R.lam += h;
