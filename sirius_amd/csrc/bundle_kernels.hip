@@ -16,7 +16,7 @@
 // (X, Y) for a ray ending on the thin disk (M per pixel), the deviation there projected along
 // the ray onto the plane.
 //
-// One thread per ray, FP64 values and tangents.
+// Two lanes per ray, one per image axis, FP64 values and tangents.
 #include <hip/hip_runtime.h>
 
 #include "../../include/sirius_hip.h"
@@ -92,59 +92,59 @@ SIRIUS_HD __forceinline__ void ellipse_of(const double m[2][2], double size, flo
 
 }  // namespace
 
+// One pair of neighbouring lanes per ray: lane 0 of the pair carries the deviation d/du, lane 1 d/dv,
+// in one Dual<double, 1> state each. The value parts of both lanes are the same instructions on the
+// same numbers, so the pair takes the same decisions and stays together; what the pair does twice
+// is the values' third of a dual step. Both axes in one lane, one pass after the other, spilled
+// 212-364 bytes per lane (the state, two tangents and their derivatives beside seven stages).
+// A wave's rays that end on the disk are landed together, and the escape angles differenced
+// together, after its last ray has ended. Bound by FP64 issue and by the longest ray's steps: 641x361
+// Kerr rays at the FP32 path's tolerances take 2.15 ms (spill-free at one wave per SIMD; 2.16 at
+// two with 84 bytes spilled), one lane per ray took 4.74 (5.89 with IEEE roots and divisions).
 template <int FAM, int EMIT>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void k_trace_bundle(const CamConst* __restrict__ cams, int n_cam, TraceParams tp,
-                                                     BundleParams bp, BundleOut bo) {
-    const int64_t id = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void k_trace_bundle(
+    const CamConst* __restrict__ cams, int n_cam, TraceParams tp, BundleParams bp, BundleOut bo) {
+    const int64_t id = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 1;
+    const int axis = threadIdx.x & 1;
     if (id >= bo.n) return;
     const CamConst& c = cams[find_cam(cams, n_cam, id)];
     const int64_t pix = id - c.offset;
     const double u0 = (double)(pix % c.width) + 0.5, v0 = (double)(pix / c.width) + 0.5;
-    // one tangent at a time: a Dual<double, 1> pass per image axis keeps the step's seven stage
-    // derivatives in registers (two tangents at once spill); the value parts of both passes are
-    // the same arithmetic, so the central ray is the same in each
     using D = Dual<double, 1>;
     const Spacetime<double> s = make_spacetime<double>(c);
-    const Spacetime<D> sD = make_spacetime<D>(c);
-    double x[4], p[4], t[2][8];
-    Der<D> dA[2];  // FSAL derivative of each pass at the step's start
-    for (int a = 0; a < 2; ++a) {
-        D X[4], P[4];
-        init_state_uv<D>(c, sD, a == 0 ? D::seed(u0, 0) : D(u0), a == 1 ? D::seed(v0, 0) : D(v0), X, P);
-        eval<D, FAM>(sD, X, P, dA[a]);
-        for (int i = 0; i < 4; ++i) {
-            x[i] = X[i].v;
-            p[i] = P[i].v;
-            t[a][i] = X[i].d[0];
-            t[a][4 + i] = P[i].d[0];
-        }
+    D X[4], P[4];
+    Der<D> dA;  // FSAL derivative at the step's start
+    {
+        D u(u0), v(v0);
+        u.d[0] = axis == 0 ? 1.0 : 0.0;
+        v.d[0] = axis == 1 ? 1.0 : 0.0;
+        init_state_uv<D>(c, s, u, v, X, P);
+        X[0].d[0] = 0.0;  // nothing depends on t: its tangent is not carried (here and below)
+        eval<D, FAM>(s, X, P, dA);
     }
-    // the pass of axis a from the current state: state with that tangent, one DP45 step of h
-    auto pass = [&](int a, double hh, D X1[4], D P1[4], Der<D>& d1, D err[4], bool want_err) {
-        D X[4], P[4];
-        for (int i = 0; i < 4; ++i) {
-            X[i] = D(x[i]);
-            X[i].d[0] = t[a][i];
-            P[i] = D(p[i]);
-            P[i].d[0] = t[a][4 + i];
-        }
-        dp45_step<D, FAM, true>(sD, X, P, dA[a], D(hh), X1, P1, d1, err, want_err);
+    auto values = [](const D a[4], double o[4]) {
+        for (int i = 0; i < 4; ++i) o[i] = a[i].v;
     };
-    double h = tp.h_init;
-    if (tp.far_slope > 0) h = fmax(h, fmax(tp.h_max, event_radius(s, x) * tp.far_slope));
+    double h = tp.h_init, r0;
+    {
+        double x[4];
+        values(X, x);
+        r0 = event_radius(s, x);
+    }
+    if (tp.far_slope > 0) h = fmax(h, fmax(tp.h_max, r0 * tp.far_slope));
     int cls = SIRIUS_RAY_MAX_STEPS;
-    double jac[4] = {0, 0, 0, 0};
+    double th_land = 0.0;  // fraction of the step at which a disk ray ends
     uint32_t attempts = 0;
     while (attempts < (uint32_t)tp.max_steps) {
         double hmax = tp.h_max;
-        if (tp.far_slope > 0) hmax = fmax(hmax, event_radius(s, x) * tp.far_slope);
+        if (tp.far_slope > 0) hmax = fmax(hmax, r0 * tp.far_slope);
         D X1[4], P1[4], err[4];
         Der<D> d1;
-        pass(0, h, X1, P1, d1, err, true);
+        dp45_step<D, FAM, true>(s, X, P, dA, h, X1, P1, d1, err, true);
         ++attempts;
         double e = 0;
         for (int i = 0; i < 4; ++i) {
-            const double q = err[i].v / (tp.atol + tp.rtol * fabs(X1[i].v));
+            const double q = err[i].v * rcp_t(tp.atol + tp.rtol * fabs(X1[i].v));
             e += q * q;
         }
         e = sqrt(0.25 * e);
@@ -153,34 +153,23 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
             if (!sfinite(e) || h <= tp.h_min) { cls = SIRIUS_RAY_FAILED; break; }
             continue;
         }
-        double x1[4], p1[4], k0[4], k1[4];
+        double x1[4];
+        values(X1, x1);
         bool bad = false;
-        for (int i = 0; i < 4; ++i) {
-            x1[i] = X1[i].v;
-            p1[i] = P1[i].v;
-            k0[i] = dA[0].k[i].v;
-            k1[i] = d1.k[i].v;
-            bad |= !sfinite(x1[i]) || !sfinite(p1[i]);
-        }
+        for (int i = 0; i < 4; ++i) bad |= !sfinite(x1[i]) || !sfinite(P1[i].v);
         if (bad) { cls = SIRIUS_RAY_FAILED; break; }
-        // thin disk: first crossing inside [r_in, r_out], landed with a DP45 step to the plane
+        // thin disk: first crossing inside [r_in, r_out]
         if constexpr (FAM == 0 && EMIT == SIRIUS_EMISSION_THIN_DISK) {
-            if (x[3] * x1[3] < 0) {
+            if (X[3].v * x1[3] < 0) {
+                double x[4], k0[4], k1[4], xc[4];
+                values(X, x);
+                values(dA.k, k0);
+                values(d1.k, k1);
                 const double th = locate_event(s, EV_Z, 0.0, x, k0, x1, k1, h);
-                double xc[4];
                 hermite(x, k0, x1, k1, h, th, xc);
                 const double rc = kerr_r(s, xc[1], xc[2], xc[3]);
                 if (rc >= c.r_in && rc <= c.r_out) {
-                    // deviation of the hit point: along the ray onto the plane z = 0
-                    for (int a = 0; a < 2; ++a) {
-                        D XL[4], PL[4], el[4];
-                        Der<D> dl;
-                        pass(a, th * h, XL, PL, dl, el, false);
-                        const double kz = dl.k[3].v;
-                        const double dz = fabs(kz) > 1e-300 ? XL[3].d[0] / kz : 0.0;
-                        jac[a] = XL[1].d[0] - dz * dl.k[1].v;
-                        jac[2 + a] = XL[2].d[0] - dz * dl.k[2].v;
-                    }
+                    th_land = th;
                     cls = SIRIUS_RAY_DISK;
                     break;
                 }
@@ -188,50 +177,58 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
         }
         const double r1 = event_radius(s, x1);
         if (FAM == 0 && r1 < c.r_cap) { cls = SIRIUS_RAY_CAPTURED; break; }
-        // accepted: the second axis's pass, then both tangents and FSAL derivatives advance
-        {
-            D X2[4], P2[4], e2[4];
-            Der<D> d2;
-            pass(1, h, X2, P2, d2, e2, false);
-            for (int i = 0; i < 4; ++i) {
-                t[0][i] = X1[i].d[0];
-                t[0][4 + i] = P1[i].d[0];
-                t[1][i] = X2[i].d[0];
-                t[1][4 + i] = P2[i].d[0];
-            }
-            dA[0] = d1;
-            dA[1] = d2;
-        }
-        for (int i = 0; i < 4; ++i) { x[i] = x1[i]; p[i] = p1[i]; }
+        // accepted: the state, its tangent and the FSAL derivative advance
+        for (int i = 0; i < 4; ++i) { X[i] = X1[i]; P[i] = P1[i]; }
+        X[0].d[0] = 0.0;
+        dA = d1;
+        r0 = r1;
         if (r1 > tp.r_escape) {
-            const double radial = (FAM == 1) ? x1[1] * k1[1] : x1[1] * k1[1] + x1[2] * k1[2] + x1[3] * k1[3];
-            if (radial > 0) {
-                // the escape direction (a closed-form function of the final state and, for the
-                // wormhole, of the image point) differentiated along the two deviations
-                for (int a = 0; a < 2; ++a) {
-                    const double eps = fd_eps(x, p, t[a]);
-                    double ang[2][2];
-                    for (int sg = 0; sg < 2; ++sg) {
-                        const double e3 = sg ? -eps : eps;
-                        double xs[4], ps[4];
-                        for (int i = 0; i < 4; ++i) {
-                            xs[i] = x[i] + e3 * t[a][i];
-                            ps[i] = p[i] + e3 * t[a][4 + i];
-                        }
-                        escape_angles<FAM>(c, s, u0 + (a == 0 ? e3 : 0.0), v0 + (a == 1 ? e3 : 0.0), xs, ps,
-                                           ang[sg][0], ang[sg][1]);
-                    }
-                    double dph = ang[0][1] - ang[1][1];
-                    dph = remainder(dph, 2.0 * M_PI);
-                    jac[a] = (ang[0][0] - ang[1][0]) / (2.0 * eps);
-                    jac[2 + a] = dph / (2.0 * eps);
-                }
-                cls = SIRIUS_RAY_ESCAPED;
-                break;
-            }
+            const double radial = (FAM == 1) ? x1[1] * d1.k[1].v : x1[1] * d1.k[1].v + x1[2] * d1.k[2].v + x1[3] * d1.k[3].v;
+            if (radial > 0) { cls = SIRIUS_RAY_ESCAPED; break; }
         }
         h = next_step(h, e, tp.h_min, hmax);
     }
+    // derivative of the outcome along this lane's axis
+    double j0 = 0.0, j1 = 0.0;
+    double x[4], p[4];
+    values(X, x);
+    values(P, p);
+    if (EMIT == SIRIUS_EMISSION_THIN_DISK && cls == SIRIUS_RAY_DISK) {
+        // landed with a DP45 step to the plane; the deviation of the hit point goes along the ray
+        // onto the plane z = 0
+        D XL[4], PL[4], el[4];
+        Der<D> dl;
+        dp45_step<D, FAM, true>(s, X, P, dA, th_land * h, XL, PL, dl, el, false);
+        const double kz = dl.k[3].v;
+        const double dz = fabs(kz) > 1e-300 ? XL[3].d[0] / kz : 0.0;
+        j0 = XL[1].d[0] - dz * dl.k[1].v;
+        j1 = XL[2].d[0] - dz * dl.k[2].v;
+    } else if (cls == SIRIUS_RAY_ESCAPED) {
+        // the escape direction (a closed-form function of the final state and, for the wormhole, of
+        // the image point) differentiated along the deviation
+        double t[8];
+        for (int i = 0; i < 4; ++i) { t[i] = X[i].d[0]; t[4 + i] = P[i].d[0]; }
+        const double eps = fd_eps(x, p, t);
+        double ang[2][2];
+        for (int sg = 0; sg < 2; ++sg) {
+            const double e3 = sg ? -eps : eps;
+            double xs[4], ps[4];
+            for (int i = 0; i < 4; ++i) {
+                xs[i] = x[i] + e3 * t[i];
+                ps[i] = p[i] + e3 * t[4 + i];
+            }
+            escape_angles<FAM>(c, s, u0 + (axis == 0 ? e3 : 0.0), v0 + (axis == 1 ? e3 : 0.0), xs, ps, ang[sg][0],
+                               ang[sg][1]);
+        }
+        double dph = ang[0][1] - ang[1][1];
+        dph = remainder(dph, 2.0 * M_PI);
+        j0 = (ang[0][0] - ang[1][0]) / (2.0 * eps);
+        j1 = dph / (2.0 * eps);
+    }
+    // both lanes hold the whole Jacobian; lane 0 of the pair writes the ray's outputs
+    const double o0 = __shfl_xor(j0, 1), o1 = __shfl_xor(j1, 1);
+    if (axis) return;
+    const double jac[4] = {j0, o0, j1, o1};
     bo.cls[id] = (uint8_t)cls;
     uint8_t flags = 0;
     float beam[3] = {0.f, 0.f, 0.f};
@@ -260,7 +257,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
 hipError_t launch_trace_bundle(int family, int emission, const CamConst* cams, int n_cam, const TraceParams& tp,
                                const BundleParams& bp, const BundleOut& bo, hipStream_t st) {
     if (bo.n <= 0) return hipSuccess;
-    const dim3 grid((unsigned)((bo.n + 63) / 64)), block(64);
+    const dim3 grid((unsigned)((2 * bo.n + 63) / 64)), block(64);  // two lanes per ray
     const bool disk = emission == SIRIUS_EMISSION_THIN_DISK;
     if (family == 1)
         hipLaunchKernelGGL((k_trace_bundle<1, 0>), grid, block, 0, st, cams, n_cam, tp, bp, bo);

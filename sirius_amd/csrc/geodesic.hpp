@@ -226,6 +226,36 @@ template <class T, int N> SIRIUS_HD __forceinline__ Dual<T, N> operator/(const D
     for (int i = 0; i < N; ++i) r.d[i] = (a.d[i] - r.v * b.d[i]) * ib;
     return r;
 }
+// A plain scalar operand has no derivatives: the mixed forms leave its zero tangents out (IEEE rules
+// keep the compiler from dropping 0 * x), so a constant times a dual number is two products, not four
+// operations. S is the scalar type of T (T itself unless T is a dual number).
+template <class T> struct ScalarOf { using type = T; };
+template <class T, int N> struct ScalarOf<Dual<T, N>> { using type = T; };
+template <class T> using scalar_t = typename ScalarOf<T>::type;
+template <class T, int N> SIRIUS_HD __forceinline__ Dual<T, N> operator+(const Dual<T, N>& a, scalar_t<Dual<T, N>> b) {
+    Dual<T, N> r = a;
+    r.v = a.v + b;
+    return r;
+}
+template <class T, int N> SIRIUS_HD __forceinline__ Dual<T, N> operator+(scalar_t<Dual<T, N>> a, const Dual<T, N>& b) { return b + a; }
+template <class T, int N> SIRIUS_HD __forceinline__ Dual<T, N> operator-(const Dual<T, N>& a, scalar_t<Dual<T, N>> b) {
+    Dual<T, N> r = a;
+    r.v = a.v - b;
+    return r;
+}
+template <class T, int N> SIRIUS_HD __forceinline__ Dual<T, N> operator-(scalar_t<Dual<T, N>> a, const Dual<T, N>& b) {
+    Dual<T, N> r = -b;
+    r.v = a - b.v;
+    return r;
+}
+template <class T, int N> SIRIUS_HD __forceinline__ Dual<T, N> operator*(const Dual<T, N>& a, scalar_t<Dual<T, N>> b) {
+    Dual<T, N> r;
+    r.v = a.v * b;
+    for (int i = 0; i < N; ++i) r.d[i] = a.d[i] * b;
+    return r;
+}
+template <class T, int N> SIRIUS_HD __forceinline__ Dual<T, N> operator*(scalar_t<Dual<T, N>> a, const Dual<T, N>& b) { return b * a; }
+template <class T, int N> SIRIUS_HD __forceinline__ Dual<T, N> operator/(const Dual<T, N>& a, scalar_t<Dual<T, N>> b) { return a * (T(1) / b); }
 template <class T, int N> SIRIUS_HD __forceinline__ bool operator<(const Dual<T, N>& a, const Dual<T, N>& b) { return a.v < b.v; }
 template <class T, int N> SIRIUS_HD __forceinline__ bool operator>(const Dual<T, N>& a, const Dual<T, N>& b) { return a.v > b.v; }
 template <class T, int N> SIRIUS_HD __forceinline__ bool operator<=(const Dual<T, N>& a, const Dual<T, N>& b) { return a.v <= b.v; }
@@ -263,6 +293,7 @@ template <class T, int N> SIRIUS_HD __forceinline__ Dual<T, N> sqrt_from(const D
 }
 template <class T, int N> SIRIUS_HD __forceinline__ Dual<T, N> fabs(const Dual<T, N>& a) { return a.v < T(0) ? -a : a; }
 template <class T, int N> SIRIUS_HD __forceinline__ Dual<T, N> fmax(const Dual<T, N>& a, const Dual<T, N>& b) { return a.v < b.v ? b : a; }
+template <class T, int N> SIRIUS_HD __forceinline__ Dual<T, N> fmax(const Dual<T, N>& a, scalar_t<Dual<T, N>> b) { return a.v < b ? Dual<T, N>(b) : a; }
 template <class T, int N> SIRIUS_HD __forceinline__ Dual<T, N> fmin(const Dual<T, N>& a, const Dual<T, N>& b) { return b.v < a.v ? b : a; }
 template <class T, int N> SIRIUS_HD __forceinline__ Dual<T, N> exp(const Dual<T, N>& a) {
     const T e = exp(a.v);
@@ -276,6 +307,12 @@ template <class T, int N> SIRIUS_HD __forceinline__ Dual<T, N> fma(const Dual<T,
     Dual<T, N> r;
     r.v = fma(a.v, b.v, c.v);
     for (int i = 0; i < N; ++i) r.d[i] = a.d[i] * b.v + a.v * b.d[i] + c.d[i];
+    return r;
+}
+template <class T, int N> SIRIUS_HD __forceinline__ Dual<T, N> tfma(scalar_t<Dual<T, N>> a, const Dual<T, N>& b, const Dual<T, N>& c) {
+    Dual<T, N> r;
+    r.v = fma(a, b.v, c.v);
+    for (int i = 0; i < N; ++i) r.d[i] = fma(a, b.d[i], c.d[i]);
     return r;
 }
 
@@ -308,13 +345,14 @@ SIRIUS_HD __forceinline__ Spacetime<T> make_spacetime(const CamConst& c) {
 // varies, so it keeps the digits the tanh of sigma (r_s - R) keeps; E v = e^{-2 sigma (r_s + R)}
 // and E v^2 = e^{-4 sigma r_s} stay below one, and v below e^{2 sigma R} (sigma R <= 40).
 template <class T>
-SIRIUS_HD __forceinline__ T warp_shape(const Spacetime<T>& s, T rs, T& dfdr) {
-    const T v = exp(-T(2) * s.wsig * (rs - s.wR));
+SIRIUS_HD __forceinline__ T warp_shape(const Spacetime<scalar_t<T>>& s, T rs, T& dfdr) {
+    using S = scalar_t<T>;
+    const T v = exp(-S(2) * s.wsig * (rs - s.wR));
     const T ev = s.wE * v;
-    const T D = tfma(v, T(1) + s.wE + ev, T(1));
+    const T D = tfma(v, S(1) + s.wE + ev, T(1));
     const T iD = T(1) / D;
     const T f = s.wN * v * iD;
-    dfdr = -T(2) * s.wsig * f * (T(1) - ev * v) * iD;
+    dfdr = -S(2) * s.wsig * f * (S(1) - ev * v) * iD;
     return f;
 }
 
@@ -397,25 +435,26 @@ SIRIUS_HD __forceinline__ void metric_cov(const Spacetime<T>& s, const T x[4], T
 // Returns p.k = g_{mu nu} k^mu k^nu (the null-constraint value).
 // ------------------------------------------------------------------------------------------
 template <class T>
-SIRIUS_HD __forceinline__ T rhs_ks(const Spacetime<T>& s, const T x[4], const T p[4], T k[4], T dp[3]) {
+SIRIUS_HD __forceinline__ T rhs_ks(const Spacetime<scalar_t<T>>& s, const T x[4], const T p[4], T k[4], T dp[3]) {
     // Hamilton's equations for H = (eta^{mu nu} - H l^mu l^nu) p_mu p_nu / 2 with the position
     // gradient in closed form. r depends on (x, y, z) through r^4 - (R^2 - a^2) r^2 - a^2 z^2 = 0:
     //   dr/dx = x r / s, dr/dy = y r / s, dr/dz = z (r^2 + a^2) / (r s),
     //   s = sqrt((R^2 - a^2)^2 + 4 a^2 z^2) = 2 r^2 - R^2 + a^2;
     // then dH_i = H_r dr_i + H_z [i = z] and sum_j k_j d_i l_j = A_i + B dr_i.
+    using S = scalar_t<T>;
     const T X = x[1], Y = x[2], Z = x[3];
     const T R2v = X * X + Y * Y + Z * Z;
     const T w = R2v - s.a2;                           // R^2 - a^2
-    T disc = tfma(T(4) * s.a2, Z * Z, w * w);         // (R^2 - a^2)^2 + 4 a^2 z^2
-    disc = fmax(disc, T(1e-20));  // guards only the ring singularity, deep inside the horizon
+    T disc = tfma(S(4) * s.a2, Z * Z, w * w);         // (R^2 - a^2)^2 + 4 a^2 z^2
+    disc = fmax(disc, S(1e-20));  // guards only the ring singularity, deep inside the horizon
     // square roots and their reciprocals from one reciprocal square root each, and 1 / rho, 1 / Dn
     // from one reciprocal of their product (three transcendental instructions instead of six or,
     // in FP64, two IEEE roots and five IEEE divisions: a third of the FP64 right-hand side's
     // instructions; rho Dn ~ r^6 stays far inside the FP32 range for r < 1e6)
     const T isq = rsqrt_t(disc);
     const T sq = sqrt_from(disc, isq);
-    T r2 = (w + sq) * T(0.5);
-    r2 = fmax(r2, T(1e-10));
+    T r2 = (w + sq) * S(0.5);
+    r2 = fmax(r2, S(1e-10));
     const T ir = rsqrt_t(r2);
     const T r = sqrt_from(r2, ir);
     const T rho = r2 + s.a2;
@@ -426,7 +465,7 @@ SIRIUS_HD __forceinline__ T rhs_ks(const Spacetime<T>& s, const T x[4], const T 
     const T l1 = tfma(r, X, s.a * Y) * irho;          // (r x + a y) / (r^2 + a^2)
     const T l2 = tfma(r, Y, -s.a * X) * irho;         // (r y - a x) / (r^2 + a^2)
     const T l3 = Z * ir;                              // z / r
-    const T q = T(2) * s.M * r - s.Q2;                // 2 M r - Q^2
+    const T q = S(2) * s.M * r - s.Q2;                // 2 M r - Q^2
     const T H = q * r2 * iDn;
     // k = (eta - H l l) p, l^mu = (-1, l1, l2, l3)
     T lp = -p[0] + l1 * p[1] + l2 * p[2] + l3 * p[3];
@@ -435,29 +474,29 @@ SIRIUS_HD __forceinline__ T rhs_ks(const Spacetime<T>& s, const T x[4], const T 
     k[1] = p[1] - Hl * l1;
     k[2] = p[2] - Hl * l2;
     k[3] = p[3] - Hl * l3;
-    T lam3 = T(0);
-    if (s.Lambda != T(0)) {
+    S lam3 = S(0);
+    if (s.Lambda != S(0)) {
         // g = g0 + c e0 e0^T with c = -Lambda R^2 / 3; g^-1 by Sherman-Morrison.
-        T c = -s.Lambda * R2v / T(3);
-        T u0 = -T(1) - H;
-        T fac = c * k[0] / (T(1) + c * u0);
+        T c = -s.Lambda * R2v / S(3);
+        T u0 = -S(1) - H;
+        T fac = c * k[0] / (S(1) + c * u0);
         k[0] -= fac * u0;
         k[1] -= fac * H * l1;
         k[2] -= fac * H * l2;
         k[3] -= fac * H * l3;
-        lam3 = s.Lambda / T(3);
+        lam3 = s.Lambda / S(3);
     }
     T lk = k[0] + l1 * k[1] + l2 * k[2] + l3 * k[3];
-    T hl = T(0.5) * lk * lk, Hlk = H * lk, k00 = k[0] * k[0];
+    T hl = S(0.5) * lk * lk, Hlk = H * lk, k00 = k[0] * k[0];
     // gradient of r
     const T rs = r * isq;
     const T drx = X * rs, dry = Y * rs, drz = Z * rho * ir * isq;
     // H_r = (N_r - H Dn_r) / Dn with N = q r^2, N_r = r (6 M r - 2 Q^2), Dn_r = 4 r^3;
     // H_z = -2 a^2 z H / Dn
-    const T Hr = (r * (T(6) * s.M * r - T(2) * s.Q2) - H * T(4) * r2 * r) * iDn;
-    const T Hz = -T(2) * s.a2 * Z * H * iDn;
+    const T Hr = (r * (S(6) * s.M * r - S(2) * s.Q2) - H * S(4) * r2 * r) * iDn;
+    const T Hz = -S(2) * s.a2 * Z * H * iDn;
     const T A1 = (k[1] * r - k[2] * s.a) * irho, A2 = (k[1] * s.a + k[2] * r) * irho, A3 = k[3] * ir;
-    const T B = (k[1] * X + k[2] * Y - T(2) * r * (k[1] * l1 + k[2] * l2)) * irho - k[3] * l3 * ir;
+    const T B = (k[1] * X + k[2] * Y - S(2) * r * (k[1] * l1 + k[2] * l2)) * irho - k[3] * l3 * ir;
     const T Cr = hl * Hr + Hlk * B;
     dp[0] = Cr * drx + Hlk * A1 - lam3 * X * k00;
     dp[1] = Cr * dry + Hlk * A2 - lam3 * Y * k00;
@@ -467,7 +506,7 @@ SIRIUS_HD __forceinline__ T rhs_ks(const Spacetime<T>& s, const T x[4], const T 
 
 // Ellis wormhole, orbital-plane reduction (t, l, psi, w): g = diag(-1, 1, l^2 + b0^2, 1).
 template <class T>
-SIRIUS_HD __forceinline__ T rhs_mt(const Spacetime<T>& s, const T x[4], const T p[4], T k[4], T dp[3]) {
+SIRIUS_HD __forceinline__ T rhs_mt(const Spacetime<scalar_t<T>>& s, const T x[4], const T p[4], T k[4], T dp[3]) {
     T r2 = x[1] * x[1] + s.b02;
     k[0] = -p[0];
     k[1] = p[1];
@@ -481,7 +520,8 @@ SIRIUS_HD __forceinline__ T rhs_mt(const Spacetime<T>& s, const T x[4], const T 
 
 // Alcubierre, static bubble: g^{00} = -1, g^{01} = -v f, g^{11} = 1 - v^2 f^2.
 template <class T>
-SIRIUS_HD __forceinline__ T rhs_warp(const Spacetime<T>& s, const T x[4], const T p[4], T k[4], T dp[3]) {
+SIRIUS_HD __forceinline__ T rhs_warp(const Spacetime<scalar_t<T>>& s, const T x[4], const T p[4], T k[4], T dp[3]) {
+    using S = scalar_t<T>;
     T R2 = x[1] * x[1] + x[2] * x[2] + x[3] * x[3];
     R2 = R2 < T(1e-20) ? T(1e-20) : R2;
     T rs = sqrt(R2);
@@ -489,7 +529,7 @@ SIRIUS_HD __forceinline__ T rhs_warp(const Spacetime<T>& s, const T x[4], const 
     T f = warp_shape(s, rs, dfdr);
     T vf = s.wv * f;
     k[0] = -p[0] - vf * p[1];
-    k[1] = -vf * p[0] + (T(1) - vf * vf) * p[1];
+    k[1] = -vf * p[0] + (S(1) - vf * vf) * p[1];
     k[2] = p[2];
     k[3] = p[3];
     T c = s.wv * dfdr / rs * (vf * k[0] * k[0] - k[0] * k[1]);
@@ -500,7 +540,7 @@ SIRIUS_HD __forceinline__ T rhs_warp(const Spacetime<T>& s, const T x[4], const 
 }
 
 template <class T, int FAM>
-SIRIUS_HD __forceinline__ T rhs(const Spacetime<T>& s, const T x[4], const T p[4], T k[4], T dp[3]) {
+SIRIUS_HD __forceinline__ T rhs(const Spacetime<scalar_t<T>>& s, const T x[4], const T p[4], T k[4], T dp[3]) {
     if constexpr (FAM == 1) return rhs_mt<T>(s, x, p, k, dp);
     else if constexpr (FAM == 2) return rhs_warp<T>(s, x, p, k, dp);
     else return rhs_ks<T>(s, x, p, k, dp);
@@ -551,7 +591,7 @@ struct Der {
 };
 
 template <class T, int FAM>
-SIRIUS_HD __forceinline__ void eval(const Spacetime<T>& s, const T x[4], const T p[4], Der<T>& d) {
+SIRIUS_HD __forceinline__ void eval(const Spacetime<scalar_t<T>>& s, const T x[4], const T p[4], Der<T>& d) {
     d.pk = rhs<T, FAM>(s, x, p, d.k, d.f);
 }
 
@@ -585,9 +625,10 @@ SIRIUS_HD __forceinline__ T sum_lo(T y0, T inc, const T* lo, T* lo1, int j) {
 // accumulated with an error-free sum whose low parts go to lo1. The FP32 path keeps its state
 // this way, so rounding of the position and momentum does not accumulate along the ray.
 template <class T, int FAM, bool TIME = true>
-SIRIUS_HD __forceinline__ void dp45_step(const Spacetime<T>& s, const T x0[4], const T p0[4], const Der<T>& d1,
-                                 T h, T x1[4], T p1[4], Der<T>& d7, T err[4], bool want_err,
+SIRIUS_HD __forceinline__ void dp45_step(const Spacetime<scalar_t<T>>& s, const T x0[4], const T p0[4], const Der<T>& d1,
+                                 scalar_t<T> h, T x1[4], T p1[4], Der<T>& d7, T err[4], bool want_err,
                                  T* dense = nullptr, const T* lo = nullptr, T* lo1 = nullptr) {
+    using S = scalar_t<T>;
     constexpr double a21 = 1.0 / 5.0;
     constexpr double a31 = 3.0 / 40.0, a32 = 9.0 / 40.0;
     constexpr double a41 = 44.0 / 45.0, a42 = -56.0 / 15.0, a43 = 32.0 / 9.0;
@@ -605,50 +646,50 @@ SIRIUS_HD __forceinline__ void dp45_step(const Spacetime<T>& s, const T x0[4], c
     xt[0] = x0[0];
     x1[0] = x0[0];
 #pragma unroll
-    for (int i = I0; i < 4; ++i) xt[i] = stage_pt(x0[i], h * (T(a21) * d1.k[i]), lo, i);
+    for (int i = I0; i < 4; ++i) xt[i] = stage_pt(x0[i], h * (S(a21) * d1.k[i]), lo, i);
 #pragma unroll
-    for (int i = 0; i < 3; ++i) pt[i + 1] = stage_pt(p0[i + 1], h * (T(a21) * d1.f[i]), lo, 5 + i);
+    for (int i = 0; i < 3; ++i) pt[i + 1] = stage_pt(p0[i + 1], h * (S(a21) * d1.f[i]), lo, 5 + i);
     eval<T, FAM>(s, xt, pt, d2);
 #pragma unroll
-    for (int i = I0; i < 4; ++i) xt[i] = stage_pt(x0[i], h * (T(a31) * d1.k[i] + T(a32) * d2.k[i]), lo, i);
+    for (int i = I0; i < 4; ++i) xt[i] = stage_pt(x0[i], h * (S(a31) * d1.k[i] + S(a32) * d2.k[i]), lo, i);
 #pragma unroll
-    for (int i = 0; i < 3; ++i) pt[i + 1] = stage_pt(p0[i + 1], h * (T(a31) * d1.f[i] + T(a32) * d2.f[i]), lo, 5 + i);
+    for (int i = 0; i < 3; ++i) pt[i + 1] = stage_pt(p0[i + 1], h * (S(a31) * d1.f[i] + S(a32) * d2.f[i]), lo, 5 + i);
     eval<T, FAM>(s, xt, pt, d3);
 #pragma unroll
-    for (int i = I0; i < 4; ++i) xt[i] = stage_pt(x0[i], h * (T(a41) * d1.k[i] + T(a42) * d2.k[i] + T(a43) * d3.k[i]), lo, i);
+    for (int i = I0; i < 4; ++i) xt[i] = stage_pt(x0[i], h * (S(a41) * d1.k[i] + S(a42) * d2.k[i] + S(a43) * d3.k[i]), lo, i);
 #pragma unroll
-    for (int i = 0; i < 3; ++i) pt[i + 1] = stage_pt(p0[i + 1], h * (T(a41) * d1.f[i] + T(a42) * d2.f[i] + T(a43) * d3.f[i]), lo, 5 + i);
+    for (int i = 0; i < 3; ++i) pt[i + 1] = stage_pt(p0[i + 1], h * (S(a41) * d1.f[i] + S(a42) * d2.f[i] + S(a43) * d3.f[i]), lo, 5 + i);
     eval<T, FAM>(s, xt, pt, d4);
 #pragma unroll
     for (int i = I0; i < 4; ++i)
-        xt[i] = stage_pt(x0[i], h * (T(a51) * d1.k[i] + T(a52) * d2.k[i] + T(a53) * d3.k[i] + T(a54) * d4.k[i]), lo, i);
+        xt[i] = stage_pt(x0[i], h * (S(a51) * d1.k[i] + S(a52) * d2.k[i] + S(a53) * d3.k[i] + S(a54) * d4.k[i]), lo, i);
 #pragma unroll
     for (int i = 0; i < 3; ++i)
-        pt[i + 1] = stage_pt(p0[i + 1], h * (T(a51) * d1.f[i] + T(a52) * d2.f[i] + T(a53) * d3.f[i] + T(a54) * d4.f[i]), lo, 5 + i);
+        pt[i + 1] = stage_pt(p0[i + 1], h * (S(a51) * d1.f[i] + S(a52) * d2.f[i] + S(a53) * d3.f[i] + S(a54) * d4.f[i]), lo, 5 + i);
     eval<T, FAM>(s, xt, pt, d5);
 #pragma unroll
     for (int i = I0; i < 4; ++i)
-        xt[i] = stage_pt(x0[i], h * (T(a61) * d1.k[i] + T(a62) * d2.k[i] + T(a63) * d3.k[i] + T(a64) * d4.k[i] + T(a65) * d5.k[i]), lo, i);
+        xt[i] = stage_pt(x0[i], h * (S(a61) * d1.k[i] + S(a62) * d2.k[i] + S(a63) * d3.k[i] + S(a64) * d4.k[i] + S(a65) * d5.k[i]), lo, i);
 #pragma unroll
     for (int i = 0; i < 3; ++i)
-        pt[i + 1] = stage_pt(p0[i + 1], h * (T(a61) * d1.f[i] + T(a62) * d2.f[i] + T(a63) * d3.f[i] + T(a64) * d4.f[i] + T(a65) * d5.f[i]), lo, 5 + i);
+        pt[i + 1] = stage_pt(p0[i + 1], h * (S(a61) * d1.f[i] + S(a62) * d2.f[i] + S(a63) * d3.f[i] + S(a64) * d4.f[i] + S(a65) * d5.f[i]), lo, 5 + i);
     eval<T, FAM>(s, xt, pt, d6);
     p1[0] = p0[0];
 #pragma unroll
     for (int i = I0; i < 4; ++i)
-        x1[i] = sum_lo(x0[i], h * (T(b1) * d1.k[i] + T(b3) * d3.k[i] + T(b4) * d4.k[i] + T(b5) * d5.k[i] +
-                                   T(b6) * d6.k[i]), lo, lo1, i);
+        x1[i] = sum_lo(x0[i], h * (S(b1) * d1.k[i] + S(b3) * d3.k[i] + S(b4) * d4.k[i] + S(b5) * d5.k[i] +
+                                   S(b6) * d6.k[i]), lo, lo1, i);
 #pragma unroll
     for (int i = 0; i < 3; ++i)
-        p1[i + 1] = sum_lo(p0[i + 1], h * (T(b1) * d1.f[i] + T(b3) * d3.f[i] + T(b4) * d4.f[i] + T(b5) * d5.f[i] +
-                                           T(b6) * d6.f[i]), lo, lo1, 5 + i);
+        p1[i + 1] = sum_lo(p0[i + 1], h * (S(b1) * d1.f[i] + S(b3) * d3.f[i] + S(b4) * d4.f[i] + S(b5) * d5.f[i] +
+                                           S(b6) * d6.f[i]), lo, lo1, 5 + i);
     eval<T, FAM>(s, x1, p1, d7);
     if (want_err) {
         err[0] = T(0);
 #pragma unroll
         for (int i = I0; i < 4; ++i)
-            err[i] = h * (T(e1) * d1.k[i] + T(e3) * d3.k[i] + T(e4) * d4.k[i] + T(e5) * d5.k[i] + T(e6) * d6.k[i] +
-                          T(e7) * d7.k[i]);
+            err[i] = h * (S(e1) * d1.k[i] + S(e3) * d3.k[i] + S(e4) * d4.k[i] + S(e5) * d5.k[i] + S(e6) * d6.k[i] +
+                          S(e7) * d7.k[i]);
     }
     if (dense) {
         // Dormand-Prince continuous extension of order 4 (Hairer, Norsett & Wanner, Solving
@@ -658,10 +699,10 @@ SIRIUS_HD __forceinline__ void dp45_step(const Spacetime<T>& s, const T x0[4], c
                          q6 = -1453857185.0 / 822651844.0, q7 = 69997945.0 / 29380423.0;
 #pragma unroll
         for (int i = 0; i < 3; ++i) {
-            dense[i] = h * (T(q1) * d1.k[i + 1] + T(q3) * d3.k[i + 1] + T(q4) * d4.k[i + 1] + T(q5) * d5.k[i + 1] +
-                            T(q6) * d6.k[i + 1] + T(q7) * d7.k[i + 1]);
-            dense[3 + i] = h * (T(q1) * d1.f[i] + T(q3) * d3.f[i] + T(q4) * d4.f[i] + T(q5) * d5.f[i] +
-                                T(q6) * d6.f[i] + T(q7) * d7.f[i]);
+            dense[i] = h * (S(q1) * d1.k[i + 1] + S(q3) * d3.k[i + 1] + S(q4) * d4.k[i + 1] + S(q5) * d5.k[i + 1] +
+                            S(q6) * d6.k[i + 1] + S(q7) * d7.k[i + 1]);
+            dense[3 + i] = h * (S(q1) * d1.f[i] + S(q3) * d3.f[i] + S(q4) * d4.f[i] + S(q5) * d5.f[i] +
+                                S(q6) * d6.f[i] + S(q7) * d7.f[i]);
         }
     }
 }
@@ -919,7 +960,7 @@ SIRIUS_HD __forceinline__ void camera_cart_dir(const CamConst& c, int px, int py
 }
 
 template <class T>
-SIRIUS_HD __forceinline__ void init_state_ns(const CamConst& c, const Spacetime<T>& s, const T ns[3], T x[4], T p[4]) {
+SIRIUS_HD __forceinline__ void init_state_ns(const CamConst& c, const Spacetime<scalar_t<T>>& s, const T ns[3], T x[4], T p[4]) {
     T k[4], g[4][4];
     if (c.family == 1) {
         T nr, nt;
@@ -950,7 +991,7 @@ SIRIUS_HD __forceinline__ void init_state_ns(const CamConst& c, const Spacetime<
 }
 
 template <class T>
-SIRIUS_HD __forceinline__ void init_state(const CamConst& c, const Spacetime<T>& s, int px, int py, T x[4], T p[4]) {
+SIRIUS_HD __forceinline__ void init_state(const CamConst& c, const Spacetime<scalar_t<T>>& s, int px, int py, T x[4], T p[4]) {
     T ns[3];
     camera_dir<T>(c, px, py, ns);
     init_state_ns<T>(c, s, ns, x, p);
@@ -958,7 +999,7 @@ SIRIUS_HD __forceinline__ void init_state(const CamConst& c, const Spacetime<T>&
 
 // Initial state of the ray through the image point (u, v) (pixel units).
 template <class T>
-SIRIUS_HD __forceinline__ void init_state_uv(const CamConst& c, const Spacetime<T>& s, T u, T v, T x[4], T p[4]) {
+SIRIUS_HD __forceinline__ void init_state_uv(const CamConst& c, const Spacetime<scalar_t<T>>& s, T u, T v, T x[4], T p[4]) {
     T ns[3];
     camera_dir_uv<T>(c, u, v, ns);
     init_state_ns<T>(c, s, ns, x, p);
