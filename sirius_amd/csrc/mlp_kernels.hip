@@ -1,19 +1,12 @@
-// mlp_kernels.hip — BF16 MFMA kernels of the far-field surrogate network (gfx950).
-//
-// One GEMM kernel serves every layer, forward and backward: a 256-thread block computes a
-// 64 x 64 tile of C as four 32 x 32 wave tiles with v_mfma_f32_32x32x8_bf16 (wave64; A and B
-// fragments are 4 BF16 values per lane, C is 16 FP32 values per lane). Tiles of A (64 x 32)
-// and B (32 x 64) are staged through LDS with 16-byte global loads along each operand's
-// contiguous dimension, so transposed operands (the backward pass) cost no extra pass over
-// memory. Epilogues fuse bias + GELU + BF16 rounding (forward), the GELU derivative
-// (backward), or write split-K partials (weight gradients, reduced deterministically).
+// mlp_kernels.hip — BF16 MFMA kernels of the far-field surrogate network (gfx950): fused inference,
+// and the training step's loss and gradient (three kernels), its Adam update and the packing of
+// the weights into MFMA fragment order.
 #include <hip/hip_runtime.h>
 
 #include "mlp.hpp"
 
 namespace sirius {
 
-typedef short v4s __attribute__((ext_vector_type(4)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 
 // FP32 -> BF16, round to nearest even (NaN/Inf pass through)
@@ -34,85 +27,6 @@ __device__ __forceinline__ float gelu_f(float z) {
 __device__ __forceinline__ float gelu_df(float z) {
     float t = tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z));
     return 0.5f * (1.f + t) + 0.5f * z * (1.f - t * t) * 0.7978845608028654f * (1.f + 3.f * 0.044715f * z * z);
-}
-
-constexpr int LDS_PITCH = 40;  // halves per LDS row: 32 + 8 pad keeps 16-byte alignment (80 B)
-
-template <int EPI>
-__global__ __launch_bounds__(256) void k_gemm(GemmArgs g) {
-    __shared__ __attribute__((aligned(16))) uint16_t As[64 * LDS_PITCH];  // As[i][k]
-    __shared__ __attribute__((aligned(16))) uint16_t Bs[64 * LDS_PITCH];  // Bs[j][k]
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    const int row0 = blockIdx.y * 64, col0 = blockIdx.x * 64;
-    const int wr = (wave >> 1) * 32, wc = (wave & 1) * 32;
-    const int kbeg = blockIdx.z * g.kchunk;
-    const int kend = min(g.K, kbeg + g.kchunk);
-    v16f acc;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
-    for (int k0 = kbeg; k0 < kend; k0 += 32) {
-        if (g.sak == 1) {  // A contiguous along k: row t/4, k 8*(t%4) .. +7
-            const int r = t >> 2, kk = (t & 3) * 8;
-            *(uint4*)&As[r * LDS_PITCH + kk] = *(const uint4*)(g.A + (int64_t)(row0 + r) * g.sai + k0 + kk);
-        } else {  // A contiguous along i: k t/8, rows 8*(t%8) .. +7
-            const int kk = t >> 3, r = (t & 7) * 8;
-            uint4 v = *(const uint4*)(g.A + (int64_t)(k0 + kk) * g.sak + row0 + r);
-            const uint16_t* e = (const uint16_t*)&v;
-#pragma unroll
-            for (int q = 0; q < 8; ++q) As[(r + q) * LDS_PITCH + kk] = e[q];
-        }
-        if (g.sbk == 1) {  // B contiguous along k: column t/4, k 8*(t%4) .. +7
-            const int j = t >> 2, kk = (t & 3) * 8;
-            *(uint4*)&Bs[j * LDS_PITCH + kk] = *(const uint4*)(g.B + (int64_t)(col0 + j) * g.sbj + k0 + kk);
-        } else {  // B contiguous along j: k t/8, columns 8*(t%8) .. +7
-            const int kk = t >> 3, j = (t & 7) * 8;
-            uint4 v = *(const uint4*)(g.B + (int64_t)(k0 + kk) * g.sbk + col0 + j);
-            const uint16_t* e = (const uint16_t*)&v;
-#pragma unroll
-            for (int q = 0; q < 8; ++q) Bs[(j + q) * LDS_PITCH + kk] = e[q];
-        }
-        __syncthreads();
-#pragma unroll
-        for (int kk = 0; kk < 32; kk += 8) {
-            const int ko = kk + 4 * (lane >> 5);
-            v4s a = *(const v4s*)&As[(wr + (lane & 31)) * LDS_PITCH + ko];
-            v4s b = *(const v4s*)&Bs[(wc + (lane & 31)) * LDS_PITCH + ko];
-            acc = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(a, b, acc, 0, 0, 0);
-        }
-        __syncthreads();
-    }
-    // C fragment: lane holds column wc + lane % 32, rows 8 (r / 4) + 4 (lane / 32) + r % 4
-    const int j = col0 + wc + (lane & 31);
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        const int i = row0 + wr + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-        const int64_t o = (int64_t)i * g.N + j;
-        const float v = acc[r];
-        if constexpr (EPI == EPI_HIDDEN) {
-            const float z = v + g.bias[j];
-            if (g.zout) g.zout[o] = z;
-            g.hout[o] = f2bf(gelu_f(z));
-        } else if constexpr (EPI == EPI_OUT) {
-            g.out[o] = v + g.bias[j];
-        } else if constexpr (EPI == EPI_BWD) {
-            const float gz = v * gelu_df(g.zin[o]);
-            g.gzf[o] = gz;
-            g.gzb[o] = f2bf(gz);
-        } else {
-            g.out[(int64_t)blockIdx.z * g.M * g.N + o] = v;
-        }
-    }
-}
-
-hipError_t launch_gemm(int epi, const GemmArgs& g, int nsplit, hipStream_t st) {
-    dim3 grid((unsigned)(g.N / 64), (unsigned)(g.M / 64), (unsigned)nsplit), block(256);
-    switch (epi) {
-        case EPI_HIDDEN: hipLaunchKernelGGL(k_gemm<EPI_HIDDEN>, grid, block, 0, st, g); break;
-        case EPI_OUT: hipLaunchKernelGGL(k_gemm<EPI_OUT>, grid, block, 0, st, g); break;
-        case EPI_BWD: hipLaunchKernelGGL(k_gemm<EPI_BWD>, grid, block, 0, st, g); break;
-        default: hipLaunchKernelGGL(k_gemm<EPI_PART>, grid, block, 0, st, g); break;
-    }
-    return hipGetLastError();
 }
 
 // ------------------------------------------------------------------------------------------
@@ -309,102 +223,396 @@ hipError_t launch_mlp_fused(const MlpFusedArgs& a, int64_t cap, int max_blocks, 
 }
 
 // ------------------------------------------------------------------------------------------
-// The output head in FP32 for training (the fused inference keeps FP32 precision with split
-// BF16 products): h4 = gelu(z3) from the stored pre-activations, W4 the FP32 masters.
+// Training: loss and gradient of a batch in three kernels.
+//
+// k_mlp_train runs the whole network forward and backward for 32 samples per block: 8 waves, wave w
+// owning neurons 32 w .. 32 w + 31 of each layer. Samples are the rows of each product
+// (v_mfma_f32_32x32x16_bf16, A the tile's activations from LDS, B the weights in fragment order),
+// so a lane's accumulators hold one neuron j = 32 w + l % 32 for the 16 samples
+// 8 q + 4 (l / 32) + e. Packed to BF16 these registers are an operand of the weight-gradient
+// product as they stand (8 samples of one neuron): they go to memory as fragments, without a
+// transpose. The layer's outputs also go back to LDS, row = sample, for the next layer, and the
+// GELU derivatives stay in LDS, 16 per thread and layer, until the backward pass. Each product sums
+// its k dimension in ascending order into one accumulator, as the hidden layers of the fused
+// inference kernel do. The output head is FP32. The layers are loops and the derivatives' hyperbolic
+// tangents are too: a block runs its code once, and unrolled (72 KB of instructions) the kernel
+// spent its time fetching them: 61 us against 39 for 8192 rows (one block per CU; what is left is the
+// chain of one block: the derivatives' tangents, the barriers and the weights' loads).
+// Sums over samples whose result is small (every bias, the head's and the first layer's weights,
+// the loss) leave one row of MLP_TILE_COLS partials per tile.
+//
+// k_mlp_wgrad forms dW_l = gz_l^T h_l of the three 256 x 256 layers from those fragments, split
+// over the samples; k_mlp_grad_sum adds the splits and the tiles' rows in a fixed order.
+//
+// A batch of 8192 rows has 9.8 GFLOP of work and 1.9 MB of inputs and outputs (8 us at the rate of a
+// large matrix product): launches, latency and the fragments' traffic bound it. 32 kernels with the
+// activations and pre-activations in FP32 in memory took 490 us per call; these take 63 (39 + 10 + 6
+// and the launches). 256 rows took 393 us and take 50, 65536 rows take 357.
 // ------------------------------------------------------------------------------------------
-// y64[i][o] = b4[o] + sum_k h4[i][k] W4[o][k] (o < 6; columns 6..63 zero). One wave per row
-// group: each lane takes four k, the six partial sums are reduced across the wave.
-__global__ __launch_bounds__(256) void k_head_fwd(const float* __restrict__ z3, const float* __restrict__ W4,
-                                                  const float* __restrict__ b4, int64_t n_pad, float* __restrict__ y64) {
-    const int lane = threadIdx.x & 63;
-    const int64_t i = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (i >= n_pad) return;
-    float part[SIRIUS_MLP_OUT] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+constexpr int TR_ROWS = MLP_TRAIN_ROWS;
+constexpr int TR_THREADS = 512;
+constexpr int TR_PITCH = 264;     // BF16 values per LDS row: 16-byte reads of 8 lanes cover every bank once
+constexpr int TR_H4_PITCH = 260;  // floats per LDS row of the last hidden activation
+static_assert(TR_ROWS == 32 && MLP_H == 256, "one 32 x 32 product per wave and k step");
+static_assert(TR_ROWS * TR_H4_PITCH * 4 <= 2 * TR_ROWS * TR_PITCH * 2, "the last activation fits the two tiles");
+
+// The wave's 16 B fragments of a packed 256 x 256 matrix (k_pack_fused), one per k step: `stride`
+// BF16 values apart, from this lane's offset on.
+__device__ __forceinline__ void load_frags(v8bf wb[16], const uint16_t* p, int stride) {
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        const int k = lane * 4 + q;
-        const float h = gelu_f(z3[i * MLP_H + k]);
+    for (int ks = 0; ks < 16; ++ks) wb[ks] = ld8(p + ks * stride);
+}
+
+// acc = A W^T for the tile in LDS and the wave's weight fragments
+__device__ __forceinline__ v16f tile_product(const uint16_t* act, const v8bf wb[16], int li, int lh) {
+    v16f acc;
 #pragma unroll
-        for (int o = 0; o < SIRIUS_MLP_OUT; ++o) part[o] = fmaf(h, W4[o * MLP_H + k], part[o]);
+    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+#pragma unroll
+    for (int ks = 0; ks < 16; ++ks) {
+        const v8bf a = ld8(act + li * TR_PITCH + 16 * ks + 8 * lh);
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, wb[ks], acc, 0, 0, 0);
+    }
+    return acc;
+}
+
+// The wave's 16 values of its neuron column, rounded to BF16: into the LDS tile (row = sample) and
+// to memory as the two operand fragments of the weight gradient.
+__device__ __forceinline__ void put_tile(const float v[16], uint16_t* act, uint16_t* frag, int j, int lh) {
+    __bf16 b[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        b[r] = (__bf16)v[r];
+        __builtin_memcpy(act + (8 * (r >> 2) + 4 * lh + (r & 3)) * TR_PITCH + j, &b[r], 2);
     }
 #pragma unroll
-    for (int o = 0; o < SIRIUS_MLP_OUT; ++o)
-        for (int off = 32; off > 0; off >>= 1) part[o] += __shfl_xor(part[o], off);
-    if (lane < MLP_N4) {
-        float v = 0.f;
+    for (int s = 0; s < 2; ++s) {
+        v8bf f;
 #pragma unroll
-        for (int o = 0; o < SIRIUS_MLP_OUT; ++o) v = lane == o ? part[o] + b4[o] : v;
-        y64[i * MLP_N4 + lane] = v;
+        for (int e = 0; e < 8; ++e) f[e] = b[8 * s + e];
+        *(v8bf*)(frag + s * 64 * 8) = f;
     }
 }
 
-// gz3[i][k] = (sum_o gy[i][o] W4[o][k]) gelu'(z3[i][k]), in FP32 and BF16.
-__global__ void k_head_bwd(const float* __restrict__ gy64, const float* __restrict__ W4, const float* __restrict__ z3,
-                           int64_t n_pad, float* __restrict__ gzf, uint16_t* __restrict__ gzb) {
-    const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= n_pad * MLP_H) return;
-    const int64_t i = e / MLP_H;
-    const int k = (int)(e % MLP_H);
-    float dh = 0.f;
-#pragma unroll
-    for (int o = 0; o < SIRIUS_MLP_OUT; ++o) dh = fmaf(gy64[i * MLP_N4 + o], W4[o * MLP_H + k], dh);
-    const float g = dh * gelu_df(z3[e]);
-    gzf[e] = g;
-    gzb[e] = f2bf(g);
+// z -> gelu'(z) in place for this thread's 16 values (one of a layer's rows of TR_THREADS values each)
+__device__ __forceinline__ void derive(float* zs) {
+#pragma unroll 1
+    for (int r = 0; r < 16; r += 2) {
+        const float z0 = zs[r * TR_THREADS], z1 = zs[(r + 1) * TR_THREADS];
+        const float d0 = gelu_df(z0), d1 = gelu_df(z1);
+        zs[r * TR_THREADS] = d0;
+        zs[(r + 1) * TR_THREADS] = d1;
+    }
 }
 
-// dW4[o][k] = sum_i gy[i][o] gelu(z3[i][k]): row chunks into part[split][6][256], then a fixed-
-// order sum over the chunks (deterministic).
-__global__ __launch_bounds__(256) void k_head_wgrad_part(const float* __restrict__ gy64, const float* __restrict__ z3,
-                                                         int64_t n_pad, int64_t chunk, float* __restrict__ part) {
-    const int k = threadIdx.x;
-    const int64_t r0 = (int64_t)blockIdx.x * chunk, r1 = min(n_pad, r0 + chunk);
-    float acc[SIRIUS_MLP_OUT] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    for (int64_t i = r0; i < r1; ++i) {
-        const float h = gelu_f(z3[i * MLP_H + k]);
+__global__ __launch_bounds__(TR_THREADS) void k_mlp_train(MlpTrainArgs a) {
+    // the activations' two tiles; between the forward and the backward pass the last hidden
+    // activation in FP32
+    __shared__ __attribute__((aligned(16))) uint16_t act[2][TR_ROWS * TR_PITCH];
+    // pre-activations, then GELU derivatives of layers 0..2: [r][thread]. The last layer's pass through
+    // the tiles' space and stay in registers.
+    __shared__ float zs[3][16 * TR_THREADS];
+    __shared__ float xs[TR_ROWS][8];          // the BF16 inputs, for the first layer's weight gradient
+    __shared__ float ys[TR_ROWS][8];          // outputs
+    __shared__ float gys[TR_ROWS][8];         // output gradients
+    float* h4s = (float*)&act[0][0];
+    static_assert(sizeof(act) >= 16 * TR_THREADS * sizeof(float), "room for the last layer's pre-activations");
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    const int li = lane & 31, lh = lane >> 5;
+    const int j = 32 * w + li;  // this lane's neuron
+    const int64_t T = blockIdx.x, row0 = T * TR_ROWS;
+    // this lane's place in the packed weights (neuron block w, and column block w of a transpose) and
+    // in a layer's fragments
+    const int off_f = (w >> 1) * 16384 + (w & 1) * 512 + lane * 8, off_t = w * 8192 + lane * 8;
+    const int64_t off_g = ((T * 8 + w) * 2 * 64 + lane) * 8;
+    {
+        const int r = t >> 4, k = t & 15;
+        const int64_t i = row0 + r;
+        const uint16_t v = (k < SIRIUS_MLP_IN && i < a.n) ? f2bf(a.x[i * SIRIUS_MLP_IN + k]) : (uint16_t)0;
+        act[0][r * TR_PITCH + k] = v;
+        if (k < 8) xs[r][k] = __uint_as_float((uint32_t)v << 16);
+    }
+    const v8bf w0 = ld8(a.w0 + j * 16 + 8 * lh);
+    v8bf wb[16];
+    load_frags(wb, a.wf + off_f, 1024);
+    float h[16];
+    __syncthreads();
+    // ---- forward: hidden layers ----
+    v16f acc;
+    float d3[16];  // the last layer's GELU derivatives
 #pragma unroll
-        for (int o = 0; o < SIRIUS_MLP_OUT; ++o) acc[o] = fmaf(gy64[i * MLP_N4 + o], h, acc[o]);
+    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ld8(&act[0][li * TR_PITCH + 8 * lh]), w0, acc, 0, 0, 0);
+#pragma unroll 1
+    for (int l = 0;; ++l) {
+        const float bias = a.b[l][j];
+        float* z = (l < 3 ? zs[l] : h4s) + t;
+        if (l == 3) __syncthreads();  // every wave has read the last layer's input
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const float v = acc[r] + bias;
+            z[r * TR_THREADS] = v;
+            h[r] = gelu_f(v);
+        }
+        if (l < 3) put_tile(h, act[(l + 1) & 1], a.hf + l * a.frag + off_g, j, lh);
+        derive(z);
+        if (l == 3) break;
+        __syncthreads();
+        acc = tile_product(act[(l + 1) & 1], wb, li, lh);
+        load_frags(wb, l < 2 ? a.wf + (l + 1) * MLP_H * MLP_H + off_f : a.wt + 2 * MLP_H * MLP_H + off_t,
+                   l < 2 ? 1024 : 512);
     }
 #pragma unroll
-    for (int o = 0; o < SIRIUS_MLP_OUT; ++o) part[((int64_t)blockIdx.x * SIRIUS_MLP_OUT + o) * MLP_H + k] = acc[o];
+    for (int r = 0; r < 16; ++r) d3[r] = h4s[r * TR_THREADS + t];
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < 16; ++r) h4s[(8 * (r >> 2) + 4 * lh + (r & 3)) * TR_H4_PITCH + j] = h[r];
+    __syncthreads();
+    // ---- output head: wave w sums samples 4 w .. 4 w + 3, lane l neurons 4 l .. 4 l + 3 ----
+    {
+        float4 wv[SIRIUS_MLP_OUT];
+#pragma unroll
+        for (int o = 0; o < SIRIUS_MLP_OUT; ++o) wv[o] = *(const float4*)(a.W4 + o * MLP_H + 4 * lane);
+        const float b4 = lane < SIRIUS_MLP_OUT ? a.b4[lane] : 0.f;
+#pragma unroll 1
+        for (int s = 4 * w; s < 4 * w + 4; ++s) {
+            const float4 hv = *(const float4*)&h4s[s * TR_H4_PITCH + 4 * lane];
+            float p[SIRIUS_MLP_OUT];
+#pragma unroll
+            for (int o = 0; o < SIRIUS_MLP_OUT; ++o)
+                p[o] = fmaf(hv.w, wv[o].w, fmaf(hv.z, wv[o].z, fmaf(hv.y, wv[o].y, fmaf(hv.x, wv[o].x, 0.f))));
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1)
+#pragma unroll
+                for (int o = 0; o < SIRIUS_MLP_OUT; ++o) p[o] += __shfl_xor(p[o], off);
+            float v = 0.f;
+#pragma unroll
+            for (int o = 0; o < SIRIUS_MLP_OUT; ++o) v = lane == o ? p[o] + b4 : v;
+            if (lane < SIRIUS_MLP_OUT) ys[s][lane] = v;
+        }
+    }
+    __syncthreads();
+    // ---- loss and output gradient (1/n of the batch mean included); rows past n are zero ----
+    float loss = 0.f;
+    if (t < TR_ROWS) {
+        const int64_t i = row0 + t;
+        float g[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        if (i < a.n) {
+            const float* y = ys[t];
+            int c = a.cls[i];
+            c = c < 0 ? 0 : (c > 2 ? 2 : c);
+            float m = fmaxf(y[0], fmaxf(y[1], y[2]));
+            float e0 = expf(y[0] - m), e1 = expf(y[1] - m), e2 = expf(y[2] - m);
+            float s = e0 + e1 + e2;
+            float yc = c == 0 ? y[0] : (c == 1 ? y[1] : y[2]);
+            loss = -(yc - m - logf(s));
+            const float inv_n = 1.f / (float)a.n;
+            g[0] = (e0 / s - (c == 0)) * inv_n;
+            g[1] = (e1 / s - (c == 1)) * inv_n;
+            g[2] = (e2 / s - (c == 2)) * inv_n;
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                float d = c == 0 ? y[3 + k] - a.dir[i * 3 + k] : 0.f;
+                loss += (float)SIRIUS_MLP_DIR_WEIGHT * d * d;
+                g[3 + k] = 2.f * (float)SIRIUS_MLP_DIR_WEIGHT * d * inv_n;
+            }
+        }
+#pragma unroll
+        for (int o = 0; o < 6; ++o) gys[t][o] = g[o];
+    }
+    __syncthreads();
+    // the tile's row of partials; the two half-waves hold the same neurons for other samples
+    float* row = a.part + T * MLP_TILE_COLS;
+    auto put = [&](int col, float v) {
+        v += __shfl_xor(v, 32);
+        if (lh == 0) row[col + j] = v;
+    };
+    // ---- backward: head ----
+    float g[16], db = 0.f;
+    {
+        float w4[SIRIUS_MLP_OUT], dw4[SIRIUS_MLP_OUT];
+#pragma unroll
+        for (int o = 0; o < SIRIUS_MLP_OUT; ++o) {
+            w4[o] = a.W4[o * MLP_H + j];
+            dw4[o] = 0.f;
+        }
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const float* gy = gys[8 * (r >> 2) + 4 * lh + (r & 3)];
+            float dh = 0.f;
+#pragma unroll
+            for (int o = 0; o < SIRIUS_MLP_OUT; ++o) {
+                dh = fmaf(gy[o], w4[o], dh);
+                dw4[o] = fmaf(gy[o], h[r], dw4[o]);
+            }
+            g[r] = dh * d3[r];
+            db += g[r];
+        }
+#pragma unroll
+        for (int o = 0; o < SIRIUS_MLP_OUT; ++o) put(MLP_COL_DW4 + o * MLP_H, dw4[o]);
+        put(MLP_COL_DB + 3 * MLP_H, db);
+    }
+    if (w == 0) {
+        for (int off = 16; off > 0; off >>= 1) loss += __shfl_xor(loss, off);
+        if (lane == 0) row[MLP_COL_LOSS] = loss;
+        if (lane < SIRIUS_MLP_OUT) {
+            float db4 = 0.f;
+            for (int i = 0; i < TR_ROWS; ++i) db4 += gys[i][lane];
+            row[MLP_COL_DB4 + lane] = db4;
+        }
+    }
+    // ---- backward: hidden layers ----
+#pragma unroll 1
+    for (int l = 3;; --l) {
+        // gz_l is in g: the next product's A tile (h4s was read before the last barrier) and a
+        // weight-gradient operand
+        put_tile(g, act[l & 1], a.gf + (l - 1) * a.frag + off_g, j, lh);
+        __syncthreads();
+        acc = tile_product(act[l & 1], wb, li, lh);
+        if (l > 1) load_frags(wb, a.wt + (l - 2) * MLP_H * MLP_H + off_t, 512);
+        db = 0.f;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            g[r] = acc[r] * zs[l - 1][r * TR_THREADS + t];
+            db += g[r];
+        }
+        put(MLP_COL_DB + (l - 1) * MLP_H, db);
+        if (l == 1) break;
+    }
+    // first layer's weights: the BF16 gradient times the BF16 inputs, summed in FP32
+    float dw0[SIRIUS_MLP_IN] = {0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const float gb = (float)(__bf16)g[r];
+        const float* x = xs[8 * (r >> 2) + 4 * lh + (r & 3)];
+#pragma unroll
+        for (int k = 0; k < SIRIUS_MLP_IN; ++k) dw0[k] = fmaf(gb, x[k], dw0[k]);
+    }
+#pragma unroll
+    for (int k = 0; k < SIRIUS_MLP_IN; ++k) put(MLP_COL_DW0 + k * MLP_H, dw0[k]);
 }
-__global__ void k_head_wgrad_final(const float* __restrict__ part, int nsplit, float* __restrict__ dW4) {
-    const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= SIRIUS_MLP_OUT * MLP_H) return;
+
+// dW_l = gz_l^T h_l for the hidden layers l = 1..3 (blockIdx.z = l - 1), 128 x 128 outputs per block
+// (blockIdx.y), the 32-sample tiles of split blockIdx.x: four waves of 64 x 64. Both operands are
+// read as the fragments k_mlp_train wrote, each a contiguous kilobyte per wave, two tiles ahead of
+// the products.
+__global__ __launch_bounds__(256) void k_mlp_wgrad(MlpWgradArgs a) {
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int l = blockIdx.z;
+    const int jb = (blockIdx.y >> 1) * 4 + (w >> 1) * 2, kb = (blockIdx.y & 1) * 4 + (w & 1) * 2;
+    const int64_t t0 = (int64_t)blockIdx.x * a.chunk, t1 = min(a.tiles, t0 + a.chunk);
+    const uint16_t* A = a.gf + l * a.frag + (int64_t)jb * 2 * 512 + lane * 8;
+    const uint16_t* B = a.hf + l * a.frag + (int64_t)kb * 2 * 512 + lane * 8;
+    v16f acc[2][2];
+#pragma unroll
+    for (int m = 0; m < 2; ++m)
+#pragma unroll
+        for (int n = 0; n < 2; ++n)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[m][n][r] = 0.f;
+    constexpr int AHEAD = 2;
+    v8bf fa[AHEAD][2][2], fb[AHEAD][2][2];  // [tile][block][half tile of 16 samples]
+    auto load = [&](int64_t T, v8bf (&xa)[2][2], v8bf (&xb)[2][2]) {
+        const int64_t at = T * (8 * 2 * 512);
+#pragma unroll
+        for (int m = 0; m < 2; ++m)
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                xa[m][s] = ld8(A + at + (m * 2 + s) * 512);
+                xb[m][s] = ld8(B + at + (m * 2 + s) * 512);
+            }
+    };
+#pragma unroll
+    for (int q = 0; q < AHEAD; ++q)
+        if (t0 + q < t1) load(t0 + q, fa[q], fb[q]);
+    for (int64_t T = t0; T < t1; T += AHEAD) {
+#pragma unroll
+        for (int q = 0; q < AHEAD; ++q) {
+            if (T + q < t1) {
+#pragma unroll
+                for (int s = 0; s < 2; ++s)
+#pragma unroll
+                    for (int m = 0; m < 2; ++m)
+#pragma unroll
+                        for (int n = 0; n < 2; ++n)
+                            acc[m][n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[q][m][s], fb[q][n][s], acc[m][n], 0, 0, 0);
+                if (T + q + AHEAD < t1) load(T + q + AHEAD, fa[q], fb[q]);
+            }
+        }
+    }
+    float* out = a.part + ((int64_t)blockIdx.x * 3 + l) * MLP_H * MLP_H;
+#pragma unroll
+    for (int m = 0; m < 2; ++m)
+#pragma unroll
+        for (int n = 0; n < 2; ++n)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int row = (jb + m) * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+                out[(int64_t)row * MLP_H + (kb + n) * 32 + (lane & 31)] = acc[m][n][r];
+            }
+}
+
+// The gradient in the public layout: blocks 0 .. GS_W - 1 add the splits of the hidden layers'
+// weights (four values per lane), the others the rows of per-tile partials (64 columns each, 16
+// groups of rows, then the groups in order). The loss's column goes to *loss.
+constexpr int GS_THREADS = 1024;
+constexpr int GS_W = 3 * MLP_H * MLP_H / 4 / GS_THREADS;
+static_assert(3 * MLP_H * MLP_H % (4 * GS_THREADS) == 0 && MLP_TILE_COLS % 64 == 0, "whole blocks");
+__global__ __launch_bounds__(GS_THREADS) void k_mlp_grad_sum(MlpGradSumArgs a) {
+    __shared__ float red[16][64];
+    const int t = threadIdx.x;
+    if (blockIdx.x < GS_W) {
+        const int e = (blockIdx.x * GS_THREADS + t) * 4;
+        float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+        for (int q = 0; q < a.splits; ++q) {
+            const float4 v = *(const float4*)(a.wpart + (int64_t)q * 3 * MLP_H * MLP_H + e);
+            s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w;
+        }
+        float* d = a.grad + a.off_w[1 + e / (MLP_H * MLP_H)] + e % (MLP_H * MLP_H);
+        d[0] = s.x; d[1] = s.y; d[2] = s.z; d[3] = s.w;  // the caller's array may not be 16-byte aligned
+        return;
+    }
+    const int c = (blockIdx.x - GS_W) * 64 + (t & 63), q = t >> 6;
     float s = 0.f;
-    for (int q = 0; q < nsplit; ++q) s += part[(int64_t)q * SIRIUS_MLP_OUT * MLP_H + e];
-    dW4[e] = s;
+    for (int r = q; r < a.rows; r += 16) s += a.part[(int64_t)r * MLP_TILE_COLS + c];
+    red[q][t & 63] = s;
+    __syncthreads();
+    if (q) return;
+    s = red[0][t];
+#pragma unroll
+    for (int k = 1; k < 16; ++k) s += red[k][t];
+    if (c < MLP_COL_DW4) a.grad[a.off_b[c / MLP_H] + c % MLP_H] = s;
+    else if (c < MLP_COL_DB4) a.grad[a.off_w[4] + c - MLP_COL_DW4] = s;
+    else if (c < MLP_COL_LOSS) a.grad[a.off_b[4] + c - MLP_COL_DB4] = s;
+    else if (c == MLP_COL_LOSS) *a.loss = s;
+    else if (c >= MLP_COL_DW0 && c < MLP_COL_DW0 + SIRIUS_MLP_IN * MLP_H) {
+        const int k = (c - MLP_COL_DW0) / MLP_H, o = (c - MLP_COL_DW0) % MLP_H;
+        a.grad[a.off_w[0] + o * SIRIUS_MLP_IN + k] = s;
+    }
 }
 
-hipError_t launch_head_fwd(const float* z3, const float* W4, const float* b4, int64_t n_pad, float* y64,
-                           hipStream_t st) {
-    hipLaunchKernelGGL(k_head_fwd, dim3((unsigned)((n_pad + 3) / 4)), dim3(256), 0, st, z3, W4, b4, n_pad, y64);
+hipError_t launch_mlp_train(const MlpTrainArgs& a, hipStream_t st) {
+    hipLaunchKernelGGL(k_mlp_train, dim3((unsigned)((a.n + TR_ROWS - 1) / TR_ROWS)), dim3(TR_THREADS), 0, st, a);
     return hipGetLastError();
 }
-hipError_t launch_head_bwd(const float* gy64, const float* W4, const float* z3, int64_t n_pad, float* gzf,
-                           uint16_t* gzb, hipStream_t st) {
-    const int64_t e = n_pad * MLP_H;
-    hipLaunchKernelGGL(k_head_bwd, dim3((unsigned)((e + 255) / 256)), dim3(256), 0, st, gy64, W4, z3, n_pad, gzf, gzb);
+hipError_t launch_mlp_wgrad(const MlpWgradArgs& a, int splits, hipStream_t st) {
+    hipLaunchKernelGGL(k_mlp_wgrad, dim3((unsigned)splits, 4, 3), dim3(256), 0, st, a);
     return hipGetLastError();
 }
-hipError_t launch_head_wgrad(const float* gy64, const float* z3, int64_t n_pad, float* part, int nsplit, float* dW4,
-                             hipStream_t st) {
-    const int64_t chunk = (n_pad + nsplit - 1) / nsplit;
-    hipLaunchKernelGGL(k_head_wgrad_part, dim3((unsigned)nsplit), dim3(MLP_H), 0, st, gy64, z3, n_pad, chunk, part);
-    hipLaunchKernelGGL(k_head_wgrad_final, dim3((SIRIUS_MLP_OUT * MLP_H + 255) / 256), dim3(256), 0, st, part, nsplit,
-                       dW4);
+hipError_t launch_mlp_grad_sum(const MlpGradSumArgs& a, hipStream_t st) {
+    hipLaunchKernelGGL(k_mlp_grad_sum, dim3(GS_W + MLP_TILE_COLS / 64), dim3(GS_THREADS), 0, st, a);
     return hipGetLastError();
 }
 
-// Operands of the fused kernel from the FP32 masters: W0 padded to 16 input columns, W1..W3 as
-// they are, the head's weights split into BF16 high and low parts (rows 6..31 zero).
-// Fused-inference operands from the FP32 masters: W0 [256][16] (input columns padded), and the
+// Operands of the inference and training kernels from the FP32 masters: W0 [256][16] (input columns padded), and the
 // hidden layers' and the head's weights in MFMA fragment order: the 16-byte A operand of lane l
 // for k-step ks, row tile mt of wave w sits at (((w 16 + ks) 2 + mt) 64 + l) 8 (hidden layer:
 // row 64 w + 32 mt + l % 32, columns 16 ks + 8 (l / 32) .. +7), so each wave's weight load is one
-// contiguous kilobyte; the head's high and low BF16 parts row-major [32][256] (rows 6..31 zero).
+// contiguous kilobyte; their transposes for the backward pass, the fragment of lane l for k-step ks,
+// column block w at ((w 16 + ks) 64 + l) 8 (W[16 ks + 8 (l / 32) .. +7][32 w + l % 32]); the head's
+// high and low BF16 parts row-major [32][256] (rows 6..31 zero).
 __global__ void k_pack_fused(const float* __restrict__ P, uint16_t* __restrict__ w0, uint16_t* __restrict__ wh,
-                             uint16_t* __restrict__ w4h, uint16_t* __restrict__ w4l, size_t off_w0, size_t off_w1,
+                             uint16_t* __restrict__ wt, uint16_t* __restrict__ w4h, uint16_t* __restrict__ w4l, size_t off_w0, size_t off_w1,
                              size_t off_w2, size_t off_w3, size_t off_w4) {
     const int e = blockIdx.x * blockDim.x + threadIdx.x;
     if (e < MLP_H * 16) {
@@ -417,6 +625,8 @@ __global__ void k_pack_fused(const float* __restrict__ P, uint16_t* __restrict__
         const int j = 64 * w + 32 * mt + (lane & 31), k = 16 * ks + 8 * (lane >> 5) + i;
         const size_t off = l == 0 ? off_w1 : (l == 1 ? off_w2 : off_w3);
         wh[e] = f2bf(P[off + (size_t)j * MLP_H + k]);
+        const int tj = 16 * ((r >> 9) & 15) + 8 * (lane >> 5) + i, tk = 32 * (r >> 13) + (lane & 31);
+        wt[e] = f2bf(P[off + (size_t)tj * MLP_H + tk]);
     }
     if (e < 32 * MLP_H) {
         const int j = e / MLP_H, k = e % MLP_H;
@@ -426,136 +636,10 @@ __global__ void k_pack_fused(const float* __restrict__ P, uint16_t* __restrict__
         w4l[e] = f2bf(w - __uint_as_float((uint32_t)hi << 16));
     }
 }
-hipError_t launch_pack_fused(const float* params, uint16_t* w0, uint16_t* wh, uint16_t* w4h, uint16_t* w4l,
+hipError_t launch_pack_fused(const float* params, uint16_t* w0, uint16_t* wh, uint16_t* wt, uint16_t* w4h, uint16_t* w4l,
                              const size_t off_w[5], hipStream_t st) {
-    hipLaunchKernelGGL(k_pack_fused, dim3((3 * MLP_H * MLP_H + 255) / 256), dim3(256), 0, st, params, w0, wh, w4h, w4l,
+    hipLaunchKernelGGL(k_pack_fused, dim3((3 * MLP_H * MLP_H + 255) / 256), dim3(256), 0, st, params, w0, wh, wt, w4h, w4l,
                        off_w[0], off_w[1], off_w[2], off_w[3], off_w[4]);
-    return hipGetLastError();
-}
-
-// Input rows: h0[i][0..4] = bf16(x[i][0..4]), the rest of the padded 64-wide row zero; rows
-// n .. n_pad - 1 are zero.
-__global__ void k_mlp_input(const float* __restrict__ x, int64_t n, int64_t n_pad, uint16_t* __restrict__ h0) {
-    int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= n_pad * MLP_X0) return;
-    int64_t i = e / MLP_X0;
-    int k = (int)(e % MLP_X0);
-    h0[e] = (i < n && k < SIRIUS_MLP_IN) ? f2bf(x[i * SIRIUS_MLP_IN + k]) : (uint16_t)0;
-}
-
-__global__ void k_mlp_extract(const float* __restrict__ y64, int64_t n, float* __restrict__ y) {
-    int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= n * SIRIUS_MLP_OUT) return;
-    int64_t i = e / SIRIUS_MLP_OUT;
-    y[e] = y64[i * MLP_N4 + (e % SIRIUS_MLP_OUT)];
-}
-
-// Per-sample loss and the output gradient (1/n of the batch mean included), padded to 64
-// columns; rows past n are zero.
-__global__ void k_mlp_loss(const float* __restrict__ y64, const int32_t* __restrict__ cls,
-                           const float* __restrict__ dir, int64_t n, int64_t n_pad, float* __restrict__ gyf,
-                           uint16_t* __restrict__ gyb, float* __restrict__ loss_i) {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n_pad) return;
-    float g[MLP_N4];
-#pragma unroll
-    for (int o = 0; o < MLP_N4; ++o) g[o] = 0.f;
-    float loss = 0.f;
-    if (i < n) {
-        const float* y = y64 + i * MLP_N4;
-        int c = cls[i];
-        c = c < 0 ? 0 : (c > 2 ? 2 : c);
-        float m = fmaxf(y[0], fmaxf(y[1], y[2]));
-        float e0 = expf(y[0] - m), e1 = expf(y[1] - m), e2 = expf(y[2] - m);
-        float s = e0 + e1 + e2;
-        float yc = c == 0 ? y[0] : (c == 1 ? y[1] : y[2]);
-        loss = -(yc - m - logf(s));
-        const float inv_n = 1.f / (float)n;
-        g[0] = (e0 / s - (c == 0)) * inv_n;
-        g[1] = (e1 / s - (c == 1)) * inv_n;
-        g[2] = (e2 / s - (c == 2)) * inv_n;
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            float d = c == 0 ? y[3 + k] - dir[i * 3 + k] : 0.f;
-            loss += (float)SIRIUS_MLP_DIR_WEIGHT * d * d;
-            g[3 + k] = 2.f * (float)SIRIUS_MLP_DIR_WEIGHT * d * inv_n;
-        }
-    }
-#pragma unroll
-    for (int o = 0; o < MLP_N4; ++o) {
-        gyf[i * MLP_N4 + o] = g[o];
-        gyb[i * MLP_N4 + o] = f2bf(g[o]);
-    }
-    loss_i[i] = loss;
-}
-
-// Column sums of src[rows][ld] over the first `cols` columns: nsplit row chunks into
-// part[nsplit][cols], then dst[c] = sum of the chunks (fixed order: deterministic).
-__global__ __launch_bounds__(256) void k_colsum_part(const float* __restrict__ src, int64_t rows, int cols, int ld,
-                                                     int64_t chunk, float* __restrict__ part) {
-    __shared__ float red[4][64];
-    const int c = blockIdx.x * 64 + (threadIdx.x & 63), q = threadIdx.x >> 6;
-    const int64_t r0 = (int64_t)blockIdx.y * chunk, r1 = min(rows, r0 + chunk);
-    float s = 0.f;
-    if (c < cols)
-        for (int64_t r = r0 + q; r < r1; r += 4) s += src[r * ld + c];
-    red[q][threadIdx.x & 63] = s;
-    __syncthreads();
-    if (q == 0 && c < cols)
-        part[(int64_t)blockIdx.y * cols + c] = red[0][threadIdx.x] + red[1][threadIdx.x] + red[2][threadIdx.x] +
-                                               red[3][threadIdx.x];
-}
-__global__ void k_colsum_final(const float* __restrict__ part, int nsplit, int cols, float* __restrict__ dst) {
-    int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= cols) return;
-    float s = 0.f;
-    for (int k = 0; k < nsplit; ++k) s += part[(int64_t)k * cols + c];
-    dst[c] = s;
-}
-
-hipError_t launch_colsum(const float* src, int64_t rows, int cols, int ld, float* part, int nsplit, float* dst,
-                         hipStream_t st) {
-    int64_t chunk = (rows + nsplit - 1) / nsplit;
-    hipLaunchKernelGGL(k_colsum_part, dim3((unsigned)((cols + 63) / 64), (unsigned)nsplit), dim3(256), 0, st, src,
-                       rows, cols, ld, chunk, part);
-    hipLaunchKernelGGL(k_colsum_final, dim3((unsigned)((cols + 255) / 256)), dim3(256), 0, st, part, nsplit, cols,
-                       dst);
-    return hipGetLastError();
-}
-
-// dst[r][c] (rows x cols, row-major) = sum over splits of part[s][r][c] (part is M x N).
-__global__ void k_reduce_partials(const float* __restrict__ part, int nsplit, int M, int N, int rows, int cols,
-                                  float* __restrict__ dst) {
-    int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= rows * cols) return;
-    int r = e / cols, c = e % cols;
-    float s = 0.f;
-    for (int k = 0; k < nsplit; ++k) s += part[(int64_t)k * M * N + (int64_t)r * N + c];
-    dst[e] = s;
-}
-hipError_t launch_reduce_partials(const float* part, int nsplit, int M, int N, int rows, int cols, float* dst,
-                                  hipStream_t st) {
-    hipLaunchKernelGGL(k_reduce_partials, dim3((unsigned)((rows * cols + 255) / 256)), dim3(256), 0, st, part, nsplit,
-                       M, N, rows, cols, dst);
-    return hipGetLastError();
-}
-
-// Sum of n floats: 256 block partials, then one block (deterministic order).
-__global__ __launch_bounds__(256) void k_sum_part(const float* __restrict__ src, int64_t n, float* __restrict__ part) {
-    __shared__ float red[256];
-    float s = 0.f;
-    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) s += src[i];
-    red[threadIdx.x] = s;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) part[blockIdx.x] = red[0];
-}
-hipError_t launch_sum(const float* src, int64_t n, float* part, float* dst, hipStream_t st) {
-    hipLaunchKernelGGL(k_sum_part, dim3(256), dim3(256), 0, st, src, n, part);
-    hipLaunchKernelGGL(k_sum_part, dim3(1), dim3(256), 0, st, part, (int64_t)256, dst);
     return hipGetLastError();
 }
 
@@ -574,42 +658,6 @@ __global__ void k_adam(float* __restrict__ p, const float* __restrict__ g, float
 hipError_t launch_adam(float* params, const float* grad, float* m, float* v, int64_t P, float lr, float c1, float c2,
                        hipStream_t st) {
     hipLaunchKernelGGL(k_adam, dim3((unsigned)((P + 255) / 256)), dim3(256), 0, st, params, grad, m, v, P, lr, c1, c2);
-    return hipGetLastError();
-}
-
-// Padded BF16 weights and padded biases of one layer from the FP32 masters.
-__global__ void k_pack_layer(const float* __restrict__ W, const float* __restrict__ b, int out, int in, int NP, int KP,
-                             uint16_t* __restrict__ w, float* __restrict__ bp) {
-    int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= NP * KP) return;
-    int j = e / KP, k = e % KP;
-    w[e] = (j < out && k < in) ? f2bf(W[j * in + k]) : (uint16_t)0;
-    if (k == 0) bp[j] = j < out ? b[j] : 0.f;
-}
-hipError_t launch_pack(const float* params, uint16_t* const* w, float* const* b, hipStream_t st) {
-    for (int l = 0; l < MLP_NL; ++l) {
-        int n = MLP_NP[l] * MLP_KP[l];
-        hipLaunchKernelGGL(k_pack_layer, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st,
-                           params + mlp_param_offset_w(l), params + mlp_param_offset_b(l), MLP_OUTD[l], MLP_IN[l],
-                           MLP_NP[l], MLP_KP[l], w[l], b[l]);
-    }
-    return hipGetLastError();
-}
-
-hipError_t launch_mlp_input(const float* x, int64_t n, int64_t n_pad, uint16_t* h0, hipStream_t st) {
-    int64_t e = n_pad * MLP_X0;
-    hipLaunchKernelGGL(k_mlp_input, dim3((unsigned)((e + 255) / 256)), dim3(256), 0, st, x, n, n_pad, h0);
-    return hipGetLastError();
-}
-hipError_t launch_mlp_extract(const float* y64, int64_t n, float* y, hipStream_t st) {
-    int64_t e = n * SIRIUS_MLP_OUT;
-    hipLaunchKernelGGL(k_mlp_extract, dim3((unsigned)((e + 255) / 256)), dim3(256), 0, st, y64, n, y);
-    return hipGetLastError();
-}
-hipError_t launch_mlp_loss(const float* y64, const int32_t* cls, const float* dir, int64_t n, int64_t n_pad,
-                           float* gyf, uint16_t* gyb, float* loss_i, hipStream_t st) {
-    hipLaunchKernelGGL(k_mlp_loss, dim3((unsigned)((n_pad + 255) / 256)), dim3(256), 0, st, y64, cls, dir, n, n_pad,
-                       gyf, gyb, loss_i);
     return hipGetLastError();
 }
 

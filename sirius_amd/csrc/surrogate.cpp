@@ -26,11 +26,8 @@ void mlp_release(Handle& H) {
     MlpState& S = *H.mlp;
     for (void* p : {(void*)S.params, (void*)S.adam_m, (void*)S.adam_v, (void*)S.grad})
         if (p) (void)hipFree(p);
-    for (int l = 0; l < MLP_NL; ++l) {
-        if (S.w[l]) (void)hipFree(S.w[l]);
-        if (S.b[l]) (void)hipFree(S.b[l]);
-    }
-    for (void* p : {(void*)S.fw0, (void*)S.fwh, (void*)S.fw4h, (void*)S.fw4l, (void*)S.cal_err, (void*)S.cal_n,
+    if (S.loss_host) (void)hipHostFree(S.loss_host);
+    for (void* p : {(void*)S.fw0, (void*)S.fwh, (void*)S.fwt, (void*)S.fw4h, (void*)S.fw4l, (void*)S.cal_err, (void*)S.cal_n,
                     (void*)S.cal_bad, (void*)S.cal_dmax})
         if (p) (void)hipFree(p);
     delete H.mlp;
@@ -47,13 +44,10 @@ static int mlp_alloc(Handle& H) {
     hipError_t e;
     for (float** p : {&S.params, &S.adam_m, &S.adam_v, &S.grad})
         if ((e = hipMalloc((void**)p, P * sizeof(float))) != hipSuccess) return H.hip_fail(e, "mlp alloc");
-    for (int l = 0; l < MLP_NL; ++l) {
-        if ((e = hipMalloc((void**)&S.w[l], (size_t)MLP_NP[l] * MLP_KP[l] * 2)) != hipSuccess ||
-            (e = hipMalloc((void**)&S.b[l], (size_t)MLP_NP[l] * 4)) != hipSuccess)
-            return H.hip_fail(e, "mlp alloc");
-    }
     if ((e = hipMalloc((void**)&S.fw0, (size_t)MLP_H * 16 * 2)) != hipSuccess ||
         (e = hipMalloc((void**)&S.fwh, (size_t)3 * MLP_H * MLP_H * 2)) != hipSuccess ||
+        (e = hipMalloc((void**)&S.fwt, (size_t)3 * MLP_H * MLP_H * 2)) != hipSuccess ||
+        (e = hipHostMalloc((void**)&S.loss_host, 64, hipHostMallocDefault)) != hipSuccess ||
         (e = hipMalloc((void**)&S.fw4h, (size_t)32 * MLP_H * 2)) != hipSuccess ||
         (e = hipMalloc((void**)&S.fw4l, (size_t)32 * MLP_H * 2)) != hipSuccess ||
         (e = hipMalloc((void**)&S.cal_err, SUR_BINS * 4)) != hipSuccess ||
@@ -80,11 +74,9 @@ static hipError_t mlp_clear_calibration(MlpState& S, hipStream_t st) {
 
 // BF16 operands of every kernel from the FP32 masters (after each update).
 static hipError_t mlp_pack(MlpState& S, hipStream_t st) {
-    hipError_t e = launch_pack(S.params, S.w, S.b, st);
-    if (e != hipSuccess) return e;
     const size_t off_w[5] = {mlp_param_offset_w(0), mlp_param_offset_w(1), mlp_param_offset_w(2),
                              mlp_param_offset_w(3), mlp_param_offset_w(4)};
-    return launch_pack_fused(S.params, S.fw0, S.fwh, S.fw4h, S.fw4l, off_w, st);
+    return launch_pack_fused(S.params, S.fw0, S.fwh, S.fwt, S.fw4h, S.fw4l, off_w, st);
 }
 
 static int mlp_reset_adam(Handle& H) {
@@ -102,143 +94,59 @@ static int mlp_reset_adam(Handle& H) {
     return SIRIUS_HIP_OK;
 }
 
-static inline int64_t pad64(int64_t n) { return (n + 63) / 64 * 64; }
-
-// Workspace of a training batch of n_pad rows
-struct MlpWork {
-    uint16_t* h[MLP_NL];  // h[0]: [n_pad][64], h[1..4]: [n_pad][256]
-    float* z[MLP_NL - 1];
-    float* y64;
-    float* gyf;
-    uint16_t* gyb;
-    float* gzf[2];
-    uint16_t* gzb[2];
-    float* part;
-    float* colpart;
-    float* loss_i;
-    float* loss_part;
-    float* loss;
-};
-
-constexpr int COLSPLIT = 64;
-
-static int mlp_workspace(Handle& H, int64_t n_pad, bool train, MlpWork& W) {
-    int rc = SIRIUS_HIP_OK;
-    const size_t r = (size_t)n_pad;
-    W.h[0] = (uint16_t*)H.scratch("mlp_h0", r * MLP_X0 * 2, &rc);
-    const char* hn[4] = {"mlp_h1", "mlp_h2", "mlp_h3", "mlp_h4"};
-    const char* zn[4] = {"mlp_z0", "mlp_z1", "mlp_z2", "mlp_z3"};
-    for (int l = 1; l < MLP_NL; ++l)
-        W.h[l] = (uint16_t*)H.scratch(train ? hn[l - 1] : hn[(l - 1) & 1], r * MLP_H * 2, &rc);
-    for (int l = 0; l < MLP_NL - 1; ++l) W.z[l] = train ? (float*)H.scratch(zn[l], r * MLP_H * 4, &rc) : nullptr;
-    W.y64 = (float*)H.scratch("mlp_y64", r * MLP_N4 * 4, &rc);
-    if (train) {
-        W.gyf = (float*)H.scratch("mlp_gyf", r * MLP_N4 * 4, &rc);
-        W.gyb = (uint16_t*)H.scratch("mlp_gyb", r * MLP_N4 * 2, &rc);
-        W.gzf[0] = (float*)H.scratch("mlp_gzf0", r * MLP_H * 4, &rc);
-        W.gzf[1] = (float*)H.scratch("mlp_gzf1", r * MLP_H * 4, &rc);
-        W.gzb[0] = (uint16_t*)H.scratch("mlp_gzb0", r * MLP_H * 2, &rc);
-        W.gzb[1] = (uint16_t*)H.scratch("mlp_gzb1", r * MLP_H * 2, &rc);
-        W.part = (float*)H.scratch("mlp_part", (size_t)64 * MLP_H * MLP_H * 4, &rc);
-        W.colpart = (float*)H.scratch("mlp_colpart", (size_t)COLSPLIT * MLP_H * 4, &rc);
-        W.loss_i = (float*)H.scratch("mlp_loss_i", r * 4, &rc);
-        W.loss_part = (float*)H.scratch("mlp_loss_part", 256 * 4, &rc);
-        W.loss = (float*)H.scratch("mlp_loss", 256, &rc);
-    }
-    return rc;
-}
-
-static GemmArgs gemm(const uint16_t* A, int64_t sai, int64_t sak, const uint16_t* B, int64_t sbk, int64_t sbj, int M,
-                     int N, int K) {
-    GemmArgs g;
-    std::memset(&g, 0, sizeof(g));
-    g.A = A; g.sai = sai; g.sak = sak;
-    g.B = B; g.sbk = sbk; g.sbj = sbj;
-    g.M = M; g.N = N; g.K = K; g.kchunk = K;
-    return g;
-}
-
-// Training forward of n_pad rows already in W.h[0]: the hidden layers on BF16 MFMA (keeping
-// their pre-activations z), the output head in FP32 from z3.
-static hipError_t mlp_forward_rows(MlpState& S, MlpWork& W, int64_t n_pad, hipStream_t st) {
-    hipError_t e;
-    for (int l = 0; l < MLP_NL - 1; ++l) {
-        const int64_t lda = l == 0 ? MLP_X0 : MLP_H;
-        GemmArgs g = gemm(W.h[l], lda, 1, S.w[l], 1, MLP_KP[l], (int)n_pad, MLP_H, MLP_KP[l]);
-        g.bias = S.b[l];
-        g.zout = W.z[l];
-        g.hout = W.h[l + 1];
-        if ((e = launch_gemm(EPI_HIDDEN, g, 1, st)) != hipSuccess) return e;
-    }
-    return launch_head_fwd(W.z[3], S.params + mlp_param_offset_w(4), S.params + mlp_param_offset_b(4), n_pad, W.y64,
-                           st);
-}
-
-// Split of the sample dimension for the weight-gradient GEMMs
-static void split_k(int64_t n_pad, int* nsplit, int* kchunk) {
-    int s = (int)std::min<int64_t>(64, std::max<int64_t>(1, n_pad / 1024));
-    int64_t c = (n_pad + s - 1) / s;
-    c = (c + 31) / 32 * 32;
-    *kchunk = (int)c;
-    *nsplit = (int)((n_pad + c - 1) / c);
-}
-
 // Loss and gradient (into grad, public layout) of a batch; *loss_host gets the mean loss.
 static int mlp_loss_grad_dev(Handle& H, const float* x, const int32_t* cls, const float* dir, int n, float* grad,
                              float* loss_host) {
     MlpState& S = *H.mlp;
-    const int64_t n_pad = pad64(n);
-    MlpWork W;
-    int rc = mlp_workspace(H, n_pad, true, W);
+    const int64_t tiles = ((int64_t)n + MLP_TRAIN_ROWS - 1) / MLP_TRAIN_ROWS;
+    // splits of the weight gradients' sample dimension: 16 tiles (512 samples) each, 12 blocks per
+    // split; 16 splits fill three quarters of the chip in one round, and each adds 0.8 MB of
+    // partials to write and read, so at most 32
+    const int64_t want = std::min<int64_t>(32, std::max<int64_t>(1, tiles / 16));
+    const int64_t chunk = (tiles + want - 1) / want;
+    const int splits = (int)((tiles + chunk - 1) / chunk);
+    const size_t frag = (size_t)tiles * MLP_TRAIN_ROWS * MLP_H;  // BF16 values of one layer's fragments
+    int rc = SIRIUS_HIP_OK;
+    uint16_t* fr = (uint16_t*)H.scratch("mlp_frag", 6 * frag * 2, &rc);
+    float* part = (float*)H.scratch("mlp_part", (size_t)tiles * MLP_TILE_COLS * 4, &rc);
+    float* wpart = (float*)H.scratch("mlp_wpart", (size_t)splits * 3 * MLP_H * MLP_H * 4, &rc);
     if (rc) return rc;
-    hipStream_t st = H.stream;
+    MlpTrainArgs t;
+    t.x = x;
+    t.cls = cls;
+    t.dir = dir;
+    t.n = n;
+    t.w0 = S.fw0;
+    MlpWgradArgs g;
+    t.wf = S.fwh;
+    t.wt = S.fwt;
+    g.hf = t.hf = fr;
+    g.gf = t.gf = fr + 3 * frag;
+    g.frag = t.frag = (int64_t)frag;
+    for (int l = 0; l < 4; ++l) t.b[l] = S.params + mlp_param_offset_b(l);
+    t.W4 = S.params + mlp_param_offset_w(4);
+    t.b4 = S.params + mlp_param_offset_b(4);
+    t.part = part;
+    g.tiles = tiles;
+    g.chunk = chunk;
+    g.part = wpart;
+    MlpGradSumArgs s;
+    s.wpart = wpart;
+    s.part = part;
+    s.splits = splits;
+    s.rows = (int)tiles;
+    for (int l = 0; l < MLP_NL; ++l) {
+        s.off_w[l] = mlp_param_offset_w(l);
+        s.off_b[l] = mlp_param_offset_b(l);
+    }
+    s.grad = grad;
+    s.loss = S.loss_host;
     hipError_t e;
-    if ((e = launch_mlp_input(x, n, n_pad, W.h[0], st)) != hipSuccess) return H.hip_fail(e, "mlp input");
-    if ((e = mlp_forward_rows(S, W, n_pad, st)) != hipSuccess) return H.hip_fail(e, "mlp forward");
-    if ((e = launch_mlp_loss(W.y64, cls, dir, n, n_pad, W.gyf, W.gyb, W.loss_i, st)) != hipSuccess)
-        return H.hip_fail(e, "mlp loss");
-    int nsplit, kchunk;
-    split_k(n_pad, &nsplit, &kchunk);
-    // layer 4 (the FP32 head): dW4 = gy^T gelu(z3), db4 = colsum(gy), gz3 = (gy W4) * gelu'(z3)
-    {
-        const int hsplit = (int)std::min<int64_t>(128, std::max<int64_t>(1, n_pad / 64));
-        if ((e = launch_head_wgrad(W.gyf, W.z[3], n_pad, W.part, hsplit, grad + mlp_param_offset_w(4), st)) !=
-            hipSuccess)
-            return H.hip_fail(e, "dW4");
-        if ((e = launch_colsum(W.gyf, n_pad, SIRIUS_MLP_OUT, MLP_N4, W.colpart, COLSPLIT, grad + mlp_param_offset_b(4),
-                               st)) != hipSuccess)
-            return H.hip_fail(e, "db4");
-        if ((e = launch_head_bwd(W.gyf, S.params + mlp_param_offset_w(4), W.z[3], n_pad, W.gzf[0], W.gzb[0], st)) !=
-            hipSuccess)
-            return H.hip_fail(e, "dX4");
-    }
-    int cur = 0;
-    for (int l = MLP_NL - 2; l >= 0; --l) {
-        const int ncols = l == 0 ? MLP_X0 : MLP_H;  // width of the stored layer input rows
-        GemmArgs g = gemm(W.gzb[cur], 1, MLP_H, W.h[l], ncols, 1, MLP_H, ncols, (int)n_pad);
-        g.kchunk = kchunk;
-        g.out = W.part;
-        if ((e = launch_gemm(EPI_PART, g, nsplit, st)) != hipSuccess) return H.hip_fail(e, "dW");
-        if ((e = launch_reduce_partials(W.part, nsplit, MLP_H, ncols, MLP_H, MLP_IN[l], grad + mlp_param_offset_w(l),
-                                        st)) != hipSuccess)
-            return H.hip_fail(e, "dW reduce");
-        if ((e = launch_colsum(W.gzf[cur], n_pad, MLP_H, MLP_H, W.colpart, COLSPLIT, grad + mlp_param_offset_b(l),
-                               st)) != hipSuccess)
-            return H.hip_fail(e, "db");
-        if (l == 0) break;
-        GemmArgs d = gemm(W.gzb[cur], MLP_H, 1, S.w[l], MLP_H, 1, (int)n_pad, MLP_H, MLP_H);
-        d.zin = W.z[l - 1];
-        d.gzf = W.gzf[cur ^ 1];
-        d.gzb = W.gzb[cur ^ 1];
-        if ((e = launch_gemm(EPI_BWD, d, 1, st)) != hipSuccess) return H.hip_fail(e, "dX");
-        cur ^= 1;
-    }
-    if ((e = launch_sum(W.loss_i, n_pad, W.loss_part, W.loss, st)) != hipSuccess) return H.hip_fail(e, "loss sum");
-    float total = 0.f;
-    if ((e = hipMemcpyAsync(&total, W.loss, 4, hipMemcpyDeviceToHost, st)) != hipSuccess ||
-        (e = hipStreamSynchronize(st)) != hipSuccess)
-        return H.hip_fail(e, "loss copy");
-    if (loss_host) *loss_host = total / (float)n;
+    if ((e = launch_mlp_train(t, H.stream)) != hipSuccess ||
+        (e = launch_mlp_wgrad(g, splits, H.stream)) != hipSuccess ||
+        (e = launch_mlp_grad_sum(s, H.stream)) != hipSuccess || (e = hipStreamSynchronize(H.stream)) != hipSuccess)
+        return H.hip_fail(e, "mlp loss and gradient");
+    if (loss_host) *loss_host = *S.loss_host / (float)n;
     return SIRIUS_HIP_OK;
 }
 
@@ -251,7 +159,7 @@ MlpFusedArgs mlp_fused_args(const MlpState& S, const float* x, float* y, int64_t
     a.x_stride = SIRIUS_MLP_IN;
     a.w0 = S.fw0;
     for (int l = 1; l < 4; ++l) a.w[l - 1] = S.fwh + (size_t)(l - 1) * MLP_H * MLP_H;
-    for (int l = 0; l < 4; ++l) a.b[l] = S.b[l];
+    for (int l = 0; l < 4; ++l) a.b[l] = S.params + mlp_param_offset_b(l);
     a.w4h = S.fw4h;
     a.w4l = S.fw4l;
     a.b4 = S.params + mlp_param_offset_b(4);
