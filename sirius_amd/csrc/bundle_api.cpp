@@ -39,7 +39,7 @@ int bundle_for_launch(Handle& H, Batch& B, int emission, int n_cam, BundleOut& b
     if (!rc) bo.jac = (float*)H.scratch("b_jac", 16 * (size_t)B.n, &rc);
     if (!rc) bo.beam = (float*)H.scratch("b_beam", 12 * (size_t)B.n, &rc);
     if (rc) return rc;
-    hipError_t e = launch_trace_bundle(B.family, emission, B.cams_dev, n_cam, B.tp, params_of(H.bundle), bo, H.stream);
+    hipError_t e = launch_trace_bundle(B.kernels, emission, B.cams_dev, n_cam, B.tp, params_of(H.bundle), bo, H.stream);
     if (e != hipSuccess) return H.hip_fail(e, "bundle trace");
     return SIRIUS_HIP_OK;
 }
@@ -104,7 +104,7 @@ int sirius_hip_trace_bundle(SiriusHipHandle hh, const SiriusHipCamera* cams, int
         if (!rc) bo.beam = (float*)get("b_beam", out->beam, 12 * (size_t)n);
         if (rc) return rc;
         const int emission = opts->emission == SIRIUS_EMISSION_THIN_DISK ? SIRIUS_EMISSION_THIN_DISK : 0;
-        hipError_t e = launch_trace_bundle(B.family, emission, B.cams_dev, n_cam, B.tp, params_of(H->bundle), bo,
+        hipError_t e = launch_trace_bundle(B.kernels, emission, B.cams_dev, n_cam, B.tp, params_of(H->bundle), bo,
                                            H->stream);
         if (e != hipSuccess) return H->hip_fail(e, "bundle trace");
         if (!out->on_device) {

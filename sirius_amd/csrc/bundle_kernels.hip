@@ -99,8 +99,8 @@ SIRIUS_HD __forceinline__ void ellipse_of(const double m[2][2], double size, flo
 // 212-364 bytes per lane (the state, two tangents and their derivatives beside seven stages).
 // A wave's rays that end on the disk are landed together, and the escape angles differenced
 // together, after its last ray has ended. Bound by FP64 issue and by the longest ray's steps: 641x361
-// Kerr rays at the FP32 path's tolerances take 2.15 ms (spill-free at one wave per SIMD; 2.16 at
-// two with 84 bytes spilled), one lane per ray took 4.74 (5.89 with IEEE roots and divisions).
+// Kerr rays at the FP32 path's tolerances take 1.83 ms without Lambda, 2.15 with its terms (spill-free
+// at one wave per SIMD); one lane per ray took 4.74 (5.89 with IEEE roots and divisions).
 template <int FAM, int EMIT>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void k_trace_bundle(
     const CamConst* __restrict__ cams, int n_cam, TraceParams tp, BundleParams bp, BundleOut bo) {
@@ -144,7 +144,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
         ++attempts;
         double e = 0;
         for (int i = 0; i < 4; ++i) {
-            const double q = err[i].v * rcp_t(tp.atol + tp.rtol * fabs(X1[i].v));
+            const double q = err[i].v * rcp_t(fmax(tp.atol, 1e-70) + tp.rtol * fabs(X1[i].v));
             e += q * q;
         }
         e = sqrt(0.25 * e);
@@ -159,7 +159,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
         for (int i = 0; i < 4; ++i) bad |= !sfinite(x1[i]) || !sfinite(P1[i].v);
         if (bad) { cls = SIRIUS_RAY_FAILED; break; }
         // thin disk: first crossing inside [r_in, r_out]
-        if constexpr (FAM == 0 && EMIT == SIRIUS_EMISSION_THIN_DISK) {
+        if constexpr (is_ks(FAM) && EMIT == SIRIUS_EMISSION_THIN_DISK) {
             if (X[3].v * x1[3] < 0) {
                 double x[4], k0[4], k1[4], xc[4];
                 values(X, x);
@@ -175,8 +175,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
                 }
             }
         }
-        const double r1 = event_radius(s, x1);
-        if (FAM == 0 && r1 < c.r_cap) { cls = SIRIUS_RAY_CAPTURED; break; }
+        double r1;
+        if constexpr (FAM == FAM_KS_FLAT) r1 = d1.r.v;
+        else r1 = event_radius(s, x1);
+        if (is_ks(FAM) && r1 < c.r_cap) { cls = SIRIUS_RAY_CAPTURED; break; }
         // accepted: the state, its tangent and the FSAL derivative advance
         for (int i = 0; i < 4; ++i) { X[i] = X1[i]; P[i] = P1[i]; }
         X[0].d[0] = 0.0;
@@ -263,6 +265,10 @@ hipError_t launch_trace_bundle(int family, int emission, const CamConst* cams, i
         hipLaunchKernelGGL((k_trace_bundle<1, 0>), grid, block, 0, st, cams, n_cam, tp, bp, bo);
     else if (family == 2)
         hipLaunchKernelGGL((k_trace_bundle<2, 0>), grid, block, 0, st, cams, n_cam, tp, bp, bo);
+    else if (family == FAM_KS_FLAT && disk)
+        hipLaunchKernelGGL((k_trace_bundle<FAM_KS_FLAT, SIRIUS_EMISSION_THIN_DISK>), grid, block, 0, st, cams, n_cam, tp, bp, bo);
+    else if (family == FAM_KS_FLAT)
+        hipLaunchKernelGGL((k_trace_bundle<FAM_KS_FLAT, 0>), grid, block, 0, st, cams, n_cam, tp, bp, bo);
     else if (disk)
         hipLaunchKernelGGL((k_trace_bundle<0, SIRIUS_EMISSION_THIN_DISK>), grid, block, 0, st, cams, n_cam, tp, bp, bo);
     else

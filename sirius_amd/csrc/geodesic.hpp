@@ -121,18 +121,18 @@ struct DevOut {
 
 // Reciprocal square root, reciprocal and square root of a positive value well inside the range
 // (no zero, infinity or denormal: callers clamp). In FP32 device code the hardware instructions
-// (about 1 ulp); in FP64 device code the hardware estimate (about 24 bits) refined by two Newton
-// steps to the last bit or two; on the host the correctly rounded forms. The IEEE FP64 division
-// and square root carry range scaling and special cases: about 12 and 16 instructions, against 5 for
-// the reciprocal and 8 for the reciprocal square root, which yields the root with 3 more.
+// (about 1 ulp); in FP64 device code the hardware estimate (at least 22 bits) refined by one step of
+// third order (its error is the cube of the estimate's) to the last bit or two; on the host the
+// correctly rounded forms. The IEEE FP64 division and square root carry range scaling and special
+// cases: about 12 and 16 instructions, against 4 for the reciprocal and 6 for the reciprocal
+// square root, which yields the root with one more.
 template <class T> SIRIUS_HD __forceinline__ T rsqrt_t(T x) {
 #ifdef __HIP_DEVICE_COMPILE__
     if constexpr (std::is_same_v<T, float>) return __builtin_amdgcn_rsqf(x);
     if constexpr (std::is_same_v<T, double>) {
-        double y = __builtin_amdgcn_rsq(x);
-        const double hx = 0.5 * x;
-        y = ::fma(y, ::fma(-hx * y, y, 0.5), y);
-        return ::fma(y, ::fma(-hx * y, y, 0.5), y);
+        const double y = __builtin_amdgcn_rsq(x);
+        const double e = ::fma(-x * y, y, 1.0);  // 1 - x y^2: 1/sqrt(x) = y (1 + e / 2 + 3 e^2 / 8 + ..)
+        return ::fma(y * e, ::fma(0.375, e, 0.5), y);
     }
 #endif
     return T(1) / sqrt(x);
@@ -141,26 +141,19 @@ template <class T> SIRIUS_HD __forceinline__ T rcp_t(T x) {
 #ifdef __HIP_DEVICE_COMPILE__
     if constexpr (std::is_same_v<T, float>) return __builtin_amdgcn_rcpf(x);
     if constexpr (std::is_same_v<T, double>) {
-        double y = __builtin_amdgcn_rcp(x);
-        y = ::fma(::fma(-x, y, 1.0), y, y);
-        return ::fma(::fma(-x, y, 1.0), y, y);
+        const double y = __builtin_amdgcn_rcp(x);
+        const double e = ::fma(-x, y, 1.0);  // 1/x = y (1 + e + e^2 + ..)
+        return ::fma(y, ::fma(e, e, e), y);
     }
 #endif
     return T(1) / x;
 }
-// sqrt(x) from is = rsqrt_t(x): x is in FP32, with one correction of the residual x - g^2 in FP64
-// (within about half an ulp), sqrt itself on the host.
+// sqrt(x) from is = rsqrt_t(x): x is on the device (within 2 ulp), sqrt itself on the host in FP64.
 template <class T> SIRIUS_HD __forceinline__ T sqrt_from(T x, T is) {
-#ifdef __HIP_DEVICE_COMPILE__
-    if constexpr (std::is_same_v<T, double>) {
-        const double g = x * is;
-        return ::fma(::fma(-g, g, x), 0.5 * is, g);
-    }
-    return x * is;
-#else
-    if constexpr (std::is_same_v<T, float>) return x * is;
-    return sqrt(x);
+#ifndef __HIP_DEVICE_COMPILE__
+    if constexpr (std::is_same_v<T, double>) return sqrt(x);
 #endif
+    return x * is;
 }
 
 // a * b + c with one rounding in the working precision (fmaf for FP32, also in host builds of
@@ -403,6 +396,13 @@ SIRIUS_HD __forceinline__ T event_radius_rate(const Spacetime<T>& s, const T x[4
     return r;
 }
 
+// Spacetime codes of the kernels' template parameter FAM: the metric families, and Kerr-Schild with
+// Lambda = 0 in every camera of the batch. Without the Lambda terms a step is one straight run of
+// instructions; with them each right-hand side carries a branch, seven multiply-adds by a zero
+// Lambda after it, and splits the step for the scheduler.
+enum { FAM_KS = 0, FAM_MT = 1, FAM_WARP = 2, FAM_KS_FLAT = 3 };
+constexpr bool is_ks(int fam) { return fam == FAM_KS || fam == FAM_KS_FLAT; }
+
 // Covariant metric values (no gradient), for initial conditions and emitter velocities.
 template <class T>
 SIRIUS_HD __forceinline__ void metric_cov(const Spacetime<T>& s, const T x[4], T g[4][4]) {
@@ -504,6 +504,57 @@ SIRIUS_HD __forceinline__ T rhs_ks(const Spacetime<scalar_t<T>>& s, const T x[4]
     return p[0] * k[0] + p[1] * k[1] + p[2] * k[2] + p[3] * k[3];
 }
 
+// The same with Lambda = 0 (FP64): one straight run of instructions, and l null gives l_mu k^mu = l^mu p_mu.
+// r is the Kerr radius of x.
+template <class T>
+SIRIUS_HD __forceinline__ T rhs_ks_flat(const Spacetime<scalar_t<T>>& s, const T x[4], const T p[4], T k[4], T dp[3],
+                                        T& r) {
+    using S = scalar_t<T>;
+    const T X = x[1], Y = x[2], Z = x[3];
+    const T R2v = X * X + Y * Y + Z * Z;
+    const T w = R2v - s.a2;                           // R^2 - a^2
+    T disc = tfma(S(4) * s.a2, Z * Z, w * w);         // (R^2 - a^2)^2 + 4 a^2 z^2
+    disc = fmax(disc, S(1e-20));  // guards only the ring singularity, deep inside the horizon
+    const T isq = rsqrt_t(disc);
+    const T sq = sqrt_from(disc, isq);
+    T r2 = (w + sq) * S(0.5);
+    r2 = fmax(r2, S(1e-10));
+    const T ir = rsqrt_t(r2);
+    r = sqrt_from(r2, ir);
+    const T rho = r2 + s.a2;
+    const T Dn = tfma(s.a2 * Z, Z, r2 * r2);          // r^4 + a^2 z^2
+    const T inv = rcp_t(rho * Dn);
+    const T irho = Dn * inv;
+    const T iDn = rho * inv;
+    const T l1 = tfma(r, X, s.a * Y) * irho;          // (r x + a y) / (r^2 + a^2)
+    const T l2 = tfma(r, Y, -s.a * X) * irho;         // (r y - a x) / (r^2 + a^2)
+    const T l3 = Z * ir;                              // z / r
+    const T q = S(2) * s.M * r - s.Q2;                // 2 M r - Q^2
+    const T H = q * r2 * iDn;
+    // k = (eta - H l l) p, l^mu = (-1, l1, l2, l3)
+    T lp = -p[0] + l1 * p[1] + l2 * p[2] + l3 * p[3];
+    T Hl = H * lp;
+    k[0] = -p[0] + Hl;
+    k[1] = p[1] - Hl * l1;
+    k[2] = p[2] - Hl * l2;
+    k[3] = p[3] - Hl * l3;
+    const T hl = S(0.5) * lp * lp, Hlk = H * lp;
+    // gradient of r
+    const T rs = r * isq;
+    const T drx = X * rs, dry = Y * rs, drz = Z * rho * ir * isq;
+    // H_r = (N_r - H Dn_r) / Dn with N = q r^2, N_r = r (6 M r - 2 Q^2), Dn_r = 4 r^3;
+    // H_z = -2 a^2 z H / Dn
+    const T Hr = (r * (S(6) * s.M * r - S(2) * s.Q2) - H * S(4) * r2 * r) * iDn;
+    const T Hz = -S(2) * s.a2 * Z * H * iDn;
+    const T A1 = (k[1] * r - k[2] * s.a) * irho, A2 = (k[1] * s.a + k[2] * r) * irho, A3 = k[3] * ir;
+    const T B = (k[1] * X + k[2] * Y - S(2) * r * (k[1] * l1 + k[2] * l2)) * irho - k[3] * l3 * ir;
+    const T Cr = hl * Hr + Hlk * B;
+    dp[0] = Cr * drx + Hlk * A1;
+    dp[1] = Cr * dry + Hlk * A2;
+    dp[2] = Cr * drz + hl * Hz + Hlk * A3;
+    return p[0] * k[0] + p[1] * k[1] + p[2] * k[2] + p[3] * k[3];
+}
+
 // Ellis wormhole, orbital-plane reduction (t, l, psi, w): g = diag(-1, 1, l^2 + b0^2, 1).
 template <class T>
 SIRIUS_HD __forceinline__ T rhs_mt(const Spacetime<scalar_t<T>>& s, const T x[4], const T p[4], T k[4], T dp[3]) {
@@ -570,7 +621,7 @@ SIRIUS_HD __forceinline__ void raise_index(const Spacetime<T>& s, const T x[4], 
         k[1] = p[1] - Hl * l1;
         k[2] = p[2] - Hl * l2;
         k[3] = p[3] - Hl * l3;
-        if (s.Lambda != T(0)) {
+        if (FAM == FAM_KS && s.Lambda != T(0)) {
             T c = -s.Lambda * (x[1] * x[1] + x[2] * x[2] + x[3] * x[3]) / T(3);
             T u0 = -T(1) - H;
             T fac = c * k[0] / (T(1) + c * u0);
@@ -588,11 +639,36 @@ struct Der {
     T k[4];
     T f[3];
     T pk;
+    T r;  // Kerr radius of the position (FAM_KS_FLAT)
 };
+// FP32 has no use for the radius, and the member alone would change which of two products the compiler
+// fuses into an add in the FP32 steps: the last bits of every FP32 ray.
+template <>
+struct Der<float> {
+    float k[4];
+    float f[3];
+    float pk;
+};
+
+// Dual-number steps: pins a stage's values and tangents here. Nothing in a stage's values depends on
+// the stages' tangents, so the compiler would run the values of all seven stages ahead and hold
+// every intermediate the tangents need (956 bytes spilled per lane).
+template <class T>
+SIRIUS_HD __forceinline__ void stage_fence(Der<T>&) {}
+template <class T>
+SIRIUS_HD __forceinline__ void stage_fence(Der<Dual<T, 1>>& d) {
+#ifdef __HIP_DEVICE_COMPILE__
+#pragma unroll
+    for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(d.k[i].v), "+v"(d.k[i].d[0]));
+#pragma unroll
+    for (int i = 0; i < 3; ++i) asm volatile("" : "+v"(d.f[i].v), "+v"(d.f[i].d[0]));
+#endif
+}
 
 template <class T, int FAM>
 SIRIUS_HD __forceinline__ void eval(const Spacetime<scalar_t<T>>& s, const T x[4], const T p[4], Der<T>& d) {
-    d.pk = rhs<T, FAM>(s, x, p, d.k, d.f);
+    if constexpr (FAM == FAM_KS_FLAT) d.pk = rhs_ks_flat<T>(s, x, p, d.k, d.f, d.r);
+    else d.pk = rhs<T, FAM>(s, x, p, d.k, d.f);
 }
 
 // Stage point y0 + inc, and the step update y0 + inc: with a compensated state (lo non-null) the
@@ -650,16 +726,19 @@ SIRIUS_HD __forceinline__ void dp45_step(const Spacetime<scalar_t<T>>& s, const 
 #pragma unroll
     for (int i = 0; i < 3; ++i) pt[i + 1] = stage_pt(p0[i + 1], h * (S(a21) * d1.f[i]), lo, 5 + i);
     eval<T, FAM>(s, xt, pt, d2);
+    stage_fence(d2);
 #pragma unroll
     for (int i = I0; i < 4; ++i) xt[i] = stage_pt(x0[i], h * (S(a31) * d1.k[i] + S(a32) * d2.k[i]), lo, i);
 #pragma unroll
     for (int i = 0; i < 3; ++i) pt[i + 1] = stage_pt(p0[i + 1], h * (S(a31) * d1.f[i] + S(a32) * d2.f[i]), lo, 5 + i);
     eval<T, FAM>(s, xt, pt, d3);
+    stage_fence(d3);
 #pragma unroll
     for (int i = I0; i < 4; ++i) xt[i] = stage_pt(x0[i], h * (S(a41) * d1.k[i] + S(a42) * d2.k[i] + S(a43) * d3.k[i]), lo, i);
 #pragma unroll
     for (int i = 0; i < 3; ++i) pt[i + 1] = stage_pt(p0[i + 1], h * (S(a41) * d1.f[i] + S(a42) * d2.f[i] + S(a43) * d3.f[i]), lo, 5 + i);
     eval<T, FAM>(s, xt, pt, d4);
+    stage_fence(d4);
 #pragma unroll
     for (int i = I0; i < 4; ++i)
         xt[i] = stage_pt(x0[i], h * (S(a51) * d1.k[i] + S(a52) * d2.k[i] + S(a53) * d3.k[i] + S(a54) * d4.k[i]), lo, i);
@@ -667,6 +746,7 @@ SIRIUS_HD __forceinline__ void dp45_step(const Spacetime<scalar_t<T>>& s, const 
     for (int i = 0; i < 3; ++i)
         pt[i + 1] = stage_pt(p0[i + 1], h * (S(a51) * d1.f[i] + S(a52) * d2.f[i] + S(a53) * d3.f[i] + S(a54) * d4.f[i]), lo, 5 + i);
     eval<T, FAM>(s, xt, pt, d5);
+    stage_fence(d5);
 #pragma unroll
     for (int i = I0; i < 4; ++i)
         xt[i] = stage_pt(x0[i], h * (S(a61) * d1.k[i] + S(a62) * d2.k[i] + S(a63) * d3.k[i] + S(a64) * d4.k[i] + S(a65) * d5.k[i]), lo, i);
@@ -674,6 +754,7 @@ SIRIUS_HD __forceinline__ void dp45_step(const Spacetime<scalar_t<T>>& s, const 
     for (int i = 0; i < 3; ++i)
         pt[i + 1] = stage_pt(p0[i + 1], h * (S(a61) * d1.f[i] + S(a62) * d2.f[i] + S(a63) * d3.f[i] + S(a64) * d4.f[i] + S(a65) * d5.f[i]), lo, 5 + i);
     eval<T, FAM>(s, xt, pt, d6);
+    stage_fence(d6);
     p1[0] = p0[0];
 #pragma unroll
     for (int i = I0; i < 4; ++i)
@@ -684,6 +765,7 @@ SIRIUS_HD __forceinline__ void dp45_step(const Spacetime<scalar_t<T>>& s, const 
         p1[i + 1] = sum_lo(p0[i + 1], h * (S(b1) * d1.f[i] + S(b3) * d3.f[i] + S(b4) * d4.f[i] + S(b5) * d5.f[i] +
                                            S(b6) * d6.f[i]), lo, lo1, 5 + i);
     eval<T, FAM>(s, x1, p1, d7);
+    stage_fence(d7);
     if (want_err) {
         err[0] = T(0);
 #pragma unroll

@@ -321,7 +321,7 @@ int sirius_hip_autotune(SiriusHipHandle hh, const SiriusHipCamera* cams, int n_c
     // every block size at full occupancy: on a sample, lower occupancies can time faster (its
     // short trace has little latency to hide) while on whole batches they ran up to 1.7x slower
     for (int bs : blocks) {
-        int occ = persistent_blocks_per_cu(false, B.family, B.tp.emission, B.tp.n_cam > 1, bs);
+        int occ = persistent_blocks_per_cu(false, B.kernels, B.tp.emission, B.tp.n_cam > 1, bs);
         int bpcs[1] = {occ};
         for (int j = 0; j < 1; ++j) {
             for (int rf : refills) {

@@ -438,6 +438,10 @@ int prepare_batch(Handle& H, const SiriusHipCamera* cams, int n_cam, const Siriu
     }
     if (off <= 0 || off > (int64_t)INT32_MAX - (1 << 20)) return H.fail(SIRIUS_HIP_E_INVALID, "ray count out of range");
     B.n = off;
+    B.kernels = B.family;
+    if (B.family == SIRIUS_METRIC_KERR_SCHILD &&
+        std::all_of(B.cc.begin(), B.cc.end(), [](const CamConst& c) { return c.Lambda == 0.0; }))
+        B.kernels = FAM_KS_FLAT;
     TraceParams& tp = B.tp;
     std::memset(&tp, 0, sizeof(tp));
     tp.rtol = o.rtol; tp.atol = o.atol; tp.h_init = o.h_init; tp.h_min = o.h_min; tp.h_max = o.h_max;
@@ -609,7 +613,7 @@ int run_trace(Handle& H, Batch& B, const SiriusHipTraceOpts& o, DevOut& dout, co
     if (time_it) (void)hipEventRecord(H.ev0, H.stream);
     if (o.integrator == SIRIUS_INTEGRATOR_SYMPLECTIC) {
         if (list_dev) return H.fail(SIRIUS_HIP_E_UNSUPPORTED, "symplectic integrator with a ray list");
-        if ((e = launch_symplectic(fp64, B.family, B.cams_dev, B.tp, dout, block, H.stream)) != hipSuccess)
+        if ((e = launch_symplectic(fp64, B.kernels, B.cams_dev, B.tp, dout, block, H.stream)) != hipSuccess)
             return H.hip_fail(e, "symplectic launch");
     } else if (!persistent) {
         // Grid schedule: one lane per ray, run to completion, no escalation queue (FP32 lanes
@@ -619,7 +623,7 @@ int run_trace(Handle& H, Batch& B, const SiriusHipTraceOpts& o, DevOut& dout, co
         TraceParams tp = B.tp;
         tp.escalate = 0;
         int grid = (int)std::max<int64_t>(1, (n_work + block - 1) / block);
-        if ((e = launch_trace_persistent(fp64, B.family, B.tp.emission, B.tp.n_cam > 1, B.cams_dev, tp, dout, list_dev,
+        if ((e = launch_trace_persistent(fp64, B.kernels, B.tp.emission, B.tp.n_cam > 1, B.cams_dev, tp, dout, list_dev,
                                          list_count_dev, n_work, work, work + 1, nullptr,
                                          (unsigned long long*)(work + 2), grid, block, 64, 0, H.stream)) !=
             hipSuccess)
@@ -628,9 +632,9 @@ int run_trace(Handle& H, Batch& B, const SiriusHipTraceOpts& o, DevOut& dout, co
         TraceParams tp = B.tp;
         tp.escalate = 0;
         int bpc = o.blocks_per_cu > 0 ? o.blocks_per_cu
-                                      : persistent_blocks_per_cu(true, B.family, B.tp.emission, B.tp.n_cam > 1, block);
+                                      : persistent_blocks_per_cu(true, B.kernels, B.tp.emission, B.tp.n_cam > 1, block);
         int refill = o.refill_min > 0 ? std::min(o.refill_min, 64) : 16;
-        if ((e = launch_trace_persistent(true, B.family, B.tp.emission, B.tp.n_cam > 1, B.cams_dev, tp, dout, list_dev,
+        if ((e = launch_trace_persistent(true, B.kernels, B.tp.emission, B.tp.n_cam > 1, B.cams_dev, tp, dout, list_dev,
                                          list_count_dev, n_work, work, work + 1, nullptr,
                                          (unsigned long long*)(work + 2), std::max(1, bpc * H.cu_count), block, refill,
                                          0, H.stream)) != hipSuccess)
@@ -722,9 +726,9 @@ int run_trace(Handle& H, Batch& B, const SiriusHipTraceOpts& o, DevOut& dout, co
             // sized for the whole chip and waves with nothing to trace retire at once.
             (void)hipEventRecord(H.ev_gate, H.stream);
             (void)hipStreamWaitEvent(H.stream2, H.ev_gate, 0);
-            int bpc64 = persistent_blocks_per_cu(true, B.family, B.tp.emission, B.tp.n_cam > 1, 64);
+            int bpc64 = persistent_blocks_per_cu(true, B.kernels, B.tp.emission, B.tp.n_cam > 1, 64);
             (void)hipEventRecord(H.ev_band0, H.stream2);
-            if ((e = launch_trace_persistent(true, B.family, B.tp.emission, B.tp.n_cam > 1, B.cams_dev, t64, dout, list_b,
+            if ((e = launch_trace_persistent(true, B.kernels, B.tp.emission, B.tp.n_cam > 1, B.cams_dev, t64, dout, list_b,
                                              work + 17, B.n, work + 12, work + 13, nullptr,
                                              (unsigned long long*)(work + 14), std::max(1, bpc64 * H.cu_count), 64, 1,
                                              SIRIUS_FLAG_ESCALATED, H.stream2)) != hipSuccess)
@@ -732,18 +736,18 @@ int run_trace(Handle& H, Batch& B, const SiriusHipTraceOpts& o, DevOut& dout, co
             (void)hipEventRecord(H.ev_band1, H.stream2);
         }
         int bpc = o.blocks_per_cu > 0 ? o.blocks_per_cu
-                                      : persistent_blocks_per_cu(false, B.family, B.tp.emission, B.tp.n_cam > 1, block);
+                                      : persistent_blocks_per_cu(false, B.kernels, B.tp.emission, B.tp.n_cam > 1, block);
         int grid = std::max(1, bpc * H.cu_count);
         int refill = o.refill_min > 0 ? std::min(o.refill_min, 64) : 16;
         if (time_it) (void)hipEventRecord(H.ev0, H.stream);
-        if ((e = launch_trace_persistent(false, B.family, B.tp.emission, B.tp.n_cam > 1, B.cams_dev, t32, dout, list_a,
+        if ((e = launch_trace_persistent(false, B.kernels, B.tp.emission, B.tp.n_cam > 1, B.cams_dev, t32, dout, list_a,
                                          count_a, cap_a, work, work + 1, esc, (unsigned long long*)(work + 2), grid,
                                          block, refill, 0, H.stream)) != hipSuccess)
             return H.hip_fail(e, "persistent launch");
         if (time_it) (void)hipEventRecord(H.ev1, H.stream);
         if (B.tp.escalate) {
-            int bpc64 = persistent_blocks_per_cu(true, B.family, B.tp.emission, B.tp.n_cam > 1, 64);
-            if ((e = launch_trace_persistent(true, B.family, B.tp.emission, B.tp.n_cam > 1, B.cams_dev, t64, dout, esc,
+            int bpc64 = persistent_blocks_per_cu(true, B.kernels, B.tp.emission, B.tp.n_cam > 1, 64);
+            if ((e = launch_trace_persistent(true, B.kernels, B.tp.emission, B.tp.n_cam > 1, B.cams_dev, t64, dout, esc,
                                              work + 1, cap_a, work + 4, work + 5, nullptr,
                                              (unsigned long long*)(work + 6), std::max(1, bpc64 * H.cu_count), 64, 1,
                                              SIRIUS_FLAG_ESCALATED, H.stream)) != hipSuccess)
@@ -765,8 +769,8 @@ int run_trace(Handle& H, Batch& B, const SiriusHipTraceOpts& o, DevOut& dout, co
             if (rc) return rc;
             TraceParams ta = fp64_reference_params(B.tp);
             if ((e = launch_fill((uint32_t*)aatt, 2, 0u, H.stream)) != hipSuccess) return H.hip_fail(e, "fill");
-            int bpc64 = persistent_blocks_per_cu(true, B.family, B.tp.emission, B.tp.n_cam > 1, 64);
-            if ((e = launch_trace_persistent(true, B.family, B.tp.emission, B.tp.n_cam > 1, B.cams_dev, ta, oa,
+            int bpc64 = persistent_blocks_per_cu(true, B.kernels, B.tp.emission, B.tp.n_cam > 1, 64);
+            if ((e = launch_trace_persistent(true, B.kernels, B.tp.emission, B.tp.n_cam > 1, B.cams_dev, ta, oa,
                                              list_audit, work + 10, B.n, work + 11, work + 5, nullptr, aatt,
                                              std::max(1, bpc64 * H.cu_count), 64, 1, SIRIUS_FLAG_AUDITED,
                                              H.stream)) != hipSuccess)
@@ -804,10 +808,10 @@ int run_trace(Handle& H, Batch& B, const SiriusHipTraceOpts& o, DevOut& dout, co
             (e = launch_fill(work + 21, 3, 0u, H.stream)) != hipSuccess)
             return H.hip_fail(e, "fill");
         TraceParams tr = fp64_reference_params(B.tp);
-        int bpc64 = persistent_blocks_per_cu(true, B.family, B.tp.emission, B.tp.n_cam > 1, 64);
+        int bpc64 = persistent_blocks_per_cu(true, B.kernels, B.tp.emission, B.tp.n_cam > 1, 64);
         if ((e = launch_precision_select(dout, B.n, o.precision_audit, o.audit_seed, plist, work + 21, H.stream)) !=
                 hipSuccess ||
-            (e = launch_trace_persistent(true, B.family, B.tp.emission, B.tp.n_cam > 1, B.cams_dev, tr, oa, plist,
+            (e = launch_trace_persistent(true, B.kernels, B.tp.emission, B.tp.n_cam > 1, B.cams_dev, tr, oa, plist,
                                          work + 21, B.n, work + 22, work + 23, nullptr, patt,
                                          std::max(1, bpc64 * H.cu_count), 64, 1, SIRIUS_FLAG_AUDITED, H.stream)) !=
                 hipSuccess ||

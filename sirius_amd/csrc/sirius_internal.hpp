@@ -132,6 +132,7 @@ struct Batch {
     CamConst* cams_dev = nullptr;
     TraceParams tp;
     int family = 0;
+    int kernels = 0;  // spacetime code of the kernels (FAM_*): the family, or FAM_KS_FLAT
     int64_t n = 0;
 };
 

@@ -386,7 +386,7 @@ SIRIUS_HD __forceinline__ int ray_attempt(Ray<T, FAM>& R, const CamConst* cams, 
                                           const TraceParams& tp, const DevOut& o) {
     constexpr bool fp32 = sizeof(T) == 4;
     constexpr bool TIME = !fp32;
-    constexpr bool vol = (FAM == 0) && EMIT == SIRIUS_EMISSION_VOLUMETRIC;
+    constexpr bool vol = is_ks(FAM) && EMIT == SIRIUS_EMISSION_VOLUMETRIC;
     T hmax = T(tp.h_max);
     T r0 = T(0);
     if (tp.far_slope > 0 || tp.step_rexp > 0) r0 = R.r_cur;
@@ -406,14 +406,27 @@ SIRIUS_HD __forceinline__ int ray_attempt(Ray<T, FAM>& R, const CamConst* cams, 
                             fp32 ? R.lo : nullptr, lo1);
     R.attempts++;
     T e = T(0);
+    if constexpr (fp32) {
 #pragma unroll
-    for (int i = TIME ? 0 : 1; i < 4; ++i) {
-        T q;
-        if constexpr (fp32) q = err[i] / (T(tp.atol) + T(tp.rtol) * fabs(x1[i]));
-        else q = err[i] * rcp_t(T(tp.atol) + T(tp.rtol) * fabs(x1[i]));
-        e += q * q;
+        for (int i = 1; i < 4; ++i) {
+            T q = err[i] / (T(tp.atol) + T(tp.rtol) * fabs(x1[i]));
+            e += q * q;
+        }
+        e = sqrt(e * T(1.0 / 3.0));
+    } else {
+        // the four tolerances' reciprocals from that of their product. Held in [1e-70, 1e70], which keeps
+        // the product in range: against any smaller tolerance a component's error is exactly zero or too
+        // large either way, and a position beyond 1e70 comes of a step that is rejected either way.
+        const T atol = fmax(T(tp.atol), T(1e-70));
+        T tol[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) tol[i] = fmin(atol + T(tp.rtol) * fabs(x1[i]), T(1e70));
+        const T t01 = tol[0] * tol[1], t23 = tol[2] * tol[3], inv = rcp_t(t01 * t23);
+        const T i01 = inv * t23, i23 = inv * t01;
+        const T q[4] = {err[0] * (i01 * tol[1]), err[1] * (i01 * tol[0]), err[2] * (i23 * tol[3]),
+                        err[3] * (i23 * tol[2])};
+        e = sqrt((q[0] * q[0] + q[1] * q[1] + q[2] * q[2] + q[3] * q[3]) * T(0.25));
     }
-    e = sqrt(e * (TIME ? T(0.25) : T(1.0 / 3.0)));
     if (!(e <= T(1))) {
         R.h = next_step(R.h, e, T(tp.h_min), hmax);
         R.rejected++;
@@ -438,7 +451,7 @@ SIRIUS_HD __forceinline__ int ray_attempt(Ray<T, FAM>& R, const CamConst* cams, 
     // ---- thin disk: first crossing of the equatorial plane inside [r_in, r_out], decided on
     // the Hermite-interpolated crossing radius, reported from the landed state ----
     T th_disk = T(1);
-    if constexpr (FAM == 0 && EMIT == SIRIUS_EMISSION_THIN_DISK) {
+    if constexpr (is_ks(FAM) && EMIT == SIRIUS_EMISSION_THIN_DISK) {
         if (R.x[3] * x1[3] < T(0)) {
             T xc[4];
             if constexpr (fp32) {
@@ -459,18 +472,21 @@ SIRIUS_HD __forceinline__ int ray_attempt(Ray<T, FAM>& R, const CamConst* cams, 
             if (rc >= T(c.r_in) && rc <= T(c.r_out)) ev = SIRIUS_RAY_DISK;
         }
     }
-    T r1 = event_radius(s, x1);
+    // without Lambda: the radius of x1 from the step's last right-hand side, which is evaluated there
+    T r1;
+    if constexpr (FAM == FAM_KS_FLAT) r1 = d1.r;
+    else r1 = event_radius(s, x1);
     if (ev < 0) {
-        if (FAM == 0 && r1 < T(c.r_cap)) {
+        if (is_ks(FAM) && r1 < T(c.r_cap)) {
             ev = SIRIUS_RAY_CAPTURED;
             target = T(c.r_cap);
-            locate = event_radius(s, R.x) > target;
+            locate = (fp32 ? event_radius(s, R.x) : R.r_cur) > target;
         } else if (r1 > T(tp.r_escape)) {
             T radial = (FAM == 1) ? x1[1] * d1.k[1] : x1[1] * d1.k[1] + x1[2] * d1.k[2] + x1[3] * d1.k[3];
             if (radial > T(0)) {
                 ev = SIRIUS_RAY_ESCAPED;
                 target = T(tp.r_escape);
-                locate = event_radius(s, R.x) < target;
+                locate = (fp32 ? event_radius(s, R.x) : R.r_cur) < target;
             }
         }
     }
@@ -523,7 +539,7 @@ SIRIUS_HD __forceinline__ int ray_attempt(Ray<T, FAM>& R, const CamConst* cams, 
         // grows exponentially with each turn
         if (FAM == 1 && tp.escalate && fabs(R.p[2] - T(c.b0)) < T(0.1 * c.b0)) return ST_ESCALATE;
         // escalation: a radial turning point inside the photon region
-        if (FAM == 0 && tp.escalate) {
+        if (is_ks(FAM) && tp.escalate) {
             T vr = x1[1] * d1.k[1] + x1[2] * d1.k[2] + x1[3] * d1.k[3];
             if (R.vr_prev < T(0) && vr >= T(0) && r1 < T(tp.escalate_margin * c.r_ph_retro)) return ST_ESCALATE;
             R.vr_prev = vr;
@@ -687,11 +703,14 @@ __device__ __forceinline__ void persistent_body(const CamConst* __restrict__ cam
 // FP64 variants: register allocation left to the compiler (the thin-disk tracer takes 256 VGPRs plus
 // 20 AGPRs, one wave per SIMD). The single-camera warp tracer, which re-traces wall crossers (a
 // tenth of a warp frame, too few rays to hide one wave's latency), is held to two waves (202
-// registers, no spills). Bound by FP64 issue: with roots and reciprocals by Newton steps, events
-// located by Newton iteration and landings deferred to the refill (land, above), the thin-disk
-// tracer runs the 1283x721 Kerr frame in 5.62 ms (8.99 with IEEE roots and divisions, 52 halvings
-// per event and each ray landed as it ended), the warp tracer its 1024x1024 frame's wall crossers
-// in 0.87 ms (1.65), the wormhole tracer its frame's near-throat rays in 0.41 ms (0.72).
+// registers, no spills). Bound by FP64 issue, so by the instructions of a step: with roots and
+// reciprocals of third order, no Lambda terms where no camera has any, the radius taken from the
+// step's last right-hand side, one reciprocal for the error norm, events located by Newton iteration
+// and landings deferred to the refill (land, above), the thin-disk tracer runs the 1283x721 Kerr
+// frame in 4.57 ms (5.62 with the Lambda terms and two Newton steps per root; 8.99 with IEEE roots
+// and divisions, 52 halvings per event and each ray landed as it ended), the warp tracer its
+// 1024x1024 frame's wall crossers in 0.87 ms (1.65), the wormhole tracer its frame's near-throat
+// rays in 0.38 ms (0.72).
 constexpr int fp64_min_waves(int fam, bool multi) { return fam == 2 && !multi ? 2 : 1; }
 // The persistent tracers start on a 4 KiB boundary of the code object. Their loops are about
 // 19 KiB of instructions, and where the linker happened to place them changed their speed: the
@@ -887,8 +906,8 @@ __global__ void k_fill_u32(uint32_t* p, int n, uint32_t v) {
 // A(h/2) B(h/2) C(h) B(h/2) A(h/2), composed to 4th order with the Yoshida triple jump
 // (weights PHSI001A.h:43-47). Fixed step; disk crossing on the cubic Hermite interpolant.
 // Bound by the serial chain of right-hand sides of the longest ray (a 320x181 Kerr frame at
-// h = 0.02 has 905 waves for 1024 SIMDs): 36 ms with 9 evaluations per step and their roots by
-// Newton steps, 63-65 ms with 12 and IEEE roots and divisions.
+// h = 0.02 has 905 waves for 1024 SIMDs): 28 ms with 9 evaluations per step, without Lambda
+// terms (36 ms with them), 63-65 ms with 12 and IEEE roots and divisions.
 // ------------------------------------------------------------------------------------------
 // Flow A with H's derivatives D at (q, y). A changes neither q nor y, so the A that ends a substep
 // and the A that begins the next have the same D: it is evaluated once for both (9 evaluations per
@@ -956,8 +975,10 @@ __global__ __launch_bounds__(256) void k_symplectic_grid(const CamConst* __restr
         bool bad = false;
         for (int i = 0; i < 4; ++i) bad |= !sfinite(q[i]) || !sfinite(p[i]);
         if (bad) { cls = SIRIUS_RAY_FAILED; break; }
-        T r = event_radius(s, q);
-        if (FAM == 0 && tp.emission == SIRIUS_EMISSION_THIN_DISK && q0[3] * q[3] < T(0)) {
+        T r;
+        if constexpr (FAM == FAM_KS_FLAT) r = DA.r;  // DA is at (q, y)
+        else r = event_radius(s, q);
+        if (is_ks(FAM) && tp.emission == SIRIUS_EMISSION_THIN_DISK && q0[3] * q[3] < T(0)) {
             // the crossing is located on the cubic Hermite interpolant of the whole state over the
             // step (H's derivatives at both ends) and the ray ends there: a linear interpolant
             // would add an O(h^2) null-constraint error of its own at the hit
@@ -979,7 +1000,7 @@ __global__ __launch_bounds__(256) void k_symplectic_grid(const CamConst* __restr
                 break;
             }
         }
-        if (FAM == 0 && r < T(c.r_cap)) { cls = SIRIUS_RAY_CAPTURED; break; }
+        if (is_ks(FAM) && r < T(c.r_cap)) { cls = SIRIUS_RAY_CAPTURED; break; }
         if (r > T(tp.r_escape) && r > rprev) { cls = SIRIUS_RAY_ESCAPED; break; }
         rprev = r;
     }
@@ -999,16 +1020,17 @@ __global__ __launch_bounds__(256) void k_symplectic_grid(const CamConst* __restr
 // ------------------------------------------------------------------------------------------
 namespace sirius {
 
-// Kernel variant for (precision, family, emission): emission only applies to Kerr-Schild.
+// Kernel variant for (precision, spacetime code, emission): emission only applies to Kerr-Schild.
+#define SIRIUS_VARIANTS_KS(MACRO, T, F, M)                                                        \
+    if (emission == SIRIUS_EMISSION_THIN_DISK) MACRO(T, F, SIRIUS_EMISSION_THIN_DISK, M);         \
+    else if (emission == SIRIUS_EMISSION_VOLUMETRIC) MACRO(T, F, SIRIUS_EMISSION_VOLUMETRIC, M);  \
+    else MACRO(T, F, SIRIUS_EMISSION_NONE, M)
 #define SIRIUS_VARIANTS_M(MACRO, T, M)                                                            \
     switch (family) {                                                                             \
         case 1: MACRO(T, 1, SIRIUS_EMISSION_NONE, M); break;                                      \
         case 2: MACRO(T, 2, SIRIUS_EMISSION_NONE, M); break;                                      \
-        default:                                                                                  \
-            if (emission == SIRIUS_EMISSION_THIN_DISK) MACRO(T, 0, SIRIUS_EMISSION_THIN_DISK, M);    \
-            else if (emission == SIRIUS_EMISSION_VOLUMETRIC) MACRO(T, 0, SIRIUS_EMISSION_VOLUMETRIC, M); \
-            else MACRO(T, 0, SIRIUS_EMISSION_NONE, M);                                            \
-            break;                                                                                \
+        case FAM_KS_FLAT: SIRIUS_VARIANTS_KS(MACRO, T, (sizeof(T) == 8 ? FAM_KS_FLAT : FAM_KS), M); break; \
+        default: SIRIUS_VARIANTS_KS(MACRO, T, FAM_KS, M); break;                                  \
     }
 #define SIRIUS_VARIANTS(MACRO, T)                      \
     if (multi) { SIRIUS_VARIANTS_M(MACRO, T, true) }   \
@@ -1075,6 +1097,7 @@ hipError_t launch_symplectic(bool fp64, int family, const CamConst* cams, const 
         switch (family) {
             case 1: hipLaunchKernelGGL((k_symplectic_grid<double, 1>), g, b, 0, st, cams, tp, o); break;
             case 2: hipLaunchKernelGGL((k_symplectic_grid<double, 2>), g, b, 0, st, cams, tp, o); break;
+            case FAM_KS_FLAT: hipLaunchKernelGGL((k_symplectic_grid<double, FAM_KS_FLAT>), g, b, 0, st, cams, tp, o); break;
             default: hipLaunchKernelGGL((k_symplectic_grid<double, 0>), g, b, 0, st, cams, tp, o); break;
         }
     } else {
