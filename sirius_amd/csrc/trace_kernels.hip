@@ -284,25 +284,35 @@ SIRIUS_HD __forceinline__ void vol_accumulate(Ray<T, FAM>& R, const CamConst& c,
         T nue = -ut * (pq[0] + Om * (xq[1] * pq[2] - xq[2] * pq[1]));
         T nuo = -pq[0] * T(c.obs_norm);
         if (nue <= T(0) || nuo <= T(0)) continue;
-        T gf = nuo / nue;
         T dl = gw[q] * hh;
         T dtau = T(tp.vol_kappa) * rho * nue * dl;
-        T w = rho * (nuo * nuo * nuo / (nue * nue)) * dl * exp(-(R.tau + T(0.5) * dtau));
-        T tv = pow_pos(T(6) / r, T(0.75));
+        // w: the node's weight; ig = nu_e / nu_o; it = 1 / T_v
+        T w, ig, it;
+        if constexpr (sizeof(T) == 4) {
+            w = rho * (nuo * nuo * nuo * rcp_t(nue * nue)) * dl * exp_neg(-(R.tau + T(0.5) * dtau));
+            ig = nue * rcp_t(nuo);
+            it = pow_pos(r * T(1.0 / 6.0), T(0.75));
+        } else {
+            w = rho * (nuo * nuo * nuo / (nue * nue)) * dl * exp(-(R.tau + T(0.5) * dtau));
+            ig = nue / nuo;
+            it = T(1) / pow_pos(T(6) / r, T(0.75));
+        }
         T xk = T(xk0), qk = T(qk0);
         if (tp.n_bins <= SIRIUS_VOL_REG) {
 #pragma unroll
             for (int k = 0; k < SIRIUS_VOL_REG; ++k) {
                 if (k < tp.n_bins) {
-                    T xe = xk / gf;
-                    R.vacc[k] += w * xe * xe * xe / expm1(xe / tv);
+                    const T xe = xk * ig;
+                    if constexpr (sizeof(T) == 4)
+                        R.vacc[k] = tfma(w * xe * xe * xe, rcp_t(expm1_pos(xe * it)), R.vacc[k]);
+                    else R.vacc[k] += w * xe * xe * xe / expm1(xe * it);
                 }
                 xk *= qk;
             }
         } else {
             for (int k = 0; k < tp.n_bins; ++k, xk *= qk) {
-                T xe = xk / gf;
-                o.vol_acc[(int64_t)k * o.n_rays + R.id] += (double)(w * xe * xe * xe / expm1(xe / tv));
+                const T xe = xk * ig;
+                o.vol_acc[(int64_t)k * o.n_rays + R.id] += (double)(w * xe * xe * xe / expm1(xe * it));
             }
         }
         R.tau += dtau;
