@@ -72,6 +72,7 @@ struct TraceParams {
     // nearest the critical curve, the longest, start first); null for none
     const int32_t* first_list;
     const uint32_t* first_count;
+    int tile_lw;  // order in which whole batches are taken (tile_pixel)
 };
 
 // Null-drift histogram of the statistics pass: log10 bins of 1/16 decade over [1e-20, 1).
@@ -402,6 +403,19 @@ SIRIUS_HD __forceinline__ T event_radius_rate(const Spacetime<T>& s, const T x[4
 // Lambda after it, and splits the step for the scheduler.
 enum { FAM_KS = 0, FAM_MT = 1, FAM_WARP = 2, FAM_KS_FLAT = 3 };
 constexpr bool is_ks(int fam) { return fam == FAM_KS || fam == FAM_KS_FLAT; }
+
+// Order in which the tracers take an image's rays: position t of a width x height image -> pixel, in
+// bands of 64 >> lw rows cut into tiles of 1 << lw columns (smaller at the right and bottom edges), so
+// the 64 rays of a wave are one tile: a row of 64 pixels (lw = 6) or a square of 8 x 8 (lw = 3).
+constexpr int TILE_ROW = 6, TILE_SQUARE = 3;
+SIRIUS_HD __forceinline__ int64_t tile_pixel(int width, int height, int lw, int64_t t) {
+    const uint32_t w = (uint32_t)width, h = (uint32_t)height, u = (uint32_t)t;  // w h < 2^31
+    const uint32_t tw = 1u << lw, th = 64u >> lw;
+    const uint32_t band = u / (th * w), y0 = th * band, bh = h - y0 < th ? h - y0 : th, v = u - y0 * w;
+    const uint32_t col = v / (tw * bh), x0 = tw * col, q = v - x0 * bh;
+    const uint32_t cw = w - x0 < tw ? w - x0 : tw, y = q / cw;
+    return (int64_t)(y0 + y) * w + x0 + (q - y * cw);
+}
 
 // Covariant metric values (no gradient), for initial conditions and emitter velocities.
 template <class T>

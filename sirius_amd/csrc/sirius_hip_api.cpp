@@ -40,7 +40,7 @@ hipError_t launch_reduce_stats(const DevOut& o, int64_t n, unsigned long long* a
                                hipStream_t st);
 hipError_t launch_critical_distance(const CamConst* cams, int n_cam, const float* tabs, int64_t n, float* out,
                                     hipStream_t st);
-hipError_t launch_gate(const CamConst* cams, int n_cam, const float* tabs, int64_t n, double band, double crit_band,
+hipError_t launch_gate(const CamConst* cams, int n_cam, const float* tabs, int tile_lw, int64_t n, double band, double crit_band,
                        double long_band, int32_t* list_a, int32_t* list_b, int32_t* list_l, uint32_t* counts,
                        uint8_t* flags, hipStream_t st);
 hipError_t launch_sur_audit(const CamConst* cams, const TraceParams& tp, const DevOut& oa, const DevOut& o,
@@ -462,6 +462,13 @@ int prepare_batch(Handle& H, const SiriusHipCamera* cams, int n_cam, const Siriu
     tp.n_bins = o.n_bins;
     bin_centres(o.x_min, o.x_max, o.n_bins, tp.bin_x0, tp.bin_q);
     tp.emission = B.family == SIRIUS_METRIC_KERR_SCHILD ? o.emission : SIRIUS_EMISSION_NONE;
+    // Waves of squares where rays are long: a wave runs as long as its longest ray, 1.36 times its rays'
+    // mean for rows of 64 pixels and 1.12 for 8 x 8 squares of the volumetric 256 x 256 images (tracer
+    // 4.07 ms in rows, 3.69 in squares; FP64 1283x721 Kerr frame 3.38 and 3.07; FP32 wormhole frame
+    // 0.48 and 0.43). FP32 thin-disk rays end after 15 steps, so their results' stores count: a row of
+    // 64 fills whole cache lines in one XCD's L2, a square's 32-byte pieces of a line meet in several
+    // (1080p tracer 1.19 ms in rows, 1.38 in squares).
+    tp.tile_lw = o.precision == SIRIUS_PRECISION_FP32_ESCALATE && tp.emission == SIRIUS_EMISSION_THIN_DISK ? TILE_ROW : TILE_SQUARE;
     tp.sym_order = o.symplectic_order;
     tp.n_cam = n_cam;
     // escalation machinery of the FP32 path: always on for the wormhole throat and the warp wall;
@@ -590,6 +597,14 @@ double flops_per_symplectic_step(int family, int order) {
     return (order >= 4 ? 3.0 : 1.0) * (4.0 * rhs + 56.0 + 72.0);
 }
 
+// Idle lanes at which a wave of a persistent queue refills: the caller's choice, or a quarter wave
+// where neighbours in the queue end apart (rows, lists of picked rays) and the whole wave where they
+// end together (squares: FP32 warp bubble 0.75 ms at 16, 0.66 at 64; volumetric 4.23 and 3.97).
+static int default_refill(const SiriusHipTraceOpts& o, const Batch& B, bool picked) {
+    if (o.refill_min > 0) return std::min(o.refill_min, 64);
+    return picked || B.tp.tile_lw == TILE_ROW ? 16 : 64;
+}
+
 int run_trace(Handle& H, Batch& B, const SiriusHipTraceOpts& o, DevOut& dout, const int32_t* list_dev,
               const uint32_t* list_count_dev, int64_t list_cap, SiriusHipStats* stats, bool time_it) {
     hipError_t e;
@@ -615,30 +630,48 @@ int run_trace(Handle& H, Batch& B, const SiriusHipTraceOpts& o, DevOut& dout, co
         if (list_dev) return H.fail(SIRIUS_HIP_E_UNSUPPORTED, "symplectic integrator with a ray list");
         if ((e = launch_symplectic(fp64, B.kernels, B.cams_dev, B.tp, dout, block, H.stream)) != hipSuccess)
             return H.hip_fail(e, "symplectic launch");
-    } else if (!persistent) {
+    } else if (!persistent || fp64) {
         // Grid schedule: one lane per ray, run to completion, no escalation queue (FP32 lanes
         // run to the end in FP32). It is the tracer kernel with a static assignment: a grid of
         // one wave per 64 rays, each wave taking one batch of 64 consecutive list slots when all
         // its lanes are idle, so both schedules run the same compiled code, bit for bit.
         TraceParams tp = B.tp;
         tp.escalate = 0;
-        int grid = (int)std::max<int64_t>(1, (n_work + block - 1) / block);
+        const bool picked = list_dev != nullptr;
+        // A whole FP64 Kerr-Schild batch of more waves than the chip has SIMDs takes the rays near
+        // the critical curve first, as the FP32 path does: the longest run 1061 steps of a mean of 59
+        // on the 1283x721 frame, and started in the middle of it they run on alone (tracer 4.57 ms,
+        // 3.38 with them first). Batches that find no memory for the lists (and no-allocation
+        // scratch, whose limit stays) go without.
+        if (fp64 && !picked && B.family == SIRIUS_METRIC_KERR_SCHILD && !H.arena && B.n > 256 * (int64_t)H.cu_count) {
+            int none = 0;
+            int32_t* la = (int32_t*)H.scratch("gate_a", 4 * (size_t)B.n, &none);
+            int32_t* ll = none ? nullptr : (int32_t*)H.scratch("gate_l", 4 * (size_t)B.n, &none);
+            float* tabs = none ? nullptr : upload_critical_tables(H, B, &none);
+            if (none) {
+                (void)hipGetLastError();  // the failed allocation's
+            } else {
+                if ((e = launch_gate(B.cams_dev, (int)B.cc.size(), tabs, B.tp.tile_lw, B.n, 0.0, 0.0, SIRIUS_LONG_BAND, la,
+                                     la, ll, work + 16, dout.flags, H.stream)) != hipSuccess)
+                    return H.hip_fail(e, "gate launch");
+                list_dev = la;
+                list_count_dev = work + 16;
+                tp.first_list = ll;
+                tp.first_count = work + 18;
+            }
+        }
+        int grid = (int)std::max<int64_t>(1, (n_work + block - 1) / block), refill = 64;
+        if (persistent) {
+            const int bpc = o.blocks_per_cu > 0 ? o.blocks_per_cu
+                                                : persistent_blocks_per_cu(true, B.kernels, B.tp.emission, B.tp.n_cam > 1, block);
+            grid = std::max(1, bpc * H.cu_count);
+            refill = default_refill(o, B, picked);
+        }
         if ((e = launch_trace_persistent(fp64, B.kernels, B.tp.emission, B.tp.n_cam > 1, B.cams_dev, tp, dout, list_dev,
                                          list_count_dev, n_work, work, work + 1, nullptr,
-                                         (unsigned long long*)(work + 2), grid, block, 64, 0, H.stream)) !=
+                                         (unsigned long long*)(work + 2), grid, block, refill, 0, H.stream)) !=
             hipSuccess)
-            return H.hip_fail(e, "grid launch");
-    } else if (fp64) {
-        TraceParams tp = B.tp;
-        tp.escalate = 0;
-        int bpc = o.blocks_per_cu > 0 ? o.blocks_per_cu
-                                      : persistent_blocks_per_cu(true, B.kernels, B.tp.emission, B.tp.n_cam > 1, block);
-        int refill = o.refill_min > 0 ? std::min(o.refill_min, 64) : 16;
-        if ((e = launch_trace_persistent(true, B.kernels, B.tp.emission, B.tp.n_cam > 1, B.cams_dev, tp, dout, list_dev,
-                                         list_count_dev, n_work, work, work + 1, nullptr,
-                                         (unsigned long long*)(work + 2), std::max(1, bpc * H.cu_count), block, refill,
-                                         0, H.stream)) != hipSuccess)
-            return H.hip_fail(e, "persistent launch");
+            return H.hip_fail(e, "trace launch");
         if (time_it) (void)hipEventRecord(H.ev1, H.stream);
     } else {
         // FP32 path. (1) Gate (Kerr-Schild): every ray's distance from the critical curve; rays
@@ -689,7 +722,7 @@ int run_trace(Handle& H, Batch& B, const SiriusHipTraceOpts& o, DevOut& dout, co
             if (rc) return rc;
             uint32_t* counts = work + 16;
             const double long_band = SIRIUS_LONG_BAND;  // the longest rays first
-            if ((e = launch_gate(B.cams_dev, (int)B.cc.size(), tabs, B.n, std::max(o.escalate_band, 0.0),
+            if ((e = launch_gate(B.cams_dev, (int)B.cc.size(), tabs, B.tp.tile_lw, B.n, std::max(o.escalate_band, 0.0),
                                  std::max(o.critical_band, 0.0), long_band, la, list_b, ll, counts, dout.flags,
                                  H.stream)) != hipSuccess)
                 return H.hip_fail(e, "gate launch");
@@ -738,7 +771,7 @@ int run_trace(Handle& H, Batch& B, const SiriusHipTraceOpts& o, DevOut& dout, co
         int bpc = o.blocks_per_cu > 0 ? o.blocks_per_cu
                                       : persistent_blocks_per_cu(false, B.kernels, B.tp.emission, B.tp.n_cam > 1, block);
         int grid = std::max(1, bpc * H.cu_count);
-        int refill = o.refill_min > 0 ? std::min(o.refill_min, 64) : 16;
+        int refill = default_refill(o, B, sur || list_dev != nullptr);
         if (time_it) (void)hipEventRecord(H.ev0, H.stream);
         if ((e = launch_trace_persistent(false, B.kernels, B.tp.emission, B.tp.n_cam > 1, B.cams_dev, t32, dout, list_a,
                                          count_a, cap_a, work, work + 1, esc, (unsigned long long*)(work + 2), grid,

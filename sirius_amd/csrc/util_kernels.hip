@@ -107,24 +107,26 @@ hipError_t launch_critical_distance(const CamConst* cams, int n_cam, const float
 // tracer takes them first: they wind near the photon region and are the longest) and all
 // others to list A; rays within `crit_band` get SIRIUS_FLAG_CRITICAL in flags[] (every ray's
 // flag byte is written). counts[0..2] = |A|, |B|, |L|. A block
-// of 256 threads classifies a contiguous chunk of GATE_RAYS rays and reserves its slots with
+// of 256 threads classifies a chunk of GATE_RAYS rays, contiguous in tile order, and reserves its slots with
 // one atomic per list (device-scope atomics on one address serialise, so one per wave is too
-// many at 1080p); within a chunk the lists keep ray order.
+// many at 1080p); within a chunk the lists keep tile order.
 constexpr int GATE_PASSES = 8;
 constexpr int GATE_RAYS = 256 * GATE_PASSES;
 
-// |distance| of ray id from its camera's critical curve (M); +inf for other spacetimes
+// |distance| of a ray from its camera's critical curve (M), +inf for other spacetimes: the ray at
+// position t of the batch in tile order; id is its number.
 __device__ __forceinline__ float gate_distance(const CamConst* __restrict__ cams, int n_cam,
-                                              const float* __restrict__ tabs, int64_t id) {
+                                              const float* __restrict__ tabs, int tile_lw, int64_t t, int64_t& id) {
     int lo = 0, hi = n_cam - 1;
     while (lo < hi) {
         int mid = (lo + hi + 1) >> 1;
-        if (cams[mid].offset <= id) lo = mid; else hi = mid - 1;
+        if (cams[mid].offset <= t) lo = mid; else hi = mid - 1;
     }
     const CamConst& c = cams[lo];
+    const int64_t pix = tile_pixel(c.width, c.height, tile_lw, t - c.offset);
+    id = c.offset + pix;
     if (c.family != 0) return INFINITY;
     // FP32 is ample for band membership (alpha, beta ~ 10 M, band ~ 0.1 M)
-    int64_t pix = id - c.offset;
     Spacetime<float> s = make_spacetime<float>(c);
     float x[4], p[4];
     init_state<float>(c, s, (int)(pix % c.width), (int)(pix / c.width), x, p);
@@ -132,7 +134,7 @@ __device__ __forceinline__ float gate_distance(const CamConst* __restrict__ cams
 }
 
 __global__ __launch_bounds__(256) void k_gate(const CamConst* __restrict__ cams, int n_cam,
-                                              const float* __restrict__ tabs, int64_t n, float band,
+                                              const float* __restrict__ tabs, int tile_lw, int64_t n, float band,
                                               float crit_band, float long_band, int32_t* __restrict__ list_a,
                                               int32_t* __restrict__ list_b, int32_t* __restrict__ list_l,
                                               uint32_t* __restrict__ counts, uint8_t* __restrict__ flags) {
@@ -141,12 +143,15 @@ __global__ __launch_bounds__(256) void k_gate(const CamConst* __restrict__ cams,
     const int lane = __lane_id(), wave = threadIdx.x >> 6;
     const int64_t chunk = (int64_t)blockIdx.x * GATE_RAYS;
     const unsigned long long below = lane ? ((1ull << lane) - 1ull) : 0ull;
+    int32_t ids[GATE_PASSES];
     uint32_t kinds = 0;  // 2 bits per pass: 0 list A, 1 list B (band), 2 list L (long), 3 invalid
 #pragma unroll
     for (int k = 0; k < GATE_PASSES; ++k) {
-        int64_t id = chunk + k * 256 + threadIdx.x;
-        bool valid = id < n;
-        float d = valid ? gate_distance(cams, n_cam, tabs, id) : INFINITY;
+        const int64_t t = chunk + k * 256 + threadIdx.x;
+        const bool valid = t < n;
+        int64_t id = 0;
+        float d = valid ? gate_distance(cams, n_cam, tabs, tile_lw, t, id) : INFINITY;
+        ids[k] = (int32_t)id;
         uint32_t kind = !valid ? 3u : (d < band ? 1u : (d < long_band ? 2u : 0u));
         if (valid) flags[id] = d < crit_band ? (uint8_t)SIRIUS_FLAG_CRITICAL : (uint8_t)0;
         kinds |= kind << (2 * k);
@@ -172,20 +177,20 @@ __global__ __launch_bounds__(256) void k_gate(const CamConst* __restrict__ cams,
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < GATE_PASSES; ++k) {
-        int64_t id = chunk + k * 256 + threadIdx.x;
+        const int32_t id = ids[k];
         uint32_t kind = (kinds >> (2 * k)) & 3u;
         unsigned long long ma = __ballot(kind == 0), mb = __ballot(kind == 1), ml = __ballot(kind == 2);
-        if (kind == 0) list_a[base[0] + off_a[k][wave] + __popcll(ma & below)] = (int32_t)id;
-        else if (kind == 1) list_b[base[1] + off_b[k][wave] + __popcll(mb & below)] = (int32_t)id;
-        else if (kind == 2) list_l[base[2] + off_l[k][wave] + __popcll(ml & below)] = (int32_t)id;
+        if (kind == 0) list_a[base[0] + off_a[k][wave] + __popcll(ma & below)] = id;
+        else if (kind == 1) list_b[base[1] + off_b[k][wave] + __popcll(mb & below)] = id;
+        else if (kind == 2) list_l[base[2] + off_l[k][wave] + __popcll(ml & below)] = id;
     }
 }
 
-hipError_t launch_gate(const CamConst* cams, int n_cam, const float* tabs, int64_t n, double band, double crit_band,
+hipError_t launch_gate(const CamConst* cams, int n_cam, const float* tabs, int tile_lw, int64_t n, double band, double crit_band,
                        double long_band, int32_t* list_a, int32_t* list_b, int32_t* list_l, uint32_t* counts,
                        uint8_t* flags, hipStream_t st) {
     hipLaunchKernelGGL(k_gate, dim3((unsigned)((n + GATE_RAYS - 1) / GATE_RAYS)), dim3(256), 0, st, cams, n_cam, tabs,
-                       n, (float)band, (float)crit_band, (float)long_band, list_a, list_b, list_l, counts, flags);
+                       tile_lw, n, (float)band, (float)crit_band, (float)long_band, list_a, list_b, list_l, counts, flags);
     return hipGetLastError();
 }
 
