@@ -30,6 +30,21 @@ BundleParams params_of(const SiriusHipRayBundle& b) {
 
 }  // namespace
 
+// The bundle pass over a prepared batch: in squares of the image, near-critical rays first.
+static int trace_bundles(Handle& H, Batch& B, int emission, int n_cam, const BundleOut& bo) {
+    int rc = SIRIUS_HIP_OK;
+    uint32_t* counts = (uint32_t*)H.scratch("b_work", 16, &rc);
+    if (rc) return rc;
+    hipError_t e = launch_fill(counts, 4, 0u, H.stream);
+    if (e != hipSuccess) return H.hip_fail(e, "fill");
+    RayOrder order;
+    if ((rc = longest_first(H, B, 32, counts, bo.flags, order))) return rc;
+    e = launch_trace_bundle(B.kernels, emission, B.cams_dev, n_cam, B.tp, params_of(H.bundle), bo, order.main, order.first,
+                            order.first_count, H.stream);
+    if (e != hipSuccess) return H.hip_fail(e, "bundle trace");
+    return SIRIUS_HIP_OK;
+}
+
 // The bundle pass over a prepared batch into library scratch (launch's beams).
 int bundle_for_launch(Handle& H, Batch& B, int emission, int n_cam, BundleOut& bo) {
     int rc = SIRIUS_HIP_OK;
@@ -39,9 +54,7 @@ int bundle_for_launch(Handle& H, Batch& B, int emission, int n_cam, BundleOut& b
     if (!rc) bo.jac = (float*)H.scratch("b_jac", 16 * (size_t)B.n, &rc);
     if (!rc) bo.beam = (float*)H.scratch("b_beam", 12 * (size_t)B.n, &rc);
     if (rc) return rc;
-    hipError_t e = launch_trace_bundle(B.kernels, emission, B.cams_dev, n_cam, B.tp, params_of(H.bundle), bo, H.stream);
-    if (e != hipSuccess) return H.hip_fail(e, "bundle trace");
-    return SIRIUS_HIP_OK;
+    return trace_bundles(H, B, emission, n_cam, bo);
 }
 
 }  // namespace sirius
@@ -104,9 +117,8 @@ int sirius_hip_trace_bundle(SiriusHipHandle hh, const SiriusHipCamera* cams, int
         if (!rc) bo.beam = (float*)get("b_beam", out->beam, 12 * (size_t)n);
         if (rc) return rc;
         const int emission = opts->emission == SIRIUS_EMISSION_THIN_DISK ? SIRIUS_EMISSION_THIN_DISK : 0;
-        hipError_t e = launch_trace_bundle(B.kernels, emission, B.cams_dev, n_cam, B.tp, params_of(H->bundle), bo,
-                                           H->stream);
-        if (e != hipSuccess) return H->hip_fail(e, "bundle trace");
+        if ((rc = trace_bundles(*H, B, emission, n_cam, bo))) return rc;
+        hipError_t e = hipSuccess;
         if (!out->on_device) {
             struct { void* dst; const void* src; size_t bytes; } c[] = {
                 {out->cls, bo.cls, (size_t)n}, {out->flags, bo.flags, (size_t)n},

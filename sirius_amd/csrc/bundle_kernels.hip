@@ -99,16 +99,23 @@ SIRIUS_HD __forceinline__ void ellipse_of(const double m[2][2], double size, flo
 // 212-364 bytes per lane (the state, two tangents and their derivatives beside seven stages).
 // A wave's rays that end on the disk are landed together, and the escape angles differenced
 // together, after its last ray has ended. Bound by FP64 issue and by the longest ray's steps: 641x361
-// Kerr rays at the FP32 path's tolerances take 1.83 ms without Lambda, 2.15 with its terms (spill-free
-// at one wave per SIMD); one lane per ray took 4.74 (5.89 with IEEE roots and divisions).
+// Kerr rays at the FP32 path's tolerances take 1.29 ms in squares with the near-critical rays first (1.83 in rows
+// and raster order, 2.15 also with the Lambda terms; spill-free at one wave per SIMD); one lane per
+// ray took 4.74 (5.89 also with IEEE roots and divisions).
 template <int FAM, int EMIT>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void k_trace_bundle(
-    const CamConst* __restrict__ cams, int n_cam, TraceParams tp, BundleParams bp, BundleOut bo) {
-    const int64_t id = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 1;
+    const CamConst* __restrict__ cams, int n_cam, TraceParams tp, BundleParams bp, BundleOut bo,
+    const int32_t* __restrict__ order, const int32_t* __restrict__ first, const uint32_t* __restrict__ first_count) {
+    int64_t id = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 1;
     const int axis = threadIdx.x & 1;
     if (id >= bo.n) return;
+    if (order) {
+        const int64_t nf = *first_count;
+        id = id < nf ? first[id] : order[id - nf];
+    }
     const CamConst& c = cams[find_cam(cams, n_cam, id)];
-    const int64_t pix = id - c.offset;
+    const int64_t pix = order ? id - c.offset : tile_pixel(c.width, c.height, TILE_SQUARE, id - c.offset);
+    id = c.offset + pix;
     const double u0 = (double)(pix % c.width) + 0.5, v0 = (double)(pix / c.width) + 0.5;
     using D = Dual<double, 1>;
     const Spacetime<double> s = make_spacetime<double>(c);
@@ -257,22 +264,23 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
 }
 
 hipError_t launch_trace_bundle(int family, int emission, const CamConst* cams, int n_cam, const TraceParams& tp,
-                               const BundleParams& bp, const BundleOut& bo, hipStream_t st) {
+                               const BundleParams& bp, const BundleOut& bo, const int32_t* order, const int32_t* first,
+                               const uint32_t* first_count, hipStream_t st) {
     if (bo.n <= 0) return hipSuccess;
     const dim3 grid((unsigned)((2 * bo.n + 63) / 64)), block(64);  // two lanes per ray
     const bool disk = emission == SIRIUS_EMISSION_THIN_DISK;
     if (family == 1)
-        hipLaunchKernelGGL((k_trace_bundle<1, 0>), grid, block, 0, st, cams, n_cam, tp, bp, bo);
+        hipLaunchKernelGGL((k_trace_bundle<1, 0>), grid, block, 0, st, cams, n_cam, tp, bp, bo, order, first, first_count);
     else if (family == 2)
-        hipLaunchKernelGGL((k_trace_bundle<2, 0>), grid, block, 0, st, cams, n_cam, tp, bp, bo);
+        hipLaunchKernelGGL((k_trace_bundle<2, 0>), grid, block, 0, st, cams, n_cam, tp, bp, bo, order, first, first_count);
     else if (family == FAM_KS_FLAT && disk)
-        hipLaunchKernelGGL((k_trace_bundle<FAM_KS_FLAT, SIRIUS_EMISSION_THIN_DISK>), grid, block, 0, st, cams, n_cam, tp, bp, bo);
+        hipLaunchKernelGGL((k_trace_bundle<FAM_KS_FLAT, SIRIUS_EMISSION_THIN_DISK>), grid, block, 0, st, cams, n_cam, tp, bp, bo, order, first, first_count);
     else if (family == FAM_KS_FLAT)
-        hipLaunchKernelGGL((k_trace_bundle<FAM_KS_FLAT, 0>), grid, block, 0, st, cams, n_cam, tp, bp, bo);
+        hipLaunchKernelGGL((k_trace_bundle<FAM_KS_FLAT, 0>), grid, block, 0, st, cams, n_cam, tp, bp, bo, order, first, first_count);
     else if (disk)
-        hipLaunchKernelGGL((k_trace_bundle<0, SIRIUS_EMISSION_THIN_DISK>), grid, block, 0, st, cams, n_cam, tp, bp, bo);
+        hipLaunchKernelGGL((k_trace_bundle<0, SIRIUS_EMISSION_THIN_DISK>), grid, block, 0, st, cams, n_cam, tp, bp, bo, order, first, first_count);
     else
-        hipLaunchKernelGGL((k_trace_bundle<0, 0>), grid, block, 0, st, cams, n_cam, tp, bp, bo);
+        hipLaunchKernelGGL((k_trace_bundle<0, 0>), grid, block, 0, st, cams, n_cam, tp, bp, bo, order, first, first_count);
     return hipGetLastError();
 }
 

@@ -26,6 +26,7 @@ struct BundleOut {
 };
 
 hipError_t launch_trace_bundle(int family, int emission, const CamConst* cams, int n_cam, const TraceParams& tp,
-                               const BundleParams& bp, const BundleOut& bo, hipStream_t st);
+                               const BundleParams& bp, const BundleOut& bo, const int32_t* order, const int32_t* first,
+                               const uint32_t* first_count, hipStream_t st);
 
 }  // namespace sirius

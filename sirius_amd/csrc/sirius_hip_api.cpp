@@ -597,6 +597,32 @@ double flops_per_symplectic_step(int family, int order) {
     return (order >= 4 ? 3.0 : 1.0) * (4.0 * rhs + 56.0 + 72.0);
 }
 
+// A whole Kerr-Schild batch of more waves than the chip has SIMDs: lists that take the rays near the
+// critical curve first, as the FP32 path does. They are the longest (1061 steps of a mean of 59 on the
+// FP64 1283x721 frame), and started in the middle of it they run on alone (tracer 4.57 ms, 3.38 with
+// them first). Smaller batches, batches that find no memory for the lists, and no-allocation
+// scratch, whose limit stays, go without. counts: three cleared words.
+int longest_first(Handle& H, Batch& B, int rays_per_wave, uint32_t* counts, uint8_t* flags, RayOrder& r) {
+    r = RayOrder{};
+    if (B.family != SIRIUS_METRIC_KERR_SCHILD || H.arena || B.n <= 4 * (int64_t)rays_per_wave * H.cu_count) return SIRIUS_HIP_OK;
+    int none = 0;
+    int32_t* la = (int32_t*)H.scratch("gate_a", 4 * (size_t)B.n, &none);
+    int32_t* ll = none ? nullptr : (int32_t*)H.scratch("gate_l", 4 * (size_t)B.n, &none);
+    float* tabs = none ? nullptr : upload_critical_tables(H, B, &none);
+    if (none) {
+        (void)hipGetLastError();  // the failed allocation's
+        return SIRIUS_HIP_OK;
+    }
+    hipError_t e = launch_gate(B.cams_dev, (int)B.cc.size(), tabs, TILE_SQUARE, B.n, 0.0, 0.0, SIRIUS_LONG_BAND, la, la, ll,
+                               counts, flags, H.stream);
+    if (e != hipSuccess) return H.hip_fail(e, "gate launch");
+    r.main = la;
+    r.main_count = counts;
+    r.first = ll;
+    r.first_count = counts + 2;
+    return SIRIUS_HIP_OK;
+}
+
 // Idle lanes at which a wave of a persistent queue refills: the caller's choice, or a quarter wave
 // where neighbours in the queue end apart (rows, lists of picked rays) and the whole wave where they
 // end together (squares: FP32 warp bubble 0.75 ms at 16, 0.66 at 64; volumetric 4.23 and 3.97).
@@ -638,26 +664,14 @@ int run_trace(Handle& H, Batch& B, const SiriusHipTraceOpts& o, DevOut& dout, co
         TraceParams tp = B.tp;
         tp.escalate = 0;
         const bool picked = list_dev != nullptr;
-        // A whole FP64 Kerr-Schild batch of more waves than the chip has SIMDs takes the rays near
-        // the critical curve first, as the FP32 path does: the longest run 1061 steps of a mean of 59
-        // on the 1283x721 frame, and started in the middle of it they run on alone (tracer 4.57 ms,
-        // 3.38 with them first). Batches that find no memory for the lists (and no-allocation
-        // scratch, whose limit stays) go without.
-        if (fp64 && !picked && B.family == SIRIUS_METRIC_KERR_SCHILD && !H.arena && B.n > 256 * (int64_t)H.cu_count) {
-            int none = 0;
-            int32_t* la = (int32_t*)H.scratch("gate_a", 4 * (size_t)B.n, &none);
-            int32_t* ll = none ? nullptr : (int32_t*)H.scratch("gate_l", 4 * (size_t)B.n, &none);
-            float* tabs = none ? nullptr : upload_critical_tables(H, B, &none);
-            if (none) {
-                (void)hipGetLastError();  // the failed allocation's
-            } else {
-                if ((e = launch_gate(B.cams_dev, (int)B.cc.size(), tabs, B.tp.tile_lw, B.n, 0.0, 0.0, SIRIUS_LONG_BAND, la,
-                                     la, ll, work + 16, dout.flags, H.stream)) != hipSuccess)
-                    return H.hip_fail(e, "gate launch");
-                list_dev = la;
-                list_count_dev = work + 16;
-                tp.first_list = ll;
-                tp.first_count = work + 18;
+        if (fp64 && !picked) {
+            RayOrder order;
+            if ((rc = longest_first(H, B, 64, work + 16, dout.flags, order))) return rc;
+            if (order.main) {
+                list_dev = order.main;
+                list_count_dev = order.main_count;
+                tp.first_list = order.first;
+                tp.first_count = order.first_count;
             }
         }
         int grid = (int)std::max<int64_t>(1, (n_work + block - 1) / block), refill = 64;

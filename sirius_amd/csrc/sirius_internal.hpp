@@ -149,6 +149,15 @@ int run_trace(Handle& H, Batch& B, const SiriusHipTraceOpts& o, DevOut& dout, co
 double flops_per_step(int family);
 
 float* upload_critical_tables(Handle& H, Batch& B, int* rc);
+// Order of a batch's rays: those of `first`, then those of `main`; null: the batch in tile order.
+struct RayOrder {
+    const int32_t* main = nullptr;
+    const uint32_t* main_count = nullptr;
+    const int32_t* first = nullptr;
+    const uint32_t* first_count = nullptr;
+};
+int longest_first(Handle& H, Batch& B, int rays_per_wave, uint32_t* counts, uint8_t* flags, RayOrder& r);
+hipError_t launch_fill(uint32_t* p, int n, uint32_t v, hipStream_t st);
 
 // surrogate (mlp_kernels.hip / surrogate.cpp)
 void mlp_release(Handle& H);

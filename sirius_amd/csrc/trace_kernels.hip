@@ -721,11 +721,10 @@ __device__ __forceinline__ void persistent_body(const CamConst* __restrict__ cam
 // reciprocals of third order, no Lambda terms where no camera has any, the radius taken from the
 // step's last right-hand side, one reciprocal for the error norm, events located by Newton iteration
 // and landings deferred to the refill (land, above), the thin-disk tracer runs the 1283x721 Kerr
-// frame in 3.0 ms (4.57 in rows and raster order, 5.62 with the Lambda terms and two Newton steps per
-// root; 8.99 with IEEE roots
-// and divisions, 52 halvings per event and each ray landed as it ended), the warp tracer its
-// 1024x1024 frame's wall crossers in 0.87 ms (1.65), the wormhole tracer its frame's near-throat
-// rays in 0.38 ms (0.72).
+// frame in 3.0 ms (4.57 in rows and raster order; 5.62 also with the Lambda terms and two Newton steps
+// per root; 8.99 also with IEEE roots and divisions, 52 halvings per event and each ray landed as it
+// ended), the warp tracer its 1024x1024 frame's wall crossers in 0.82 ms (1.65), the wormhole tracer
+// its frame's near-throat rays in 0.38 ms (0.72).
 constexpr int fp64_min_waves(int fam, bool multi) { return fam == 2 && !multi ? 2 : 1; }
 // The persistent tracers start on a 4 KiB boundary of the code object. Their loops are about
 // 19 KiB of instructions, and where the linker happened to place them changed their speed: the

@@ -48,3 +48,18 @@ def test_lists_change_no_ray(acc, emission):
     last, _ = acc.trace_batch([tiny, other], [m], o)
     for k in FIELDS:
         assert np.array_equal(getattr(large, k)[..., n:], getattr(last, k)[..., 1:]), k
+
+
+@pytest.mark.gpu
+def test_lists_change_no_bundle(acc):
+    w, h = 181, 173  # 31,313 bundles: one camera is below the line of 32,768, two are above it
+    m = abi.metric_ks(1.0, 0.7)
+    cams = [abi.camera(40.0, 70.0, 40.0, w, h, disk=(0.0, 20.0), phi_deg=p) for p in (10.0, 75.0)]
+    o = O.default_opts(abi.PRECISION_FP64)
+    o.rtol, o.atol = 1e-6, 1e-8
+    print(f"[case] bundle lists {w}x{h}", flush=True)
+    both, n = acc.trace_bundle(cams, [m], o), w * h
+    for i, cam in enumerate(cams):
+        one = acc.trace_bundle([cam], [m], o)
+        for k in ("cls", "flags", "jac", "beam"):
+            assert np.array_equal(both[k][..., i * n:(i + 1) * n], one[k]), (k, i)
