@@ -118,17 +118,9 @@ int sirius_hip_trace_bundle(SiriusHipHandle hh, const SiriusHipCamera* cams, int
         if (rc) return rc;
         const int emission = opts->emission == SIRIUS_EMISSION_THIN_DISK ? SIRIUS_EMISSION_THIN_DISK : 0;
         if ((rc = trace_bundles(*H, B, emission, n_cam, bo))) return rc;
-        hipError_t e = hipSuccess;
-        if (!out->on_device) {
-            struct { void* dst; const void* src; size_t bytes; } c[] = {
-                {out->cls, bo.cls, (size_t)n}, {out->flags, bo.flags, (size_t)n},
-                {out->jac, bo.jac, 16 * (size_t)n}, {out->beam, bo.beam, 12 * (size_t)n}};
-            for (auto& x : c)
-                if (x.dst && (e = hipMemcpyAsync(x.dst, x.src, x.bytes, hipMemcpyDeviceToHost, H->stream)) != hipSuccess)
-                    return H->hip_fail(e, "bundle results copy");
-        }
-        if ((e = hipStreamSynchronize(H->stream)) != hipSuccess) return H->hip_fail(e, "bundle trace");
-        return SIRIUS_HIP_OK;
+        const HostCopy c[] = {{out->cls, bo.cls, (size_t)n}, {out->flags, bo.flags, (size_t)n},
+                              {out->jac, bo.jac, 16 * (size_t)n}, {out->beam, bo.beam, 12 * (size_t)n}};
+        return copy_to_host(*H, c, out->on_device ? 0 : 4, "bundle results copy");
     GUARD_END(H)
 }
 

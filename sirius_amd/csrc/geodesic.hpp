@@ -75,6 +75,13 @@ struct TraceParams {
     int tile_lw;  // order in which whole batches are taken (tile_pixel)
 };
 
+// Arrays that one kernel gathers into a block (k_gather): sources, 16-byte aligned offsets, bytes.
+constexpr int HOST_COPIES = 16;
+struct GatherArgs {
+    const void* src[HOST_COPIES];
+    uint32_t off[HOST_COPIES], bytes[HOST_COPIES];
+};
+
 // Null-drift histogram of the statistics pass: log10 bins of 1/16 decade over [1e-20, 1).
 constexpr int SIRIUS_DRIFT_BINS = 320;
 

@@ -267,6 +267,9 @@ void Handle::release() {
     if (pinned) (void)hipHostFree(pinned);
     pinned = nullptr;
     pinned_bytes = 0;
+    if (stage) (void)hipHostFree(stage);
+    stage = nullptr;
+    stage_refused = false;
     image.clear();
     image.shrink_to_fit();
     mlp_release(*this);
@@ -559,25 +562,64 @@ static int bind_audit_outputs(Handle& H, int64_t n, int n_bins, DevOut& o) {
     return rc;
 }
 
+int copy_to_host(Handle& H, const HostCopy* c, int n, const char* what) {
+    GatherArgs g;
+    int m = 0;
+    size_t used = 0;
+    bool fits = !H.arena && n <= HOST_COPIES;  // no-allocation mode owns no pinned memory
+    for (int i = 0; i < n && fits; ++i) {
+        if (!c[i].dst || !c[i].src || !c[i].bytes) continue;
+        fits = c[i].bytes <= STAGE_BYTES - used && (uintptr_t)c[i].src % 16 == 0;
+        if (!fits) break;
+        g.src[m] = c[i].src;
+        g.off[m] = (uint32_t)used;
+        g.bytes[m++] = (uint32_t)c[i].bytes;
+        used = std::min((used + c[i].bytes + 15) & ~(size_t)15, STAGE_BYTES);
+    }
+    hipError_t e;
+    if (fits && m && !H.stage && !H.stage_refused) {
+        if (hipHostMalloc((void**)&H.stage, STAGE_BYTES, hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();
+            H.stage = nullptr;
+            H.stage_refused = true;
+        }
+    }
+    const bool staged = fits && m && H.stage;
+    if (staged) {
+        if ((e = launch_gather(g, m, H.stage, H.stream)) != hipSuccess) return H.hip_fail(e, what);
+    } else {
+        for (int i = 0; i < n; ++i)
+            if (c[i].dst && c[i].src && c[i].bytes &&
+                (e = hipMemcpyAsync(c[i].dst, c[i].src, c[i].bytes, hipMemcpyDeviceToHost, H.stream)) != hipSuccess)
+                return H.hip_fail(e, what);
+    }
+    if ((e = hipStreamSynchronize(H.stream)) != hipSuccess) return H.hip_fail(e, "synchronize");
+    if (staged)
+        for (int i = 0, k = 0; i < n; ++i)
+            if (c[i].dst && c[i].src && c[i].bytes) std::memcpy(c[i].dst, H.stage + g.off[k++], c[i].bytes);
+    return SIRIUS_HIP_OK;
+}
+
+// A batch's arrays and where the caller wants them in host memory.
+constexpr int OUTPUTS = 11;
+static void output_copies(const SiriusHipRayOutput* out, const DevOut& o, int n_bins, HostCopy* c) {
+    const size_t n = (size_t)o.n_rays;
+    const HostCopy all[OUTPUTS] = {
+        {out->cls, o.cls, n},           {out->flags, o.flags, n},
+        {out->theta, o.theta, 4 * n},   {out->phi, o.phi, 4 * n},
+        {out->lambda, o.lam, 4 * n},    {out->disk_r, o.disk_r, 4 * n},
+        {out->redshift, o.redshift, 4 * n}, {out->null_drift, o.null_drift, 4 * n},
+        {out->steps, o.steps, 4 * n},   {out->intensity, o.intensity, 4 * n * n_bins},
+        {out->state, o.state, 64 * n},
+    };
+    std::copy(all, all + OUTPUTS, c);
+}
+
 int copy_outputs_to_host(Handle& H, const SiriusHipRayOutput* out, const DevOut& o, int n_bins) {
     if (!out || out->on_device) return SIRIUS_HIP_OK;
-    int64_t n = o.n_rays;
-    struct { void* dst; const void* src; size_t bytes; } c[] = {
-        {out->cls, o.cls, (size_t)n},           {out->flags, o.flags, (size_t)n},
-        {out->theta, o.theta, 4 * (size_t)n},   {out->phi, o.phi, 4 * (size_t)n},
-        {out->lambda, o.lam, 4 * (size_t)n},    {out->disk_r, o.disk_r, 4 * (size_t)n},
-        {out->redshift, o.redshift, 4 * (size_t)n}, {out->null_drift, o.null_drift, 4 * (size_t)n},
-        {out->steps, o.steps, 4 * (size_t)n},   {out->intensity, o.intensity, 4 * (size_t)n * n_bins},
-        {out->state, o.state, 64 * (size_t)n},
-    };
-    for (auto& x : c) {
-        if (!x.dst || !x.src || !x.bytes) continue;
-        hipError_t e = hipMemcpyAsync(x.dst, x.src, x.bytes, hipMemcpyDeviceToHost, H.stream);
-        if (e != hipSuccess) return H.hip_fail(e, "copy results to host");
-    }
-    hipError_t e = hipStreamSynchronize(H.stream);
-    if (e != hipSuccess) return H.hip_fail(e, "synchronize");
-    return SIRIUS_HIP_OK;
+    HostCopy c[OUTPUTS];
+    output_copies(out, o, n_bins, c);
+    return copy_to_host(H, c, OUTPUTS, "copy results to host");
 }
 
 // Per-family algorithmic flops of one DP45 attempt (6 RHS + 426, fixed constants).
@@ -632,7 +674,8 @@ static int default_refill(const SiriusHipTraceOpts& o, const Batch& B, bool pick
 }
 
 int run_trace(Handle& H, Batch& B, const SiriusHipTraceOpts& o, DevOut& dout, const int32_t* list_dev,
-              const uint32_t* list_count_dev, int64_t list_cap, SiriusHipStats* stats, bool time_it) {
+              const uint32_t* list_count_dev, int64_t list_cap, SiriusHipStats* stats, bool time_it,
+              const SiriusHipRayOutput* host_out, bool* delivered) {
     hipError_t e;
     int rc = SIRIUS_HIP_OK;
     bool fp64 = o.precision == SIRIUS_PRECISION_FP64;
@@ -645,10 +688,17 @@ int run_trace(Handle& H, Batch& B, const SiriusHipTraceOpts& o, DevOut& dout, co
     // work[12] band queue head, work[13] unused, work[14..15] band attempts (u64),
     // work[16..18] gate counts (A, B, L), work[19] surrogate candidates, work[20] candidates the
     // calibrated error gate refused
-    uint32_t* work = (uint32_t*)H.scratch("work", 128, &rc);
+    // work[32..47] statistics sums (u64), work[48..] the null-drift histogram
+    struct {
+        uint32_t wk[32];
+        unsigned long long h[8];
+        uint32_t hh[SIRIUS_DRIFT_BINS];
+    } host;
+    static_assert(sizeof(host) == 4 * (48 + SIRIUS_DRIFT_BINS), "the device's layout");
+    uint32_t* work = (uint32_t*)H.scratch("work", sizeof(host), &rc);
     if (rc) return rc;
     unsigned int* audit_acc = nullptr;  // surrogate audit: largest direction error, class mismatches
-    if ((e = launch_fill(work, 32, 0u, H.stream)) != hipSuccess) return H.hip_fail(e, "fill");
+    if ((e = launch_fill(work, (int)(sizeof(host) / 4), 0u, H.stream)) != hipSuccess) return H.hip_fail(e, "fill");
     H.last_band = false;
     H.last_audit = false;  // set again below only when this call audits surrogate answers
     if (time_it) (void)hipEventRecord(H.ev0, H.stream);
@@ -868,25 +918,21 @@ int run_trace(Handle& H, Batch& B, const SiriusHipTraceOpts& o, DevOut& dout, co
         if (time_it) (void)hipEventRecord(H.ev_p1, H.stream);
     }
     if (stats) {
-        unsigned long long* acc = (unsigned long long*)H.scratch("stat_acc", 8 * 8, &rc);
-        if (rc) return rc;
-        uint32_t* hist = (uint32_t*)H.scratch("stat_hist", 4 * SIRIUS_DRIFT_BINS, &rc);
-        if (rc) return rc;
-        if ((e = launch_fill((uint32_t*)acc, 16, 0u, H.stream)) != hipSuccess) return H.hip_fail(e, "fill");
-        if ((e = launch_fill(hist, SIRIUS_DRIFT_BINS, 0u, H.stream)) != hipSuccess) return H.hip_fail(e, "fill");
-        if ((e = launch_reduce_stats(dout, B.n, acc, hist, H.stream)) != hipSuccess) return H.hip_fail(e, "reduce");
-        unsigned long long h[8] = {0};
-        if ((e = hipMemcpyAsync(h, acc, sizeof(h), hipMemcpyDeviceToHost, H.stream)) != hipSuccess)
-            return H.hip_fail(e, "stats copy");
-        uint32_t hh[SIRIUS_DRIFT_BINS];
-        if ((e = hipMemcpyAsync(hh, hist, sizeof(hh), hipMemcpyDeviceToHost, H.stream)) != hipSuccess)
-            return H.hip_fail(e, "stats copy");
-        uint32_t wk[32] = {0};
-        if (persistent) {
-            if ((e = hipMemcpyAsync(wk, work, sizeof(wk), hipMemcpyDeviceToHost, H.stream)) != hipSuccess)
-                return H.hip_fail(e, "stats copy");
+        if ((e = launch_reduce_stats(dout, B.n, (unsigned long long*)(work + 32), work + 48, H.stream)) != hipSuccess)
+            return H.hip_fail(e, "reduce");
+        // small results for the host travel with the statistics
+        HostCopy c[1 + OUTPUTS] = {{&host, work, sizeof(host)}};
+        int m = 1;
+        if (host_out && !host_out->on_device && !H.arena) {
+            output_copies(host_out, dout, o.n_bins, c + 1);
+            size_t all = 0;
+            for (const HostCopy& x : c) all += x.dst ? x.bytes + 16 : 0;
+            if (all <= STAGE_BYTES) m = 1 + OUTPUTS;
         }
-        if ((e = hipStreamSynchronize(H.stream)) != hipSuccess) return H.hip_fail(e, "synchronize");
+        if ((rc = copy_to_host(H, c, m, "results and statistics copy"))) return rc;
+        if (m > 1) *delivered = true;
+        const unsigned long long* h = host.h;
+        const uint32_t *hh = host.hh, *wk = host.wk;
         // h: attempts, rejected, landings, drift_max bits, escalated, surrogate, audited, esc attempts
         stats->rays += (uint64_t)B.n;
         stats->steps_accepted += h[0] - h[1];
@@ -1184,7 +1230,8 @@ int sirius_hip_trace_batch(SiriusHipHandle hh, const SiriusHipCamera* cams, int 
     H->last_bins = opts->n_bins;
     if (stats) std::memset(stats, 0, sizeof(*stats));
     (void)hipEventRecord(H->ev2, H->stream);
-    rc = run_trace(*H, B, *opts, dout, nullptr, nullptr, 0, stats, true);
+    bool delivered = false;
+    rc = run_trace(*H, B, *opts, dout, nullptr, nullptr, 0, stats, true, out, &delivered);
     if (rc) return rc;
     (void)hipEventRecord(H->ev3, H->stream);
     hipError_t e = hipEventSynchronize(H->ev3);
@@ -1194,7 +1241,7 @@ int sirius_hip_trace_batch(SiriusHipHandle hh, const SiriusHipCamera* cams, int 
         (void)hipEventElapsedTime(&ms, H->ev2, H->ev3);
         stats->total_ms = ms;
     }
-    return copy_outputs_to_host(*H, out, dout, opts->n_bins);
+    return delivered ? SIRIUS_HIP_OK : copy_outputs_to_host(*H, out, dout, opts->n_bins);
     GUARD_END(H)
 }
 

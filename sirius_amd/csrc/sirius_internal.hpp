@@ -105,6 +105,8 @@ struct Handle {
     std::vector<unsigned char> image;
     unsigned char* pinned = nullptr;
     size_t pinned_bytes = 0;
+    unsigned char* stage = nullptr;  // pinned staging of small results (copy_to_host), STAGE_BYTES
+    bool stage_refused = false;      // its allocation failed once: results are copied array by array
     // surrogate network
     MlpState* mlp = nullptr;
     // No-allocation mode (sirius_hip_trace_batch_noalloc): while `arena` is set, scratch()
@@ -143,9 +145,22 @@ bool make_cam_const(const SiriusHipCamera& cam, const SiriusHipMetric& m, int64_
 int prepare_batch(Handle& H, const SiriusHipCamera* cams, int n_cam, const SiriusHipMetric* metrics, int n_metric,
                   const SiriusHipTraceOpts& o, Batch& B);
 int bind_outputs(Handle& H, const SiriusHipRayOutput* out, int64_t n, int n_bins, DevOut& o, bool volumetric);
+// A device array on its way to host memory (skipped without destination, source or bytes).
+struct HostCopy {
+    void* dst;
+    const void* src;
+    size_t bytes;
+};
+// Results up to this size go to the host through one kernel and pinned staging.
+constexpr size_t STAGE_BYTES = (size_t)1 << 20;
+hipError_t launch_gather(const GatherArgs& a, int n, unsigned char* dst, hipStream_t st);
+// Copies and waits for the stream: n <= HOST_COPIES arrays.
+int copy_to_host(Handle& H, const HostCopy* c, int n, const char* what);
 int copy_outputs_to_host(Handle& H, const SiriusHipRayOutput* out, const DevOut& o, int n_bins);
+// host_out: results that go to the host with the statistics if they are small; *delivered says so.
 int run_trace(Handle& H, Batch& B, const SiriusHipTraceOpts& o, DevOut& dout, const int32_t* list_dev,
-              const uint32_t* list_count_dev, int64_t list_cap, SiriusHipStats* stats, bool time_it);
+              const uint32_t* list_count_dev, int64_t list_cap, SiriusHipStats* stats, bool time_it,
+              const SiriusHipRayOutput* host_out = nullptr, bool* delivered = nullptr);
 double flops_per_step(int family);
 
 float* upload_critical_tables(Handle& H, Batch& B, int* rc);

@@ -102,6 +102,28 @@ hipError_t launch_critical_distance(const CamConst* cams, int n_cam, const float
     return hipGetLastError();
 }
 
+// Arrays into one block of pinned host memory, each at its 16-byte aligned offset: small results reach
+// the host with one launch and one wait. A copy of each array to pageable memory costs about 40 us
+// whatever its size (host work and a wait per copy): a 96x54 frame's nine arrays and three statistics
+// copies took 0.40 ms of its 0.88 ms call, this kernel takes 0.02.
+__global__ __launch_bounds__(256) void k_gather(GatherArgs a, unsigned char* __restrict__ dst) {
+    const int k = blockIdx.y;
+    const unsigned char* src = (const unsigned char*)a.src[k];
+    unsigned char* d = dst + a.off[k];
+    const uint32_t words = a.bytes[k] / 16;
+    for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < words; i += gridDim.x * 256)
+        ((uint4*)d)[i] = ((const uint4*)src)[i];
+    if (blockIdx.x == 0 && threadIdx.x < a.bytes[k] % 16) d[16 * words + threadIdx.x] = src[16 * words + threadIdx.x];
+}
+
+hipError_t launch_gather(const GatherArgs& a, int n, unsigned char* dst, hipStream_t st) {
+    uint32_t most = 0;
+    for (int i = 0; i < n; ++i) most = a.bytes[i] > most ? a.bytes[i] : most;
+    const uint32_t blocks = (most / 16 + 255) / 256;
+    hipLaunchKernelGGL(k_gather, dim3(blocks < 1 ? 1 : (blocks > 64 ? 64 : blocks), (unsigned)n), dim3(256), 0, st, a, dst);
+    return hipGetLastError();
+}
+
 // Gate of the FP32 path: rays within `band` of the critical curve go to list B (traced in FP64
 // from the start, on a second stream), the others within `long_band` to list L (the FP32
 // tracer takes them first: they wind near the photon region and are the longest) and all
