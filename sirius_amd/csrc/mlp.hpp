@@ -76,7 +76,7 @@ struct MlpFusedArgs {
     const uint16_t* w0;    // [256][16] BF16, input columns padded to 16
     const uint16_t* w[3];  // layers 1..3, [256][256] BF16 in MFMA fragment order (k_pack_fused)
     const float* b[4];     // biases of layers 0..3, [256]
-    const uint16_t* w4h;   // head weights [32][256], BF16 high parts (rows 6..31 zero)
+    const uint16_t* w4h;   // head weights, 32 rows (6..31 zero) x 256, BF16 high parts (k_pack_fused)
     const uint16_t* w4l;   // and low parts
     const float* b4;       // head bias [6]
     float* y;              // n x 6 outputs
@@ -104,7 +104,7 @@ struct MlpState {
     float* grad = nullptr;
     int64_t step = 0;
     uint16_t* fw0 = nullptr;   // packed BF16 operands: W0 [256][16], hidden layers 1..3 (3 x 256 x 256,
-    uint16_t* fwh = nullptr;   // fragment order), their transposes, head W_hi / W_lo [32][256]
+    uint16_t* fwh = nullptr;   // fragment order), their transposes, head W_hi / W_lo, 32 x 256
     uint16_t* fwt = nullptr;
     uint16_t* fw4h = nullptr;
     uint16_t* fw4l = nullptr;

@@ -36,7 +36,7 @@ __device__ __forceinline__ float gelu_df(float z) {
 // column l % 32, rows 8 (r / 4) + 4 (l / 32) + r % 4).
 //  - Each layer is computed transposed, H'^T = W H^T: the weights are the A operand (16 bytes per
 //    lane, stored in fragment order so that a wave's load for one k-step is one contiguous
-//    kilobyte, streamed from L2 one k-step ahead of the MFMAs) and the tile's
+//    kilobyte, streamed from L2 MF_AHEAD k-steps ahead of the MFMAs) and the tile's
 //    activations the B operand, read from LDS ([128][264] BF16, row = sample; rows padded by 8
 //    values so that the 16-byte reads of eight consecutive lanes cover every bank once).
 //  - A lane's accumulators then hold, for one sample, runs of four consecutive neurons: the bias
@@ -46,14 +46,23 @@ __device__ __forceinline__ float gelu_df(float z) {
 //    accumulator registers).
 //  - The output head (256 -> 6) keeps FP32 precision with three BF16 products: the last hidden
 //    activation h = hi + lo and the head's weights W = W_hi + W_lo, each split into BF16 parts,
-//    and y = W_hi hi + W_lo hi + W_hi lo (the W_lo lo term is below FP32's resolution of y).
-//    hi, then lo, pass through the same LDS buffer.
+//    and y = W_hi hi + W_lo hi + W_hi lo (the W_lo lo term is below FP32's resolution of y). Each
+//    wave multiplies its own 64 neurons straight from its accumulators; the four partial sums of a
+//    sample meet in LDS.
+// Bound by the vector unit (a GELU is five FP32 instructions at 1.8 ns per SIMD, an exponential and a
+// reciprocal at 3.7; 512 per lane and tile with the rest are 10 us, 190 us for 600,001 rows) beside
+// 121 us of MFMAs, which the two blocks of a CU overlap in part: 324 us for 600,001 rows (379 with the
+// last layer's parts written to LDS and read back, high then low, by the head). Without the GELUs the
+// kernel takes 285 us, without the head's former round trip 220. Tried: the two halves of a tile in
+// alternate stages, GELU between the other half's MFMAs, with the weights read twice (352 us, 369 for
+// this kernel on the same run); 512 threads of 32 neurons (514, 429 then); 256-row tiles (495, 435).
 // ------------------------------------------------------------------------------------------
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef __bf16 v4bf __attribute__((ext_vector_type(4)));
 
 constexpr int MF_ROWS = 128;
 constexpr int MF_PITCH = 264;
+constexpr int MF_AHEAD = 2;  // k-steps that the weights are fetched ahead (divides 16)
 
 __device__ __forceinline__ v8bf ld8(const uint16_t* p) { return *(const v8bf*)p; }
 
@@ -78,7 +87,6 @@ __global__ __launch_bounds__(256, 2) void k_mlp_fused(MlpFusedArgs a) {
         }
         __syncthreads();
         v16f acc[2][4];
-        uint32_t lo_pk[2][4][8];  // low BF16 parts of the last hidden activation, four to two registers
         // the accumulators start at the layer's bias (row 8 q + 4 lh + e of tile mt is neuron
         // j0 + 32 mt + 8 q + 4 lh + e)
         auto init_bias = [&](int l) {
@@ -96,6 +104,21 @@ __global__ __launch_bounds__(256, 2) void k_mlp_fused(MlpFusedArgs a) {
                     }
                 }
         };
+        // ring of the weights' fragments, MF_AHEAD k-steps ahead of the MFMAs and on across layers (a
+        // layer's first fragments are on their way during the previous layer's epilogue). This
+        // lane's fragment of k-step ks, row tile mt of a layer: 1024 ks + 512 mt from its wf
+        v8bf wq[MF_AHEAD][2];
+        const uint32_t wf = 2 * (wave * 16384 + lane * 8);  // bytes
+        auto rsrc = [&](int l) { return __builtin_amdgcn_make_buffer_rsrc((void*)a.w[l], 0, 2 * MLP_H * MLP_H, 0x00027000); };
+        auto fragment = [&](__amdgpu_buffer_rsrc_t w, int ks, int mt) {
+            typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+            const v4u u = __builtin_amdgcn_raw_buffer_load_b128(w, wf + 1024 * mt, 2048 * ks, 0);
+            return __builtin_bit_cast(v8bf, u);
+        };
+#pragma unroll
+        for (int ks = 0; ks < MF_AHEAD; ++ks)
+#pragma unroll
+            for (int mt = 0; mt < 2; ++mt) wq[ks][mt] = fragment(rsrc(0), ks, mt);
         init_bias(0);
         {
             v8bf w[2];
@@ -109,106 +132,87 @@ __global__ __launch_bounds__(256, 2) void k_mlp_fused(MlpFusedArgs a) {
                     acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[mt], hv, acc[mt][nt], 0, 0, 0);
             }
         }
-        for (int l = 0; l < 4; ++l) {
-            if (l > 0) {
-                const uint16_t* Wl = a.w[l - 1];
-                init_bias(l);
-                // this lane's fragment of k-step ks, row tile mt: Wp + 1024 ks + 512 mt (one running
-                // pointer; the row-tile offset is an immediate)
-                const uint16_t* Wp = Wl + wave * 16384 + lane * 8;
-                v8bf w[2], wn[2];
+        // one hidden layer's products: its weights from Wl, the next one's first from Wn
+        auto products = [&](int l, __amdgpu_buffer_rsrc_t Wl, __amdgpu_buffer_rsrc_t Wn) {
+            init_bias(l);
 #pragma unroll
-                for (int mt = 0; mt < 2; ++mt) w[mt] = ld8(Wp + 512 * mt);
+            for (int ks = 0; ks < MLP_H / 16; ++ks) {
+                v8bf w[2];
 #pragma unroll
-                for (int ks = 0; ks < MLP_H / 16; ++ks) {
-                    const int k0 = ks * 16;
-                    if (ks + 1 < MLP_H / 16) {
-                        Wp += 1024;
+                for (int mt = 0; mt < 2; ++mt) w[mt] = wq[ks % MF_AHEAD][mt];
+                const int kn = ks + MF_AHEAD;
 #pragma unroll
-                        for (int mt = 0; mt < 2; ++mt) wn[mt] = ld8(Wp + 512 * mt);
-                    }
+                for (int mt = 0; mt < 2; ++mt)
+                    wq[ks % MF_AHEAD][mt] = kn < MLP_H / 16 ? fragment(Wl, kn, mt) : fragment(Wn, kn - MLP_H / 16, mt);
 #pragma unroll
-                    for (int nt = 0; nt < 4; ++nt) {
-                        const v8bf hv = ld8(&act[(nt * 32 + li) * MF_PITCH + k0 + 8 * lh]);
+                for (int nt = 0; nt < 4; ++nt) {
+                    const v8bf hv = ld8(&act[(nt * 32 + li) * MF_PITCH + ks * 16 + 8 * lh]);
 #pragma unroll
-                        for (int mt = 0; mt < 2; ++mt)
-                            acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[mt], hv, acc[mt][nt], 0, 0, 0);
-                    }
-                    if (ks + 1 < MLP_H / 16) {
-#pragma unroll
-                        for (int mt = 0; mt < 2; ++mt) w[mt] = wn[mt];
-                    }
+                    for (int mt = 0; mt < 2; ++mt)
+                        acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[mt], hv, acc[mt][nt], 0, 0, 0);
                 }
             }
+        };
+        // GELU on runs of four neurons; BF16 back into the sample's LDS row
+#pragma unroll 1
+        for (int l = 0; l < 3; ++l) {
+            if (l > 0) products(l, rsrc(l - 1), rsrc(l));
             __syncthreads();  // every wave has read this layer's input
-            // GELU on runs of four neurons; BF16 (the last layer: its high parts) back into the
-            // sample's LDS row, the last layer's low parts kept in registers
 #pragma unroll
             for (int mt = 0; mt < 2; ++mt)
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const int jb = j0 + mt * 32 + 8 * q + 4 * lh;
+                for (int q = 0; q < 4; ++q)
 #pragma unroll
                     for (int nt = 0; nt < 4; ++nt) {
-                        const float h0 = gelu_f(acc[mt][nt][4 * q + 0]), h1 = gelu_f(acc[mt][nt][4 * q + 1]);
-                        const float h2 = gelu_f(acc[mt][nt][4 * q + 2]), h3 = gelu_f(acc[mt][nt][4 * q + 3]);
-                        const v4bf hv = {(__bf16)h0, (__bf16)h1, (__bf16)h2, (__bf16)h3};
-                        *(v4bf*)&act[(nt * 32 + li) * MF_PITCH + jb] = hv;
-                        if (l == 3) {
-                            const v4bf lv = {(__bf16)(h0 - (float)hv[0]), (__bf16)(h1 - (float)hv[1]),
-                                             (__bf16)(h2 - (float)hv[2]), (__bf16)(h3 - (float)hv[3])};
-                            uint32_t u[2];
-                            __builtin_memcpy(u, &lv, 8);
-                            lo_pk[mt][nt][2 * q] = u[0];
-                            lo_pk[mt][nt][2 * q + 1] = u[1];
-                        }
+                        const v4bf hv = {(__bf16)gelu_f(acc[mt][nt][4 * q + 0]), (__bf16)gelu_f(acc[mt][nt][4 * q + 1]),
+                                         (__bf16)gelu_f(acc[mt][nt][4 * q + 2]), (__bf16)gelu_f(acc[mt][nt][4 * q + 3])};
+                        *(v4bf*)&act[(nt * 32 + li) * MF_PITCH + j0 + mt * 32 + 8 * q + 4 * lh] = hv;
                     }
-                }
             __syncthreads();
         }
-        // output head, samples 32 w .. 32 w + 31 of the tile: W_hi hi + W_lo hi, then W_hi lo. Rows
-        // 6..31 of the head's weights are zero: the lanes holding them all read row 6, so a head
-        // load fetches the six live rows and one more line.
-        const uint16_t* Hh = a.w4h + (li < SIRIUS_MLP_OUT ? li : SIRIUS_MLP_OUT) * MLP_H + 8 * lh;
-        const uint16_t* Hl = a.w4l + (li < SIRIUS_MLP_OUT ? li : SIRIUS_MLP_OUT) * MLP_H + 8 * lh;
-        v16f y;
+        products(3, rsrc(2), rsrc(2));
+        v8bf w4h[4], w4l[4];
 #pragma unroll
-        for (int r = 0; r < 16; ++r) y[r] = 0.f;
-#pragma unroll
-        for (int ks = 0; ks < MLP_H / 16; ++ks) {
-            const int k0 = ks * 16;
-            const v8bf hv = ld8(&act[(wave * 32 + li) * MF_PITCH + k0 + 8 * lh]);
-            y = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ld8(Hh + k0), hv, y, 0, 0, 0);
-            y = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ld8(Hl + k0), hv, y, 0, 0, 0);
+        for (int f = 0; f < 4; ++f) {
+            w4h[f] = ld8(a.w4h + ((wave * 4 + f) * 64 + lane) * 8);
+            w4l[f] = ld8(a.w4l + ((wave * 4 + f) * 64 + lane) * 8);
         }
-        __syncthreads();  // every wave has read the high parts
-#pragma unroll
-        for (int mt = 0; mt < 2; ++mt)
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int jb = j0 + mt * 32 + 8 * q + 4 * lh;
-#pragma unroll
-                for (int nt = 0; nt < 4; ++nt) {
-                    const uint32_t u[2] = {lo_pk[mt][nt][2 * q], lo_pk[mt][nt][2 * q + 1]};
-                    __builtin_memcpy(&act[(nt * 32 + li) * MF_PITCH + jb], u, 8);
-                }
-            }
         __syncthreads();
+        // The output head on this wave's 64 neurons, from the accumulators: a lane's runs q and q + 1 of a
+        // row tile are 8 neurons of one sample, the B operand of one MFMA whose k order the packed head
+        // weights share. y^T: rows 0..7 of the product, lane li's sample, outputs 4 lh + r.
+        float* part = (float*)act;  // [wave][sample][6]: every wave has read this layer's input
 #pragma unroll
-        for (int ks = 0; ks < MLP_H / 16; ++ks) {
-            const int k0 = ks * 16;
-            const v8bf hv = ld8(&act[(wave * 32 + li) * MF_PITCH + k0 + 8 * lh]);
-            y = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ld8(Hh + k0), hv, y, 0, 0, 0);
-        }
-        // y^T: this lane's sample is 32 w + li, its outputs are rows 4 lh + r (r < 4) of the first
-        // 8-row group
-        const int64_t gr = row0 + wave * 32 + li;
-        if (gr < n) {
+        for (int nt = 0; nt < 4; ++nt) {
+            v16f y;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int o = 4 * lh + r;
-                if (o < SIRIUS_MLP_OUT) a.y[gr * SIRIUS_MLP_OUT + o] = y[r] + a.b4[o];
+            for (int r = 0; r < 16; ++r) y[r] = 0.f;
+#pragma unroll
+            for (int f = 0; f < 4; ++f) {
+                const int mt = f >> 1, q = 2 * (f & 1);
+                v8bf hi, lo;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const float h = gelu_f(acc[mt][nt][4 * q + e]);
+                    hi[e] = (__bf16)h;
+                    lo[e] = (__bf16)(h - (float)hi[e]);
+                }
+                y = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w4h[f], hi, y, 0, 0, 0);
+                y = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w4l[f], hi, y, 0, 0, 0);
+                y = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w4h[f], lo, y, 0, 0, 0);
             }
+            float* p = part + (wave * MF_ROWS + nt * 32 + li) * SIRIUS_MLP_OUT + 4 * lh;
+            *(float2*)p = make_float2(y[0], y[1]);
+            if (lh == 0) *(float2*)(p + 2) = make_float2(y[2], y[3]);
+        }
+        __syncthreads();
+        const int64_t left = n - row0;
+        const int rows = left < MF_ROWS ? (int)left : MF_ROWS;
+        for (int e = t; e < rows * SIRIUS_MLP_OUT; e += 256) {
+            float v = a.b4[e % SIRIUS_MLP_OUT];
+#pragma unroll
+            for (int w = 0; w < 4; ++w) v += part[w * MF_ROWS * SIRIUS_MLP_OUT + e];
+            a.y[row0 * SIRIUS_MLP_OUT + e] = v;
         }
     }
 }
@@ -610,7 +614,7 @@ hipError_t launch_mlp_grad_sum(const MlpGradSumArgs& a, hipStream_t st) {
 // row 64 w + 32 mt + l % 32, columns 16 ks + 8 (l / 32) .. +7), so each wave's weight load is one
 // contiguous kilobyte; their transposes for the backward pass, the fragment of lane l for k-step ks,
 // column block w at ((w 16 + ks) 64 + l) 8 (W[16 ks + 8 (l / 32) .. +7][32 w + l % 32]); the head's
-// high and low BF16 parts row-major [32][256] (rows 6..31 zero).
+// high and low BF16 parts (rows 6..31 zero) in the k order of the fused kernel's accumulators.
 __global__ void k_pack_fused(const float* __restrict__ P, uint16_t* __restrict__ w0, uint16_t* __restrict__ wh,
                              uint16_t* __restrict__ wt, uint16_t* __restrict__ w4h, uint16_t* __restrict__ w4l, size_t off_w0, size_t off_w1,
                              size_t off_w2, size_t off_w3, size_t off_w4) {
@@ -629,7 +633,10 @@ __global__ void k_pack_fused(const float* __restrict__ P, uint16_t* __restrict__
         wt[e] = f2bf(P[off + (size_t)tj * MLP_H + tk]);
     }
     if (e < 32 * MLP_H) {
-        const int j = e / MLP_H, k = e % MLP_H;
+        // fragment (wave w, row tile mt, run pair): value i of lane l is W4[l % 32][64 w + 32 mt +
+        // 16 pair + 8 (i / 4) + 4 (l / 32) + i % 4]
+        const int i = e & 7, lane = (e >> 3) & 63, j = lane & 31;
+        const int k = 16 * (e >> 9) + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
         const float w = j < SIRIUS_MLP_OUT ? P[off_w4 + (size_t)j * MLP_H + k] : 0.f;
         const uint16_t hi = f2bf(w);
         w4h[e] = hi;
