@@ -99,7 +99,7 @@ SIRIUS_HD __forceinline__ void ellipse_of(const double m[2][2], double size, flo
 // 212-364 bytes per lane (the state, two tangents and their derivatives beside seven stages).
 // A wave's rays that end on the disk are landed together, and the escape angles differenced
 // together, after its last ray has ended. Bound by FP64 issue and by the longest ray's steps: 641x361
-// Kerr rays at the FP32 path's tolerances take 1.29 ms in squares with the near-critical rays first (1.83 in rows
+// Kerr rays at the FP32 path's tolerances take 1.18 ms in squares with the near-critical rays first (1.83 in rows
 // and raster order, 2.15 also with the Lambda terms; spill-free at one wave per SIMD); one lane per
 // ray took 4.74 (5.89 also with IEEE roots and divisions).
 template <int FAM, int EMIT>

@@ -721,7 +721,7 @@ __device__ __forceinline__ void persistent_body(const CamConst* __restrict__ cam
 // reciprocals of third order, no Lambda terms where no camera has any, the radius taken from the
 // step's last right-hand side, one reciprocal for the error norm, events located by Newton iteration
 // and landings deferred to the refill (land, above), the thin-disk tracer runs the 1283x721 Kerr
-// frame in 3.0 ms (4.57 in rows and raster order; 5.62 also with the Lambda terms and two Newton steps
+// frame in 2.9 ms (4.57 in rows and raster order; 5.62 also with the Lambda terms and two Newton steps
 // per root; 8.99 also with IEEE roots and divisions, 52 halvings per event and each ray landed as it
 // ended), the warp tracer its 1024x1024 frame's wall crossers in 0.82 ms (1.65), the wormhole tracer
 // its frame's near-throat rays in 0.38 ms (0.72).
@@ -920,8 +920,9 @@ __global__ void k_fill_u32(uint32_t* p, int n, uint32_t v) {
 // A(h/2) B(h/2) C(h) B(h/2) A(h/2), composed to 4th order with the Yoshida triple jump
 // (weights PHSI001A.h:43-47). Fixed step; disk crossing on the cubic Hermite interpolant.
 // Bound by the serial chain of right-hand sides of the longest ray (a 320x181 Kerr frame at
-// h = 0.02 has 905 waves for 1024 SIMDs): 28 ms with 9 evaluations per step, without Lambda
-// terms (36 ms with them), 63-65 ms with 12 and IEEE roots and divisions.
+// h = 0.02 has 905 waves for 1024 SIMDs): 24 ms with 9 evaluations and 946 instructions
+// per step (28 ms with 1206, 36 ms with the Lambda terms too; 63-65 ms with 12 evaluations and IEEE
+// roots and divisions).
 // ------------------------------------------------------------------------------------------
 // Flow A with H's derivatives D at (q, y). A changes neither q nor y, so the A that ends a substep
 // and the A that begins the next have the same D: it is evaluated once for both (9 evaluations per
@@ -938,13 +939,15 @@ SIRIUS_HD __forceinline__ void tao_b(const Spacetime<T>& s, T d, T q[4], const T
     for (int i = 0; i < 4; ++i) q[i] += d * D.k[i];
     for (int i = 0; i < 3; ++i) y[i + 1] += d * D.f[i];
 }
+// The rotation of (q - x, p - y) by an angle with cosine cw and sine sw, as the change of each copy: ch =
+// (cw - 1) / 2, sh = sw / 2.
 template <class T>
-SIRIUS_HD __forceinline__ void tao_c(T cw, T sw, T q[4], T p[4], T x[4], T y[4]) {
+SIRIUS_HD __forceinline__ void tao_c(T ch, T sh, T q[4], T p[4], T x[4], T y[4]) {
     for (int i = 0; i < 4; ++i) {
-        T sq = q[i] + x[i], sp = p[i] + y[i], dq = q[i] - x[i], dp = p[i] - y[i];
-        T ndq = cw * dq + sw * dp, ndp = -sw * dq + cw * dp;
-        q[i] = T(0.5) * (sq + ndq); p[i] = T(0.5) * (sp + ndp);
-        x[i] = T(0.5) * (sq - ndq); y[i] = T(0.5) * (sp - ndp);
+        const T dq = q[i] - x[i], dp = p[i] - y[i];
+        const T e = ch * dq + sh * dp, g = ch * dp - sh * dq;
+        q[i] += e; p[i] += g;
+        x[i] -= e; y[i] -= g;
     }
 }
 
@@ -962,9 +965,16 @@ __global__ __launch_bounds__(256) void k_symplectic_grid(const CamConst* __restr
     const T w = T(20);
     const T h = T(tp.sym_h);
     const T wts[3] = {T(1.3512071919596576), T(-1.7024143839193153), T(1.3512071919596576)};
-    T cw[3], sw[3];
-    for (int j = 0; j < 3; ++j) { cw[j] = cos(T(2) * w * wts[j] * h); sw[j] = sin(T(2) * w * wts[j] * h); }
-    T cw2 = cos(T(2) * w * h), sw2 = sin(T(2) * w * h);
+    const int subs = tp.sym_order >= 4 ? 3 : 1;
+    // per substep: half its length, and the rotation by 2 w times its length ((cos - 1) / 2 = -sin^2 / 2 of
+    // the half angle)
+    T hh[3], ch[3], sh[3];
+    for (int j = 0; j < 3; ++j) {
+        const T hj = subs == 3 ? wts[j] * h : h, sn = sin(w * hj);
+        hh[j] = T(0.5) * hj;
+        ch[j] = -sn * sn;
+        sh[j] = T(0.5) * sin(T(2) * w * hj);
+    }
     int cls = SIRIUS_RAY_MAX_STEPS;
     T rd = T(0), rprev = event_radius(s, q);
     uint32_t n = 0;
@@ -973,16 +983,16 @@ __global__ __launch_bounds__(256) void k_symplectic_grid(const CamConst* __restr
     while (n < (uint32_t)tp.max_steps) {
         T q0[4], p0[4];
         for (int i = 0; i < 4; ++i) { q0[i] = q[i]; p0[i] = p[i]; }
-        const int subs = tp.sym_order >= 4 ? 3 : 1;
-        for (int j = 0; j < subs; ++j) {
-            T hj = subs == 3 ? wts[j] * h : h;
-            T cj = subs == 3 ? cw[j] : cw2, sj = subs == 3 ? sw[j] : sw2;
-            tao_a<T>(DA, T(0.5) * hj, p, x);
-            tao_b<T, FAM>(s, T(0.5) * hj, q, p, x, y);
-            tao_c<T>(cj, sj, q, p, x, y);
-            tao_b<T, FAM>(s, T(0.5) * hj, q, p, x, y);
+        tao_a<T>(DA, hh[0], p, x);
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            if (j >= subs) break;
+            tao_b<T, FAM>(s, hh[j], q, p, x, y);
+            tao_c<T>(ch[j], sh[j], q, p, x, y);
+            tao_b<T, FAM>(s, hh[j], q, p, x, y);
             eval<T, FAM>(s, q, y, DA);
-            tao_a<T>(DA, T(0.5) * hj, p, x);
+            // with the next substep's first A flow, which has the same derivatives
+            tao_a<T>(DA, j + 1 < subs ? hh[j] + hh[j < 2 ? j + 1 : 2] : hh[j], p, x);
         }
         n++;
         R.lam += h;
