@@ -351,7 +351,9 @@ SIRIUS_HD __forceinline__ T warp_shape(const Spacetime<scalar_t<T>>& s, T rs, T&
     const T v = exp(-S(2) * s.wsig * (rs - s.wR));
     const T ev = s.wE * v;
     const T D = tfma(v, S(1) + s.wE + ev, T(1));
-    const T iD = T(1) / D;
+    T iD;
+    if constexpr (std::is_same_v<T, float>) iD = T(1) / D;
+    else iD = rcp_t(D);
     const T f = s.wN * v * iD;
     dfdr = -S(2) * s.wsig * f * (S(1) - ev * v) * iD;
     return f;
@@ -579,7 +581,8 @@ SIRIUS_HD __forceinline__ T rhs_mt(const Spacetime<scalar_t<T>>& s, const T x[4]
     T r2 = x[1] * x[1] + s.b02;
     k[0] = -p[0];
     k[1] = p[1];
-    k[2] = p[2] / r2;
+    if constexpr (std::is_same_v<T, float>) k[2] = p[2] / r2;
+    else k[2] = p[2] * rcp_t(r2);
     k[3] = p[3];
     dp[0] = x[1] * k[2] * k[2];
     dp[1] = T(0);
@@ -593,7 +596,13 @@ SIRIUS_HD __forceinline__ T rhs_warp(const Spacetime<scalar_t<T>>& s, const T x[
     using S = scalar_t<T>;
     T R2 = x[1] * x[1] + x[2] * x[2] + x[3] * x[3];
     R2 = R2 < T(1e-20) ? T(1e-20) : R2;
-    T rs = sqrt(R2);
+    T rs, irs;
+    if constexpr (std::is_same_v<T, float>) {
+        rs = sqrt(R2);
+    } else {
+        irs = rsqrt_t(R2);
+        rs = sqrt_from(R2, irs);
+    }
     T dfdr;
     T f = warp_shape(s, rs, dfdr);
     T vf = s.wv * f;
@@ -601,7 +610,9 @@ SIRIUS_HD __forceinline__ T rhs_warp(const Spacetime<scalar_t<T>>& s, const T x[
     k[1] = -vf * p[0] + (S(1) - vf * vf) * p[1];
     k[2] = p[2];
     k[3] = p[3];
-    T c = s.wv * dfdr / rs * (vf * k[0] * k[0] - k[0] * k[1]);
+    T c;
+    if constexpr (std::is_same_v<T, float>) c = s.wv * dfdr / rs * (vf * k[0] * k[0] - k[0] * k[1]);
+    else c = s.wv * dfdr * irs * (k[0] * (vf * k[0] - k[1]));
     dp[0] = c * x[1];
     dp[1] = c * x[2];
     dp[2] = c * x[3];
