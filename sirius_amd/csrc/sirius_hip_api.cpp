@@ -785,7 +785,11 @@ int run_trace(Handle& H, Batch& B, const SiriusHipTraceOpts& o, DevOut& dout, co
             int32_t* ll = (int32_t*)H.scratch("gate_l", 4 * (size_t)B.n, &rc);
             if (rc) return rc;
             uint32_t* counts = work + 16;
-            const double long_band = SIRIUS_LONG_BAND;  // the longest rays first
+            // the longest rays first: a volumetric ray is long wherever it passes the shell, so a wider
+            // band of them starts early (six 256x256 cameras: tracer 3.63 ms at 0.5 M, 3.50 at 1, 3.40
+            // at 2 and 4); disk rays only where they wind (1080p: 1.28 ms at 0.15 M, 1.20 at 0.5, 1.26
+            // at 1, 1.49 at 2: what is first is out of the image's order)
+            const double long_band = B.tp.emission == SIRIUS_EMISSION_VOLUMETRIC ? 4.0 * SIRIUS_LONG_BAND : SIRIUS_LONG_BAND;
             if ((e = launch_gate(B.cams_dev, (int)B.cc.size(), tabs, B.tp.tile_lw, B.n, std::max(o.escalate_band, 0.0),
                                  std::max(o.critical_band, 0.0), long_band, la, list_b, ll, counts, dout.flags,
                                  H.stream)) != hipSuccess)
