@@ -73,6 +73,7 @@ struct TraceParams {
     const int32_t* first_list;
     const uint32_t* first_count;
     int tile_lw;  // order in which whole batches are taken (tile_pixel)
+    int lanes;    // lanes of a wave that take rays (64; fewer for batches smaller than the chip)
 };
 
 // Arrays that one kernel gathers into a block (k_gather): sources, 16-byte aligned offsets, bytes.

@@ -472,6 +472,7 @@ int prepare_batch(Handle& H, const SiriusHipCamera* cams, int n_cam, const Siriu
     // 64 fills whole cache lines in one XCD's L2, a square's 32-byte pieces of a line meet in several
     // (1080p tracer 1.19 ms in rows, 1.38 in squares).
     tp.tile_lw = o.precision == SIRIUS_PRECISION_FP32_ESCALATE && tp.emission == SIRIUS_EMISSION_THIN_DISK ? TILE_ROW : TILE_SQUARE;
+    tp.lanes = 64;
     tp.sym_order = o.symplectic_order;
     tp.n_cam = n_cam;
     // escalation machinery of the FP32 path: always on for the wormhole throat and the warp wall;
@@ -840,6 +841,18 @@ int run_trace(Handle& H, Batch& B, const SiriusHipTraceOpts& o, DevOut& dout, co
                                       : persistent_blocks_per_cu(false, B.kernels, B.tp.emission, B.tp.n_cam > 1, block);
         int grid = std::max(1, bpc * H.cu_count);
         int refill = default_refill(o, B, sur || list_dev != nullptr);
+        // A batch of fewer than 64 rays per SIMD: one wave on each, with as many lanes of it taking rays as
+        // that needs. The call lasts as long as its longest ray, and every event of a ray (a crossing, a
+        // landing, a store) delays the other lanes of its wave: the tracer takes 397 us for a 96x54 Kerr
+        // frame (519 with whole waves), 518 for 200x112 (625), 644 for 320x180 (696), 124 for a 150x150
+        // wormhole (183). Not volumetric: its loop is twice the instructions, and waves on every SIMD
+        // slow each other (two 64x64 cameras 3.55 ms, 2.34 with whole waves); nor FP64, where nothing is
+        // gained (160x90 Kerr frame 2.21 ms and 2.25).
+        const int64_t simds = 4 * (int64_t)std::max(H.cu_count, 1);
+        if (!list_dev && !sur && B.tp.emission != SIRIUS_EMISSION_VOLUMETRIC && B.n < 64 * simds) {
+            t32.lanes = (int)std::max<int64_t>(4, (B.n + simds - 1) / simds);
+            if (o.blocks_per_cu <= 0) grid = std::max(1, H.cu_count * 256 / block);
+        }
         if (time_it) (void)hipEventRecord(H.ev0, H.stream);
         if ((e = launch_trace_persistent(false, B.kernels, B.tp.emission, B.tp.n_cam > 1, B.cams_dev, t32, dout, list_a,
                                          count_a, cap_a, work, work + 1, esc, (unsigned long long*)(work + 2), grid,

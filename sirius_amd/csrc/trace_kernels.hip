@@ -631,18 +631,21 @@ __device__ __forceinline__ void persistent_body(const CamConst* __restrict__ cam
     const uint32_t tail_start = tail_from > 0 ? (uint32_t)tail_from : 0u;
     const uint32_t total32 = (uint32_t)total;
     unsigned long long my_attempts = 0;  // attempts of every ray this lane traced
+    const int width = tp.lanes;
+    const unsigned long long takers = width < 64 ? (1ull << width) - 1ull : ~0ull;  // lanes that take rays
+    if (refill_min > width) refill_min = width;
     while (true) {
-        unsigned long long idle = __ballot(!active);
+        unsigned long long idle = __ballot(!active) & takers;
         int n_idle = __popcll(idle);
         if constexpr (sizeof(T) == 8) {
-            if ((n_idle == 64 || (!exhausted && n_idle >= refill_min)) && pending) {
+            if ((n_idle == width || (!exhausted && n_idle >= refill_min)) && pending) {
                 land<T, FAM, EMIT>(R, s);
                 ray_store<T, FAM, EMIT>(R, o, tp);
                 pending = false;
             }
         }
-        if (n_idle == 64 && exhausted) break;
-        if (!exhausted && (n_idle >= refill_min || n_idle == 64)) {
+        if (n_idle == width && exhausted) break;
+        if (!exhausted && (n_idle >= refill_min || n_idle == width)) {
             // idle lane of rank r takes reserved slot res_lo + r while reserved ones last, then
             // slot base + (r - from_old) of a new reservation
             const uint32_t old_lo = res_lo;
@@ -665,7 +668,7 @@ __device__ __forceinline__ void persistent_body(const CamConst* __restrict__ cam
                 res_lo += from_old;
             }
             if (queue_done && (res_hi < total32 ? res_hi : total32) <= res_lo) exhausted = true;
-            if (!active) {
+            if (!active && lane < width) {
                 unsigned long long below = lane ? (idle & ((1ull << lane) - 1ull)) : 0ull;
                 const uint32_t r = (uint32_t)__popcll(below);
                 const int64_t slot = r < from_old ? (int64_t)old_lo + r
