@@ -718,16 +718,16 @@ __device__ __forceinline__ void persistent_body(const CamConst* __restrict__ cam
     cams, tp, o, ray_list, list_count, n, head, esc_count, esc_list, attempts_out, refill_min, flag_or
 
 // FP64 variants: register allocation left to the compiler (the thin-disk tracer takes 256 VGPRs plus
-// 20 AGPRs, one wave per SIMD). The single-camera warp tracer, which re-traces wall crossers (a
-// tenth of a warp frame, too few rays to hide one wave's latency), is held to two waves (202
+// 10 AGPRs, one wave per SIMD). The single-camera warp tracer, which re-traces wall crossers (a
+// tenth of a warp frame, too few rays to hide one wave's latency), is held to two waves (204
 // registers, no spills). Bound by FP64 issue, so by the instructions of a step: with roots and
 // reciprocals of third order, no Lambda terms where no camera has any, the radius taken from the
 // step's last right-hand side, one reciprocal for the error norm, events located by Newton iteration
 // and landings deferred to the refill (land, above), the thin-disk tracer runs the 1283x721 Kerr
 // frame in 2.9 ms (4.57 in rows and raster order; 5.62 also with the Lambda terms and two Newton steps
 // per root; 8.99 also with IEEE roots and divisions, 52 halvings per event and each ray landed as it
-// ended), the warp tracer its 1024x1024 frame's wall crossers in 0.82 ms (1.65), the wormhole tracer
-// its frame's near-throat rays in 0.38 ms (0.72).
+// ended), the warp tracer its 1024x1024 frame's wall crossers in 0.66 ms (1.65), the wormhole tracer
+// its frame's near-throat rays in 0.35 ms (0.72).
 constexpr int fp64_min_waves(int fam, bool multi) { return fam == 2 && !multi ? 2 : 1; }
 // The persistent tracers start on a 4 KiB boundary of the code object. Their loops are about
 // 19 KiB of instructions, and where the linker happened to place them changed their speed: the
@@ -742,10 +742,10 @@ void k_trace_persistent(SIRIUS_PERSISTENT_PARAMS) {
 
 // FP32 variants. The thin-disk tracers, whose natural allocation lies just above the 168 VGPRs
 // of three waves per SIMD, are held to that budget (no spills at 168; three waves instead of two).
-// The single-camera volumetric tracer's natural allocation (264 registers) leaves one wave per
-// SIMD; held to the 256 of two waves it spills 5 and runs a 1024x1024 frame 1.54 times faster
-// (30.0 -> 19.5 ms, same results). The others keep the compiler's allocation (the multi-camera
-// volumetric tracer takes 256 by itself).
+// The single-camera volumetric tracer is held to the 256 registers of two waves per SIMD (it takes
+// 242; at the 264 and one wave it took by itself with the library's exponentials a 1024x1024 frame
+// ran 1.54 times longer). The others keep the compiler's allocation (the multi-camera volumetric
+// tracer takes 238 by itself).
 constexpr int fp32_min_waves(int emit, bool multi) {
     return emit == SIRIUS_EMISSION_THIN_DISK ? 3 : (emit == SIRIUS_EMISSION_VOLUMETRIC && !multi ? 2 : 1);
 }
