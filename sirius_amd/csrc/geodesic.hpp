@@ -421,7 +421,8 @@ constexpr int TILE_ROW = 6, TILE_SQUARE = 3;
 SIRIUS_HD __forceinline__ int64_t tile_pixel(int width, int height, int lw, int64_t t) {
     const uint32_t w = (uint32_t)width, h = (uint32_t)height, u = (uint32_t)t;  // w h < 2^31
     const uint32_t tw = 1u << lw, th = 64u >> lw;
-    const uint32_t band = u / (th * w), y0 = th * band, bh = h - y0 < th ? h - y0 : th, v = u - y0 * w;
+    // an image of fewer rows than a band is one band: its height in the divisor keeps that below 2^31 too
+    const uint32_t band = u / ((h < th ? h : th) * w), y0 = th * band, bh = h - y0 < th ? h - y0 : th, v = u - y0 * w;
     const uint32_t col = v / (tw * bh), x0 = tw * col, q = v - x0 * bh;
     const uint32_t cw = w - x0 < tw ? w - x0 : tw, y = q / cw;
     return (int64_t)(y0 + y) * w + x0 + (q - y * cw);
