@@ -114,6 +114,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
         id = id < nf ? first[id] : order[id - nf];
     }
     const CamConst& c = cams[find_cam(cams, n_cam, id)];
+    if (!traces_camera<double, FAM>(c)) return;
     const int64_t pix = order ? id - c.offset : tile_pixel(c.width, c.height, TILE_SQUARE, id - c.offset);
     id = c.offset + pix;
     const double u0 = (double)(pix % c.width) + 0.5, v0 = (double)(pix / c.width) + 0.5;

@@ -408,11 +408,20 @@ SIRIUS_HD __forceinline__ T event_radius_rate(const Spacetime<T>& s, const T x[4
 }
 
 // Spacetime codes of the kernels' template parameter FAM: the metric families, and Kerr-Schild with
-// Lambda = 0 in every camera of the batch. Without the Lambda terms a step is one straight run of
-// instructions; with them each right-hand side carries a branch, seven multiply-adds by a zero
-// Lambda after it, and splits the step for the scheduler.
+// Lambda = 0 (FP64). Without the Lambda terms a step is one straight run of instructions; with them
+// each right-hand side carries a branch, seven multiply-adds by a zero Lambda after it, and splits
+// the step for the scheduler.
 enum { FAM_KS = 0, FAM_MT = 1, FAM_WARP = 2, FAM_KS_FLAT = 3 };
 constexpr bool is_ks(int fam) { return fam == FAM_KS || fam == FAM_KS_FLAT; }
+
+// Whether a kernel traces this camera's rays: each FP64 Kerr-Schild kernel takes its own kind only, and a
+// batch of both kinds runs both over the same rays. So the bits of a camera's results do not depend
+// on the Lambda of the other cameras that share its call.
+template <class T, int FAM>
+SIRIUS_HD __forceinline__ bool traces_camera(const CamConst& c) {
+    if constexpr (is_ks(FAM) && !std::is_same_v<T, float>) return (c.Lambda == 0.0) == (FAM == FAM_KS_FLAT);
+    return true;
+}
 
 // Order in which the tracers take an image's rays: position t of a width x height image -> pixel, in
 // bands of 64 >> lw rows cut into tiles of 1 << lw columns (smaller at the right and bottom edges), so

@@ -442,9 +442,11 @@ int prepare_batch(Handle& H, const SiriusHipCamera* cams, int n_cam, const Siriu
     if (off <= 0 || off > (int64_t)INT32_MAX - (1 << 20)) return H.fail(SIRIUS_HIP_E_INVALID, "ray count out of range");
     B.n = off;
     B.kernels = B.family;
-    if (B.family == SIRIUS_METRIC_KERR_SCHILD &&
-        std::all_of(B.cc.begin(), B.cc.end(), [](const CamConst& c) { return c.Lambda == 0.0; }))
-        B.kernels = FAM_KS_FLAT;
+    if (B.family == SIRIUS_METRIC_KERR_SCHILD) {
+        const auto flat = std::count_if(B.cc.begin(), B.cc.end(), [](const CamConst& c) { return c.Lambda == 0.0; });
+        if (flat == n_cam) B.kernels = FAM_KS_FLAT;
+        else B.mixed = flat > 0;
+    }
     TraceParams& tp = B.tp;
     std::memset(&tp, 0, sizeof(tp));
     tp.rtol = o.rtol; tp.atol = o.atol; tp.h_init = o.h_init; tp.h_min = o.h_min; tp.h_max = o.h_max;
@@ -674,6 +676,23 @@ static int default_refill(const SiriusHipTraceOpts& o, const Batch& B, bool pick
     return picked || B.tp.tile_lw == TILE_ROW ? 16 : 64;
 }
 
+// The FP64 tracer over a list of the batch's rays, or all of them, from the queue head `head`. Cameras
+// with and without Lambda in one batch: both kernels in turn, the second from `head2`, each tracing
+// its own cameras' rays.
+static hipError_t launch_fp64(const Batch& B, const TraceParams& tp, const DevOut& o, const int32_t* list,
+                              const uint32_t* list_count, int64_t n, uint32_t* head, uint32_t* head2,
+                              uint32_t* esc_count, unsigned long long* attempts, int grid, int block, int refill_min,
+                              uint32_t flag_or, hipStream_t st) {
+    hipError_t e = launch_trace_persistent(true, B.kernels, B.tp.emission, B.tp.n_cam > 1, B.cams_dev, tp, o, list,
+                                           list_count, n, head, esc_count, nullptr, attempts, grid, block, refill_min,
+                                           flag_or, st);
+    if (e == hipSuccess && B.mixed)
+        e = launch_trace_persistent(true, FAM_KS_FLAT, B.tp.emission, B.tp.n_cam > 1, B.cams_dev, tp, o, list,
+                                    list_count, n, head2, esc_count, nullptr, attempts, grid, block, refill_min,
+                                    flag_or, st);
+    return e;
+}
+
 int run_trace(Handle& H, Batch& B, const SiriusHipTraceOpts& o, DevOut& dout, const int32_t* list_dev,
               const uint32_t* list_count_dev, int64_t list_cap, SiriusHipStats* stats, bool time_it,
               const SiriusHipRayOutput* host_out, bool* delivered) {
@@ -688,7 +707,8 @@ int run_trace(Handle& H, Batch& B, const SiriusHipTraceOpts& o, DevOut& dout, co
     // work[8..10] surrogate list counts (A, B, audit), work[11] audit queue head,
     // work[12] band queue head, work[13] unused, work[14..15] band attempts (u64),
     // work[16..18] gate counts (A, B, L), work[19] surrogate candidates, work[20] candidates the
-    // calibrated error gate refused
+    // calibrated error gate refused, work[21..23] precision audit, work[24..28] heads of the second
+    // queue of a batch with and without Lambda (bulk, band, escalation, audit, precision audit),
     // work[32..47] statistics sums (u64), work[48..] the null-drift histogram
     struct {
         uint32_t wk[32];
@@ -705,8 +725,10 @@ int run_trace(Handle& H, Batch& B, const SiriusHipTraceOpts& o, DevOut& dout, co
     if (time_it) (void)hipEventRecord(H.ev0, H.stream);
     if (o.integrator == SIRIUS_INTEGRATOR_SYMPLECTIC) {
         if (list_dev) return H.fail(SIRIUS_HIP_E_UNSUPPORTED, "symplectic integrator with a ray list");
-        if ((e = launch_symplectic(fp64, B.kernels, B.cams_dev, B.tp, dout, block, H.stream)) != hipSuccess)
-            return H.hip_fail(e, "symplectic launch");
+        const int kinds[2] = {B.kernels, FAM_KS_FLAT};
+        for (int k = 0; k < (fp64 && B.mixed ? 2 : 1); ++k)
+            if ((e = launch_symplectic(fp64, kinds[k], B.cams_dev, B.tp, dout, block, H.stream)) != hipSuccess)
+                return H.hip_fail(e, "symplectic launch");
     } else if (!persistent || fp64) {
         // Grid schedule: one lane per ray, run to completion, no escalation queue (FP32 lanes
         // run to the end in FP32). It is the tracer kernel with a static assignment: a grid of
@@ -732,11 +754,13 @@ int run_trace(Handle& H, Batch& B, const SiriusHipTraceOpts& o, DevOut& dout, co
             grid = std::max(1, bpc * H.cu_count);
             refill = default_refill(o, B, picked);
         }
-        if ((e = launch_trace_persistent(fp64, B.kernels, B.tp.emission, B.tp.n_cam > 1, B.cams_dev, tp, dout, list_dev,
-                                         list_count_dev, n_work, work, work + 1, nullptr,
-                                         (unsigned long long*)(work + 2), grid, block, refill, 0, H.stream)) !=
-            hipSuccess)
-            return H.hip_fail(e, "trace launch");
+        unsigned long long* att = (unsigned long long*)(work + 2);
+        e = fp64 ? launch_fp64(B, tp, dout, list_dev, list_count_dev, n_work, work, work + 24, work + 1, att, grid, block,
+                               refill, 0, H.stream)
+                 : launch_trace_persistent(false, B.kernels, B.tp.emission, B.tp.n_cam > 1, B.cams_dev, tp, dout,
+                                           list_dev, list_count_dev, n_work, work, work + 1, nullptr, att, grid, block,
+                                           refill, 0, H.stream);
+        if (e != hipSuccess) return H.hip_fail(e, "trace launch");
         if (time_it) (void)hipEventRecord(H.ev1, H.stream);
     } else {
         // FP32 path. (1) Gate (Kerr-Schild): every ray's distance from the critical curve; rays
@@ -830,10 +854,9 @@ int run_trace(Handle& H, Batch& B, const SiriusHipTraceOpts& o, DevOut& dout, co
             (void)hipStreamWaitEvent(H.stream2, H.ev_gate, 0);
             int bpc64 = persistent_blocks_per_cu(true, B.kernels, B.tp.emission, B.tp.n_cam > 1, 64);
             (void)hipEventRecord(H.ev_band0, H.stream2);
-            if ((e = launch_trace_persistent(true, B.kernels, B.tp.emission, B.tp.n_cam > 1, B.cams_dev, t64, dout, list_b,
-                                             work + 17, B.n, work + 12, work + 13, nullptr,
-                                             (unsigned long long*)(work + 14), std::max(1, bpc64 * H.cu_count), 64, 1,
-                                             SIRIUS_FLAG_ESCALATED, H.stream2)) != hipSuccess)
+            if ((e = launch_fp64(B, t64, dout, list_b, work + 17, B.n, work + 12, work + 25, work + 13,
+                                 (unsigned long long*)(work + 14), std::max(1, bpc64 * H.cu_count), 64, 1,
+                                 SIRIUS_FLAG_ESCALATED, H.stream2)) != hipSuccess)
                 return H.hip_fail(e, "band launch");
             (void)hipEventRecord(H.ev_band1, H.stream2);
         }
@@ -861,10 +884,9 @@ int run_trace(Handle& H, Batch& B, const SiriusHipTraceOpts& o, DevOut& dout, co
         if (time_it) (void)hipEventRecord(H.ev1, H.stream);
         if (B.tp.escalate) {
             int bpc64 = persistent_blocks_per_cu(true, B.kernels, B.tp.emission, B.tp.n_cam > 1, 64);
-            if ((e = launch_trace_persistent(true, B.kernels, B.tp.emission, B.tp.n_cam > 1, B.cams_dev, t64, dout, esc,
-                                             work + 1, cap_a, work + 4, work + 5, nullptr,
-                                             (unsigned long long*)(work + 6), std::max(1, bpc64 * H.cu_count), 64, 1,
-                                             SIRIUS_FLAG_ESCALATED, H.stream)) != hipSuccess)
+            if ((e = launch_fp64(B, t64, dout, esc, work + 1, cap_a, work + 4, work + 26, work + 5,
+                                 (unsigned long long*)(work + 6), std::max(1, bpc64 * H.cu_count), 64, 1,
+                                 SIRIUS_FLAG_ESCALATED, H.stream)) != hipSuccess)
                 return H.hip_fail(e, "escalation launch");
         }
         if (band) (void)hipStreamWaitEvent(H.stream, H.ev_band1, 0);
@@ -884,10 +906,8 @@ int run_trace(Handle& H, Batch& B, const SiriusHipTraceOpts& o, DevOut& dout, co
             TraceParams ta = fp64_reference_params(B.tp);
             if ((e = launch_fill((uint32_t*)aatt, 2, 0u, H.stream)) != hipSuccess) return H.hip_fail(e, "fill");
             int bpc64 = persistent_blocks_per_cu(true, B.kernels, B.tp.emission, B.tp.n_cam > 1, 64);
-            if ((e = launch_trace_persistent(true, B.kernels, B.tp.emission, B.tp.n_cam > 1, B.cams_dev, ta, oa,
-                                             list_audit, work + 10, B.n, work + 11, work + 5, nullptr, aatt,
-                                             std::max(1, bpc64 * H.cu_count), 64, 1, SIRIUS_FLAG_AUDITED,
-                                             H.stream)) != hipSuccess)
+            if ((e = launch_fp64(B, ta, oa, list_audit, work + 10, B.n, work + 11, work + 27, work + 5, aatt,
+                                 std::max(1, bpc64 * H.cu_count), 64, 1, SIRIUS_FLAG_AUDITED, H.stream)) != hipSuccess)
                 return H.hip_fail(e, "audit launch");
             if ((e = launch_sur_audit(B.cams_dev, ta, oa, dout, list_audit, work + 10, B.n, aacc, H.stream)) !=
                 hipSuccess)
@@ -925,10 +945,8 @@ int run_trace(Handle& H, Batch& B, const SiriusHipTraceOpts& o, DevOut& dout, co
         int bpc64 = persistent_blocks_per_cu(true, B.kernels, B.tp.emission, B.tp.n_cam > 1, 64);
         if ((e = launch_precision_select(dout, B.n, o.precision_audit, o.audit_seed, plist, work + 21, H.stream)) !=
                 hipSuccess ||
-            (e = launch_trace_persistent(true, B.kernels, B.tp.emission, B.tp.n_cam > 1, B.cams_dev, tr, oa, plist,
-                                         work + 21, B.n, work + 22, work + 23, nullptr, patt,
-                                         std::max(1, bpc64 * H.cu_count), 64, 1, SIRIUS_FLAG_AUDITED, H.stream)) !=
-                hipSuccess ||
+            (e = launch_fp64(B, tr, oa, plist, work + 21, B.n, work + 22, work + 28, work + 23, patt,
+                             std::max(1, bpc64 * H.cu_count), 64, 1, SIRIUS_FLAG_AUDITED, H.stream)) != hipSuccess ||
             (e = launch_precision_compare(B.cams_dev, tr, oa, dout, plist, work + 21, B.n, pacc, phist, H.stream)) !=
                 hipSuccess)
             return H.hip_fail(e, "precision audit");

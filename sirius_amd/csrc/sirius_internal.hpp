@@ -135,6 +135,7 @@ struct Batch {
     TraceParams tp;
     int family = 0;
     int kernels = 0;  // spacetime code of the kernels (FAM_*): the family, or FAM_KS_FLAT
+    bool mixed = false;  // some cameras with Lambda, some without: FP64 kernels run as FAM_KS and FAM_KS_FLAT
     int64_t n = 0;
 };
 

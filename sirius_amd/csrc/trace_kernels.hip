@@ -681,10 +681,12 @@ __device__ __forceinline__ void persistent_body(const CamConst* __restrict__ cam
                         const CamConst& c = cams[cam];
                         id = c.offset + tile_pixel(c.width, c.height, tp.tile_lw, id - c.offset);
                     }
-                    ray_start<T, FAM, EMIT>(R, cams, cam, id, tp, o);
-                    R.flags |= flag_or;
-                    if (MULTI) s = make_spacetime<T>(cams[cam]);
-                    active = true;
+                    if (!MULTI || traces_camera<T, FAM>(cams[cam])) {
+                        ray_start<T, FAM, EMIT>(R, cams, cam, id, tp, o);
+                        R.flags |= flag_or;
+                        if (MULTI) s = make_spacetime<T>(cams[cam]);
+                        active = true;
+                    }
                 }
             }
         }
@@ -959,6 +961,7 @@ __global__ __launch_bounds__(256) void k_symplectic_grid(const CamConst* __restr
     int64_t id = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (id >= tp.n_rays) return;
     int cam = tp.n_cam == 1 ? 0 : find_camera(cams, tp.n_cam, id);
+    if (!traces_camera<T, FAM>(cams[cam])) return;
     Ray<T, FAM> R;
     ray_start<T, FAM, SIRIUS_EMISSION_THIN_DISK>(R, cams, cam, id, tp, o);
     const CamConst& c = cams[cam];
