@@ -969,17 +969,18 @@ SIRIUS_HD __forceinline__ T dense_slope(T y0, T y1, T h, T k0, T k1, T r5, T th)
 // the signs seen so far keep (a step leaving it is replaced by the bracket's midpoint), starting
 // from the linear interpolant's root. The bracket is closed: a converged iterate has just become
 // one of its ends, and its Newton update (itself, to rounding) is kept, not bisected away. The
-// iteration ends when a Newton step moves th by less than tol, or after 24 rounds (each of them
-// at least as good as a halving: a step falling back to the midpoint halves the bracket, one
-// staying inside converges quadratically). The event functions are smooth across a step (the
-// plane z = 0, or a sphere of the event radius), so most crossings converge in two or three
-// rounds, for a fraction of the instructions of 24 halvings: a wave runs this whenever one of its
-// lanes has an event in the step, for as many rounds as its slowest lane needs.
+// iteration ends when a Newton step moves th by less than tol. A step inside the bracket may still
+// gain little (a root where the slope vanishes, two iterates that map to each other), so FP64, whose
+// events were located to the last bit by 52 halvings, halves the bracket from the ninth round on, 52
+// times; FP32 ends after 24 rounds. The event functions are smooth across a step (the plane z = 0, or a
+// sphere of the event radius), so most crossings converge in two or three rounds, for a fraction of
+// the instructions of the halvings: a wave runs this whenever one of its lanes has an event in the
+// step, for as many rounds as its slowest lane needs.
 template <class T>
 SIRIUS_HD __forceinline__ T locate_event_newton(const Spacetime<T>& s, int kind, T target, const T x0[4],
                                                 const T k0[4], const T x1[4], const T k1[4], const T dn[6], T h,
                                                 T f0, T f1) {
-    constexpr int max_iters = 24;
+    constexpr int newton_iters = sizeof(T) == 4 ? 24 : 8, max_iters = sizeof(T) == 4 ? 24 : 60;
     const T tol = T(sizeof(T) == 4 ? 2e-7 : 1e-12);  // the last step's own error is its square
     T lo = T(0), hi = T(1);
     const bool neg_lo = f0 < T(0);
@@ -1004,7 +1005,7 @@ SIRIUS_HD __forceinline__ T locate_event_newton(const Spacetime<T>& s, int kind,
         if (f == T(0)) break;
         if ((f < T(0)) == neg_lo) lo = th; else hi = th;
         const T nt = df != T(0) ? th - f / df : T(-1);
-        if (nt >= lo && nt <= hi) {
+        if (it < newton_iters && nt >= lo && nt <= hi) {
             const bool done = fabs(nt - th) <= tol;
             th = nt;
             if (done) break;
