@@ -113,16 +113,24 @@ void star_record(const SiriusHipStar& s, const SiriusHipStarfield& c, float* rec
     star_colour(s.temperature_K, rec[6], rec[7], rec[8]);
 }
 
+}  // namespace
+
 // Cell index of a catalogue of star records: for each cell of the sphere's (theta, phi) grid, the
 // stars whose cut reaches any direction of the cell, in catalogue order, so that a view direction
 // needs to look at its own cell's stars only and adds them in the order a walk of the whole
-// catalogue would. Layout: cells + 1 offsets, then the star numbers. Empty when the index would
-// exceed STAR_CELL_ENTRIES (spreads of a good part of the sky) or a record is not finite: the
-// shading kernel then walks the catalogue.
+// catalogue would. Layout: cells + 1 offsets, then the star numbers. Empty, so that the shading kernel
+// walks the catalogue, when a record is not finite, when the index would exceed STAR_CELL_ENTRIES, or
+// when a cell's list holds more than 1/STAR_CELL_SHARE of the catalogue on average: a list is read
+// from memory, lane by lane, where the walk reads LDS. Cost of both spheres in a 1024x1024 launch, index
+// and walk: 192 and 424 us for 1000 stars at a share of 0.035, 330 and 502 at 0.066, 524 and 610 at
+// 0.10, 845 and 813 at 0.18, 1830 and 1354 at 0.40. The index is built on the host, 2 ns an entry: up
+// to 1/16 it pays after 15 launches (0.75 ms for 300 stars at 0.035, 12 ms for 4096), above that after 30
+// to 160 (81 ms for 4096 stars at 0.10).
 // The device compares float cosines: a star can pass its cut at an angle whose true cosine is up to
 // 1e-6 below it (direction and product roundings, 3e-7), and a direction's cell is found from
 // its float angles (4e-7 rad); the reach is widened by both.
 constexpr size_t STAR_CELL_ENTRIES = (size_t)1 << 24;
+constexpr int STAR_CELL_SHARE = 16;
 
 std::vector<int32_t> star_cell_index(const std::vector<float>& rec, int n) {
     constexpr int NT = SIRIUS_STAR_NT, NP = SIRIUS_STAR_NP;
@@ -132,6 +140,7 @@ std::vector<int32_t> star_cell_index(const std::vector<float>& rec, int n) {
     };
     std::vector<Span> span(n);
     std::vector<int32_t> idx((size_t)NT * NP + 1, 0);
+    const size_t most = std::min(STAR_CELL_ENTRIES, (size_t)n * NT * NP / STAR_CELL_SHARE);
     size_t total = 0;
     for (int i = 0; i < n; ++i) {
         const float* s = rec.data() + (size_t)i * SIRIUS_STAR_REC;
@@ -157,7 +166,7 @@ std::vector<int32_t> star_cell_index(const std::vector<float>& rec, int n) {
         }
         span[i] = sp;
         total += (size_t)(sp.t1 - sp.t0 + 1) * sp.np;
-        if (total > STAR_CELL_ENTRIES) return {};
+        if (total > most) return {};
         for (int t = sp.t0; t <= sp.t1; ++t)
             for (int k = 0; k < sp.np; ++k) ++idx[1 + t * NP + (sp.p0 + k) % NP];
     }
@@ -170,8 +179,6 @@ std::vector<int32_t> star_cell_index(const std::vector<float>& rec, int n) {
             for (int k = 0; k < span[i].np; ++k) idx[base + at[t * NP + (span[i].p0 + k) % NP]++] = i;
     return idx;
 }
-
-}  // namespace
 
 }  // namespace sirius
 
