@@ -870,11 +870,15 @@ int run_trace(Handle& H, Batch& B, const SiriusHipTraceOpts& o, DevOut& dout, co
         // frame (519 with whole waves), 518 for 200x112 (625), 644 for 320x180 (696), 124 for a 150x150
         // wormhole (183). Not volumetric: its loop is twice the instructions, and waves on every SIMD
         // slow each other (two 64x64 cameras 3.55 ms, 2.34 with whole waves); nor FP64, where nothing is
-        // gained (160x90 Kerr frame 2.21 ms and 2.25).
+        // gained (160x90 Kerr frame 2.21 ms and 2.25). With a caller's grid the lanes follow from its waves:
+        // cut for one wave per SIMD on a grid of fewer, rays wait for others (150x150 wormhole on one block
+        // of 64 per CU 249 us, 106 in whole waves). And only Kerr-Schild, whose rays differ in length,
+        // gains from thin waves there (150x100 sky at 64/8: 535 and 655; 80x100 wormhole at 64/2: 139 and 113).
         const int64_t simds = 4 * (int64_t)std::max(H.cu_count, 1);
         if (!list_dev && !sur && B.tp.emission != SIRIUS_EMISSION_VOLUMETRIC && B.n < 64 * simds) {
-            t32.lanes = (int)std::max<int64_t>(4, (B.n + simds - 1) / simds);
             if (o.blocks_per_cu <= 0) grid = std::max(1, H.cu_count * 256 / block);
+            if (o.blocks_per_cu <= 0 || B.family == SIRIUS_METRIC_KERR_SCHILD)
+                t32.lanes = thin_lanes(B.n, (int64_t)grid * (block / 64), simds);
         }
         if (time_it) (void)hipEventRecord(H.ev0, H.stream);
         if ((e = launch_trace_persistent(false, B.kernels, B.tp.emission, B.tp.n_cam > 1, B.cams_dev, t32, dout, list_a,

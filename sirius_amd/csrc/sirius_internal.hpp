@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <array>
 #include <cstring>
 #include <map>
@@ -172,6 +173,12 @@ struct RayOrder {
     const int32_t* first = nullptr;
     const uint32_t* first_count = nullptr;
 };
+// Lanes of each wave that take rays when n rays start on `waves` waves at once, one wave to a SIMD: no fewer
+// than hold all of them in flight, up to whole waves.
+inline int thin_lanes(int64_t n, int64_t waves, int64_t simds) {
+    const int64_t w = std::max<int64_t>(1, std::min(waves, simds));
+    return (int)std::min<int64_t>(64, std::max<int64_t>(4, (n + w - 1) / w));
+}
 int longest_first(Handle& H, Batch& B, int rays_per_wave, uint32_t* counts, uint8_t* flags, RayOrder& r);
 hipError_t launch_fill(uint32_t* p, int n, uint32_t v, hipStream_t st);
 
