@@ -473,7 +473,21 @@ int prepare_batch(Handle& H, const SiriusHipCamera* cams, int n_cam, const Siriu
     // 0.48 and 0.43). FP32 thin-disk rays end after 15 steps, so their results' stores count: a row of
     // 64 fills whole cache lines in one XCD's L2, a square's 32-byte pieces of a line meet in several
     // (1080p tracer 1.19 ms in rows, 1.38 in squares).
-    tp.tile_lw = o.precision == SIRIUS_PRECISION_FP32_ESCALATE && tp.emission == SIRIUS_EMISSION_THIN_DISK ? TILE_ROW : TILE_SQUARE;
+    // FP32 rays without emission go in rows where a camera sees a part of the shadow's edge: its view is lower
+    // than the shadow (2 sqrt(27) M at the hole's distance), but not so narrow that it lies inside it.
+    // Near-critical rays fill such an image, the call lasts as long as the longest of them, and in
+    // squares these share waves, whose late landings delay each other (1280x720 frames: 15 M away with 12
+    // degrees 1.06 ms in rows, 1.57 in squares, 10 M with 25 degrees 1.57 and 1.90; of the whole
+    // shadow 1.54 and 1.36, of its inside 0.54 and 0.40). From 1.5 M rays on the other waves hide that
+    // (1920x1080, 12 M with 25 degrees 2.72 and 2.39).
+    const bool fp32 = o.precision == SIRIUS_PRECISION_FP32_ESCALATE;
+    bool rows = fp32 && tp.emission == SIRIUS_EMISSION_THIN_DISK;
+    if (fp32 && B.family == SIRIUS_METRIC_KERR_SCHILD && tp.emission == SIRIUS_EMISSION_NONE && B.n < 1500000)
+        for (int i = 0; i < n_cam; ++i) {
+            const double shadow = std::sqrt(27.0) * B.cc[i].M, h2 = cams[i].r_obs * std::tan(cams[i].fov_deg * (M_PI / 360.0));
+            rows |= h2 < shadow && h2 * std::max(1.0, (double)cams[i].width / cams[i].height) > 0.5 * shadow;
+        }
+    tp.tile_lw = rows ? TILE_ROW : TILE_SQUARE;
     tp.lanes = 64;
     tp.sym_order = o.symplectic_order;
     tp.n_cam = n_cam;
