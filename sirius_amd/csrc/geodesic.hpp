@@ -875,7 +875,9 @@ SIRIUS_HD __forceinline__ float exp_parts(float x, float& s) {
     s = ldexpf(1.f, (int)n);
     return fmaf(f * f, q, f);
 }
-// e^x - 1 for x >= 0 (held at 88, where it is 1.7e38); e^x for x <= 0 (held at -88).
+// e^x - 1 for x >= 0, held at 88, where it is 1.7e38; e^x for x <= 0, held at -88, where it is 6e-39. The
+// tracing kernels flush denormals, so the reciprocal of the one and the other itself are 0 from 87.4
+// on: a spectrum falls as e^-x down to 1e-38 of x^3 and is 0 beyond.
 SIRIUS_HD __forceinline__ float expm1_pos(float x) {
     float s;
     const float p = exp_parts(fminf(x, 88.f), s);
