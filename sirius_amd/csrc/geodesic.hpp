@@ -972,17 +972,15 @@ SIRIUS_HD __forceinline__ T dense_slope(T y0, T y1, T h, T k0, T k1, T r5, T th)
 // from the linear interpolant's root. The bracket is closed: a converged iterate has just become
 // one of its ends, and its Newton update (itself, to rounding) is kept, not bisected away. The
 // iteration ends when a Newton step moves th by less than tol. A step inside the bracket may still
-// gain little (a root where the slope vanishes, two iterates that map to each other), so FP64, whose
-// events were located to the last bit by 52 halvings, halves the bracket from the ninth round on, 52
-// times; FP32 ends after 24 rounds. The event functions are smooth across a step (the plane z = 0, or a
-// sphere of the event radius), so most crossings converge in two or three rounds, for a fraction of
-// the instructions of the halvings: a wave runs this whenever one of its lanes has an event in the
-// step, for as many rounds as its slowest lane needs.
-template <class T>
+// gain little (a root where the slope vanishes, two iterates that map to each other): after NEWTON
+// rounds the bracket is halved, and the iteration ends after ROUNDS. The event functions are smooth
+// across a step (the plane z = 0, or a sphere of the event radius), so most crossings converge in two
+// or three rounds, for a fraction of the instructions of the halvings: a wave runs this whenever one
+// of its lanes has an event in the step, for as many rounds as its slowest lane needs.
+template <class T, int NEWTON = 24, int ROUNDS = 24>
 SIRIUS_HD __forceinline__ T locate_event_newton(const Spacetime<T>& s, int kind, T target, const T x0[4],
                                                 const T k0[4], const T x1[4], const T k1[4], const T dn[6], T h,
                                                 T f0, T f1) {
-    constexpr int newton_iters = sizeof(T) == 4 ? 24 : 8, max_iters = sizeof(T) == 4 ? 24 : 60;
     const T tol = T(sizeof(T) == 4 ? 2e-7 : 1e-12);  // the last step's own error is its square
     T lo = T(0), hi = T(1);
     const bool neg_lo = f0 < T(0);
@@ -990,7 +988,7 @@ SIRIUS_HD __forceinline__ T locate_event_newton(const Spacetime<T>& s, int kind,
     T th = den != T(0) ? f0 / den : T(0.5);
     th = th > T(0) && th < T(1) ? th : T(0.5);
 #pragma unroll 1
-    for (int it = 0; it < max_iters; ++it) {
+    for (int it = 0; it < ROUNDS; ++it) {
         T f, df;
         if (kind == EV_Z) {
             f = dense_eval(x0[3], x1[3], h, k0[3], k1[3], dn[2], th);
@@ -1007,7 +1005,7 @@ SIRIUS_HD __forceinline__ T locate_event_newton(const Spacetime<T>& s, int kind,
         if (f == T(0)) break;
         if ((f < T(0)) == neg_lo) lo = th; else hi = th;
         const T nt = df != T(0) ? th - f / df : T(-1);
-        if (it < newton_iters && nt >= lo && nt <= hi) {
+        if (it < NEWTON && nt >= lo && nt <= hi) {
             const bool done = fabs(nt - th) <= tol;
             th = nt;
             if (done) break;
@@ -1040,14 +1038,16 @@ SIRIUS_HD __forceinline__ T locate_event_dense(const Spacetime<T>& s, int kind, 
     return T(0.5) * (lo + hi);
 }
 
-// Event location on the step's cubic Hermite interpolant (the dense output without its r5 term):
-// the FP64 path's locator.
+// Event location on the step's cubic Hermite interpolant (the dense output without its r5 term): the
+// locator of the FP64 paths and the FP32 symplectic integrator. Eight Newton rounds, then halvings to
+// the last bit.
 template <class T>
 SIRIUS_HD __forceinline__ T locate_event(const Spacetime<T>& s, int kind, T target, const T x0[4], const T k0[4],
                                  const T x1[4], const T k1[4], T h) {
     const T dn[6] = {T(0), T(0), T(0), T(0), T(0), T(0)};
-    return locate_event_newton(s, kind, target, x0, k0, x1, k1, dn, h, event_value(s, kind, x0, target),
-                               event_value(s, kind, x1, target));
+    return locate_event_newton<T, 8, 8 + (sizeof(T) == 8 ? 52 : 24)>(s, kind, target, x0, k0, x1, k1, dn, h,
+                                                                   event_value(s, kind, x0, target),
+                                                                   event_value(s, kind, x1, target));
 }
 
 // ------------------------------------------------------------------------------------------

@@ -1,4 +1,4 @@
-"""FP64 event location in a host build against bisection of the same interpolant
+"""Event location on a step's cubic interpolant (FP64 and FP32 symplectic) in a host build against bisection of the same interpolant
 (cpp/event_locate_check.cpp states the cases and the bar)."""
 import os
 import shutil
