@@ -39,12 +39,11 @@ static int trace_bundles(Handle& H, Batch& B, int emission, int n_cam, const Bun
     if (e != hipSuccess) return H.hip_fail(e, "fill");
     RayOrder order;
     if ((rc = longest_first(H, B, 32, counts, bo.flags, order))) return rc;
-    const int kinds[2] = {B.kernels, FAM_KS_FLAT};
-    for (int k = 0; k < (B.mixed ? 2 : 1); ++k) {
-        e = launch_trace_bundle(kinds[k], emission, B.cams_dev, n_cam, B.tp, params_of(H.bundle), bo, order.main,
-                                order.first, order.first_count, H.stream);
-        if (e != hipSuccess) return H.hip_fail(e, "bundle trace");
-    }
+    e = launch_kinds(H, B, H.stream, [&](int kernels, int, hipStream_t st) {
+        return launch_trace_bundle(kernels, emission, B.cams_dev, n_cam, B.tp, params_of(H.bundle), bo, order.main,
+                                   order.first, order.first_count, st);
+    });
+    if (e != hipSuccess) return H.hip_fail(e, "bundle trace");
     return SIRIUS_HIP_OK;
 }
 

@@ -281,7 +281,7 @@ void Handle::release() {
     ev0 = ev1 = ev2 = ev3 = ev4 = nullptr;
     delete last;
     last = nullptr;
-    for (hipEvent_t* ev : {&ev_gate, &ev_band0, &ev_band1, &ev_s0, &ev_s1, &ev_a0, &ev_a1, &ev_p0, &ev_p1}) {
+    for (hipEvent_t* ev : {&ev_gate, &ev_band0, &ev_band1, &ev_mix, &ev_s0, &ev_s1, &ev_a0, &ev_a1, &ev_p0, &ev_p1}) {
         if (*ev) (void)hipEventDestroy(*ev);
         *ev = nullptr;
     }
@@ -320,7 +320,7 @@ int Handle::ensure_device() {
     total_mem = prop.totalGlobalMem;
     if ((e = hipStreamCreateWithFlags(&stream, hipStreamNonBlocking)) != hipSuccess) return hip_fail(e, "stream");
     if ((e = hipStreamCreateWithFlags(&stream2, hipStreamNonBlocking)) != hipSuccess) return hip_fail(e, "stream");
-    for (hipEvent_t* ev : {&ev_gate, &ev_band0, &ev_band1, &ev_s0, &ev_s1, &ev_a0, &ev_a1, &ev_p0, &ev_p1})
+    for (hipEvent_t* ev : {&ev_gate, &ev_band0, &ev_band1, &ev_mix, &ev_s0, &ev_s1, &ev_a0, &ev_a1, &ev_p0, &ev_p1})
         if ((e = hipEventCreate(ev)) != hipSuccess) return hip_fail(e, "event");
     if ((e = hipEventCreate(&ev0)) != hipSuccess) return hip_fail(e, "event");
     if ((e = hipEventCreate(&ev1)) != hipSuccess) return hip_fail(e, "event");
@@ -690,21 +690,17 @@ static int default_refill(const SiriusHipTraceOpts& o, const Batch& B, bool pick
     return picked || B.tp.tile_lw == TILE_ROW ? 16 : 64;
 }
 
-// The FP64 tracer over a list of the batch's rays, or all of them, from the queue head `head`. Cameras
-// with and without Lambda in one batch: both kernels in turn, the second from `head2`, each tracing
-// its own cameras' rays.
-static hipError_t launch_fp64(const Batch& B, const TraceParams& tp, const DevOut& o, const int32_t* list,
+// The FP64 tracer over a list of the batch's rays, or all of them, from the queue head `head`; the second
+// kernel of a batch with and without Lambda starts from `head2`.
+static hipError_t launch_fp64(Handle& H, const Batch& B, const TraceParams& tp, const DevOut& o, const int32_t* list,
                               const uint32_t* list_count, int64_t n, uint32_t* head, uint32_t* head2,
                               uint32_t* esc_count, unsigned long long* attempts, int grid, int block, int refill_min,
                               uint32_t flag_or, hipStream_t st) {
-    hipError_t e = launch_trace_persistent(true, B.kernels, B.tp.emission, B.tp.n_cam > 1, B.cams_dev, tp, o, list,
-                                           list_count, n, head, esc_count, nullptr, attempts, grid, block, refill_min,
-                                           flag_or, st);
-    if (e == hipSuccess && B.mixed)
-        e = launch_trace_persistent(true, FAM_KS_FLAT, B.tp.emission, B.tp.n_cam > 1, B.cams_dev, tp, o, list,
-                                    list_count, n, head2, esc_count, nullptr, attempts, grid, block, refill_min,
-                                    flag_or, st);
-    return e;
+    return launch_kinds(H, B, st, [&](int kernels, int k, hipStream_t s) {
+        return launch_trace_persistent(true, kernels, B.tp.emission, B.tp.n_cam > 1, B.cams_dev, tp, o, list,
+                                       list_count, n, k ? head2 : head, esc_count, nullptr, attempts, grid, block,
+                                       refill_min, flag_or, s);
+    });
 }
 
 int run_trace(Handle& H, Batch& B, const SiriusHipTraceOpts& o, DevOut& dout, const int32_t* list_dev,
@@ -739,10 +735,12 @@ int run_trace(Handle& H, Batch& B, const SiriusHipTraceOpts& o, DevOut& dout, co
     if (time_it) (void)hipEventRecord(H.ev0, H.stream);
     if (o.integrator == SIRIUS_INTEGRATOR_SYMPLECTIC) {
         if (list_dev) return H.fail(SIRIUS_HIP_E_UNSUPPORTED, "symplectic integrator with a ray list");
-        const int kinds[2] = {B.kernels, FAM_KS_FLAT};
-        for (int k = 0; k < (fp64 && B.mixed ? 2 : 1); ++k)
-            if ((e = launch_symplectic(fp64, kinds[k], B.cams_dev, B.tp, dout, block, H.stream)) != hipSuccess)
-                return H.hip_fail(e, "symplectic launch");
+        e = fp64 ? launch_kinds(H, B, H.stream,
+                                [&](int kernels, int, hipStream_t st) {
+                                    return launch_symplectic(true, kernels, B.cams_dev, B.tp, dout, block, st);
+                                })
+                 : launch_symplectic(false, B.kernels, B.cams_dev, B.tp, dout, block, H.stream);
+        if (e != hipSuccess) return H.hip_fail(e, "symplectic launch");
     } else if (!persistent || fp64) {
         // Grid schedule: one lane per ray, run to completion, no escalation queue (FP32 lanes
         // run to the end in FP32). It is the tracer kernel with a static assignment: a grid of
@@ -769,7 +767,7 @@ int run_trace(Handle& H, Batch& B, const SiriusHipTraceOpts& o, DevOut& dout, co
             refill = default_refill(o, B, picked);
         }
         unsigned long long* att = (unsigned long long*)(work + 2);
-        e = fp64 ? launch_fp64(B, tp, dout, list_dev, list_count_dev, n_work, work, work + 24, work + 1, att, grid, block,
+        e = fp64 ? launch_fp64(H, B, tp, dout, list_dev, list_count_dev, n_work, work, work + 24, work + 1, att, grid, block,
                                refill, 0, H.stream)
                  : launch_trace_persistent(false, B.kernels, B.tp.emission, B.tp.n_cam > 1, B.cams_dev, tp, dout,
                                            list_dev, list_count_dev, n_work, work, work + 1, nullptr, att, grid, block,
@@ -868,7 +866,7 @@ int run_trace(Handle& H, Batch& B, const SiriusHipTraceOpts& o, DevOut& dout, co
             (void)hipStreamWaitEvent(H.stream2, H.ev_gate, 0);
             int bpc64 = persistent_blocks_per_cu(true, B.kernels, B.tp.emission, B.tp.n_cam > 1, 64);
             (void)hipEventRecord(H.ev_band0, H.stream2);
-            if ((e = launch_fp64(B, t64, dout, list_b, work + 17, B.n, work + 12, work + 25, work + 13,
+            if ((e = launch_fp64(H, B, t64, dout, list_b, work + 17, B.n, work + 12, work + 25, work + 13,
                                  (unsigned long long*)(work + 14), std::max(1, bpc64 * H.cu_count), 64, 1,
                                  SIRIUS_FLAG_ESCALATED, H.stream2)) != hipSuccess)
                 return H.hip_fail(e, "band launch");
@@ -902,7 +900,7 @@ int run_trace(Handle& H, Batch& B, const SiriusHipTraceOpts& o, DevOut& dout, co
         if (time_it) (void)hipEventRecord(H.ev1, H.stream);
         if (B.tp.escalate) {
             int bpc64 = persistent_blocks_per_cu(true, B.kernels, B.tp.emission, B.tp.n_cam > 1, 64);
-            if ((e = launch_fp64(B, t64, dout, esc, work + 1, cap_a, work + 4, work + 26, work + 5,
+            if ((e = launch_fp64(H, B, t64, dout, esc, work + 1, cap_a, work + 4, work + 26, work + 5,
                                  (unsigned long long*)(work + 6), std::max(1, bpc64 * H.cu_count), 64, 1,
                                  SIRIUS_FLAG_ESCALATED, H.stream)) != hipSuccess)
                 return H.hip_fail(e, "escalation launch");
@@ -924,7 +922,7 @@ int run_trace(Handle& H, Batch& B, const SiriusHipTraceOpts& o, DevOut& dout, co
             TraceParams ta = fp64_reference_params(B.tp);
             if ((e = launch_fill((uint32_t*)aatt, 2, 0u, H.stream)) != hipSuccess) return H.hip_fail(e, "fill");
             int bpc64 = persistent_blocks_per_cu(true, B.kernels, B.tp.emission, B.tp.n_cam > 1, 64);
-            if ((e = launch_fp64(B, ta, oa, list_audit, work + 10, B.n, work + 11, work + 27, work + 5, aatt,
+            if ((e = launch_fp64(H, B, ta, oa, list_audit, work + 10, B.n, work + 11, work + 27, work + 5, aatt,
                                  std::max(1, bpc64 * H.cu_count), 64, 1, SIRIUS_FLAG_AUDITED, H.stream)) != hipSuccess)
                 return H.hip_fail(e, "audit launch");
             if ((e = launch_sur_audit(B.cams_dev, ta, oa, dout, list_audit, work + 10, B.n, aacc, H.stream)) !=
@@ -963,7 +961,7 @@ int run_trace(Handle& H, Batch& B, const SiriusHipTraceOpts& o, DevOut& dout, co
         int bpc64 = persistent_blocks_per_cu(true, B.kernels, B.tp.emission, B.tp.n_cam > 1, 64);
         if ((e = launch_precision_select(dout, B.n, o.precision_audit, o.audit_seed, plist, work + 21, H.stream)) !=
                 hipSuccess ||
-            (e = launch_fp64(B, tr, oa, plist, work + 21, B.n, work + 22, work + 28, work + 23, patt,
+            (e = launch_fp64(H, B, tr, oa, plist, work + 21, B.n, work + 22, work + 28, work + 23, patt,
                              std::max(1, bpc64 * H.cu_count), 64, 1, SIRIUS_FLAG_AUDITED, H.stream)) != hipSuccess ||
             (e = launch_precision_compare(B.cams_dev, tr, oa, dout, plist, work + 21, B.n, pacc, phist, H.stream)) !=
                 hipSuccess)

@@ -65,9 +65,10 @@ struct Handle {
     bool ready = false;
     bool initialised = false;
     hipStream_t stream = nullptr;
-    hipStream_t stream2 = nullptr;  // second stream: the FP64 band runs beside the FP32 bulk
+    // second stream: the FP64 band beside the FP32 bulk, the second kernel of a batch with and without Lambda
+    hipStream_t stream2 = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr, ev2 = nullptr, ev3 = nullptr, ev4 = nullptr;
-    hipEvent_t ev_gate = nullptr, ev_band0 = nullptr, ev_band1 = nullptr;
+    hipEvent_t ev_gate = nullptr, ev_band0 = nullptr, ev_band1 = nullptr, ev_mix = nullptr;
     hipEvent_t ev_s0 = nullptr, ev_s1 = nullptr, ev_a0 = nullptr, ev_a1 = nullptr;  // surrogate, audit
     hipEvent_t ev_p0 = nullptr, ev_p1 = nullptr;  // precision audit
     int cu_count = 0;
@@ -178,6 +179,23 @@ struct RayOrder {
 inline int thin_lanes(int64_t n, int64_t waves, int64_t simds) {
     const int64_t w = std::max<int64_t>(1, std::min(waves, simds));
     return (int)std::min<int64_t>(64, std::max<int64_t>(4, (n + w - 1) / w));
+}
+// An FP64 pass over a batch on stream st: launch(kernels, k, stream) is called for B.kernels (k = 0) and, in
+// a batch with and without Lambda, for FAM_KS_FLAT (k = 1), which traces the other cameras' rays: beside
+// the first on the second stream, and joined to st again. In turn, the passes would last as long as the
+// longest rays of both kinds together (two 160x90 cameras: symplectic 25.1 ms, FP64 disk 8.0, bundles
+// 10.6; side by side 18.1, 6.0 and 8.3).
+template <class F>
+hipError_t launch_kinds(Handle& H, const Batch& B, hipStream_t st, F launch) {
+    if (!B.mixed) return launch(B.kernels, 0, st);
+    hipError_t e = hipSuccess;
+    const bool beside = st != H.stream2;
+    if (beside && ((e = hipEventRecord(H.ev_mix, st)) != hipSuccess ||
+                   (e = hipStreamWaitEvent(H.stream2, H.ev_mix, 0)) != hipSuccess))
+        return e;
+    if ((e = launch(B.kernels, 0, st)) != hipSuccess || (e = launch((int)FAM_KS_FLAT, 1, H.stream2)) != hipSuccess) return e;
+    if (beside && (e = hipEventRecord(H.ev_mix, H.stream2)) == hipSuccess) e = hipStreamWaitEvent(st, H.ev_mix, 0);
+    return e;
 }
 int longest_first(Handle& H, Batch& B, int rays_per_wave, uint32_t* counts, uint8_t* flags, RayOrder& r);
 hipError_t launch_fill(uint32_t* p, int n, uint32_t v, hipStream_t st);
