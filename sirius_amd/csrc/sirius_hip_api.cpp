@@ -684,7 +684,8 @@ int longest_first(Handle& H, Batch& B, int rays_per_wave, uint32_t* counts, uint
 
 // Idle lanes at which a wave of a persistent queue refills: the caller's choice, or a quarter wave
 // where neighbours in the queue end apart (rows, lists of picked rays) and the whole wave where they
-// end together (squares: FP32 warp bubble 0.75 ms at 16, 0.66 at 64; volumetric 4.23 and 3.97).
+// end together (squares: FP32 warp bubble 0.75 ms at 16, 0.66 at 64; volumetric 4.23 and 3.97; 1920x1080
+// Kerr sky 3.12 and 2.59; 1024x1024 wormhole 0.46 and 0.43; FP64 the same at both).
 static int default_refill(const SiriusHipTraceOpts& o, const Batch& B, bool picked) {
     if (o.refill_min > 0) return std::min(o.refill_min, 64);
     return picked || B.tp.tile_lw == TILE_ROW ? 16 : 64;

@@ -606,8 +606,9 @@ __global__ __launch_bounds__(256) void k_star_shade(DevOut o, int64_t n, const f
 // in catalogue order, so the sums are those of k_star_shade bit for bit. That kernel is bound by
 // its cosine tests: on a 1024x1024 wormhole frame it takes 1.48 ms for two spheres of 4096 stars and
 // 25 us for two of 22; this one, bound by the directions' FP64 sines and its reads, 16 and 7 us. So
-// it is taken for point sampling whenever the spheres have an index, at every catalogue size; a
-// beam's footprint can reach beyond its cell, so ray bundles walk the catalogue.
+// it is taken for point sampling whenever the spheres have an index (star_cell_index: while the cells' lists
+// are short; above a share of about 0.15 of the catalogue the walk is faster); a beam's footprint
+// can reach beyond its cell, so ray bundles walk the catalogue.
 __global__ __launch_bounds__(256) void k_star_cells(DevOut o, int64_t n, const float* __restrict__ rec0,
                                                     const int32_t* __restrict__ cells0, float b0,
                                                     const float* __restrict__ rec1,
